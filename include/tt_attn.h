@@ -284,11 +284,27 @@ int tt_cross_entropy_backward_f32(const float* p, const int* labels, float* grad
  * (src/Layers_kernels.cu:10-30: a cuBLAS handle created and destroyed around
  * one cublasSgemm per call), called by FcForward / FcBackward (src/Layers.cu:
  * 26-77) and ConvForward / ConvBackward (:197, :247-248).  fp32: fp32
- * products and sums on the fp32 MFMA; bf16: bf16 A, B, C with fp32 sums. */
+ * products and sums on the fp32 MFMA; bf16: bf16 A, B, C with fp32 sums.
+ * Products too small to fill the chip split k over workgroups through a
+ * 16 MiB per-stream library workspace (allocated on first use); if that
+ * allocation fails, or the stream is being captured into a graph, they run
+ * unsplit and allocate nothing. */
 int tt_gemm_f32(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha,
                 const float* A, const float* B, float beta, float* C, void* stream);
 int tt_gemm_bf16(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha,
                  const uint16_t* A, const uint16_t* B, float beta, uint16_t* C, void* stream);
+
+/* The fully connected layer on that GEMM: out[batch x fout] = in[batch x fin]
+ * weight[fin x fout] + bias, the bias added to the fp32 sum before the store
+ * (FcForward, src/Layers.cu:9-42, which adds it with a second GEMM against a
+ * column of ones).  bias holds fout values, or one for every output when
+ * bias_scalar != 0.  dtype TT_F32 or TT_BF16. */
+int tt_fc_forward(int dtype, int64_t batch, int64_t fin, int64_t fout, const void* in, const void* weight,
+                  const void* bias, int bias_scalar, void* out, void* stream);
+/* Column sums of a row-major [rows x cols] matrix, y[c] = sum_r x[r][c], in
+ * fp32 and in a fixed order: FcBackward's bias gradient (src/Layers.cu:68-78,
+ * a GEMM with a row of ones).  dtype TT_F32 or TT_BF16; rows = 0 gives 0. */
+int tt_col_sum(int dtype, const void* x, void* y, int64_t rows, int64_t cols, void* stream);
 
 /* ---------------------------------------------------------------- convolution data movement */
 

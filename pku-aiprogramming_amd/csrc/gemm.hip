@@ -11,9 +11,10 @@
 // beta = 0 does not read C.  fp32 on v_mfma_f32_32x32x2f32 (fp32 products,
 // fp32 sums) and bf16 on v_mfma_f32_32x32x16_bf16 (fp32 sums, bf16 C).
 //
-// bf16 calls with k % 32 == 0 and aligned operands run k_gemm_dma: direct
-// global -> LDS tile loads into swizzled, unpadded tiles.  Every other call
-// runs k_gemm:
+// Products too small to fill the chip with 128-row tiles run the 64 x 64
+// kernel of gemm_split.h, its contraction split over workgroups.  Larger bf16
+// calls with k % 32 == 0 and aligned operands run k_gemm_dma: direct global ->
+// LDS tile loads into swizzled, unpadded tiles.  The others run k_gemm:
 // Workgroup = 4 waves, a 128 x 128 (fp32) or 128 x 256 (bf16) tile of C
 // (each wave 64 x 64 or 64 x 128: 2 x 2 or 2 x 4 MFMA blocks of 32 x 32);
 // k in steps of BK through a two-stage LDS ring,
@@ -24,13 +25,16 @@
 //   rows contiguous (A with transa = 1, B with transb = 0):
 //     [BK][rows], bf16 operands by transpose reads (ds_read_b64_tr_b16),
 //     fp32 operands by scalar reads.
-// Tiles past m, n or k read zeros.  16-byte global loads when every row
-// stride and base is 16-byte aligned, element loads otherwise.
+// Tiles past m, n or k read zeros.  Global loads are 16 bytes at any element
+// alignment (the target reads unaligned words), element loads at the edges:
+// with element loads wherever a row was not 16-byte aligned, bf16 3001 x 2001
+// x 1003 took 111-120 us instead of 49-73.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 
 #include "attn_common.h"
+#include "gemm_split.h"
 #include "tt_internal.h"
 
 namespace tt {
@@ -48,8 +52,6 @@ struct GemmT<float> {
   static constexpr int PAD_K = 4;         // [rows][BK + PAD_K]: 80-byte rows keep 16-byte stores aligned
   static constexpr int PAD_R = 4;         // [BK][rows + PAD_R]
   static constexpr bool SWZ = false;      // k-contiguous tiles padded, not swizzled
-  static __device__ __forceinline__ float to_f(float x) { return x; }
-  static __device__ __forceinline__ float from_f(float x) { return x; }
 };
 template <>
 struct GemmT<u16> {
@@ -66,8 +68,6 @@ struct GemmT<u16> {
   static constexpr int PAD_K = 0;
   static constexpr int PAD_R = 32;
   static constexpr bool SWZ = true;
-  static __device__ __forceinline__ float to_f(u16 x) { return bf16_to_f32(x); }
-  static __device__ __forceinline__ u16 from_f(float x) { return f32_to_bf16(x); }
 };
 
 // One operand tile (A: rows = m; B: rows = n) of R rows by BK k-values.
@@ -106,7 +106,6 @@ struct OpTile {
 
   // Global -> registers.  The tile covers rows [r0, r0 + R) and k [k0, k0 + BK)
   // of op(X); rows >= nrows or k >= K read 0.
-  template <bool VEC>
   __device__ __forceinline__ void load(const T* X, int64_t ld, int r0, int k0, int nrows, int K) {
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
@@ -117,8 +116,8 @@ struct OpTile {
       const int gcol = KC ? k0 + scol : r0 + scol;
       const int rlim = KC ? nrows : K, clim = KC ? K : nrows;
       const T* p = X + (int64_t)grow * ld + gcol;
-      if (VEC && grow < rlim && gcol + EPC <= clim) {
-        reg[c] = *reinterpret_cast<const u32x4*>(p);
+      if (grow < rlim && gcol + EPC <= clim) {
+        reg[c] = *reinterpret_cast<const split_u32x4_any*>(p);
       } else {
         T v[EPC];
 #pragma unroll
@@ -165,10 +164,9 @@ __device__ __forceinline__ auto operand(const T* s, int rbase, int ks) {
   }
 }
 
-template <typename T, bool TA, bool TB, bool VEC>
-__global__ __launch_bounds__(256, 2) void k_gemm(int M, int N, int K, float alpha, const T* __restrict__ A,
-                                                int64_t lda, const T* __restrict__ B, int64_t ldb, float beta,
-                                                T* C) {
+template <typename T, bool TA, bool TB>
+__global__ __launch_bounds__(256, 2) void k_gemm(int M, int N, int K, const T* __restrict__ A, int64_t lda,
+                                                const T* __restrict__ B, int64_t ldb, MatrixEpilogue<T> ep) {
   using G = GemmT<T>;
   constexpr int GN = G::GN, NB = GN / 64;  // MFMA blocks per wave along n
   constexpr int BK = G::BK, KS = sizeof(T) == 2 ? BK / 16 : BK / 2;  // MFMA k-steps per BK
@@ -191,8 +189,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm(int M, int N, int K, float alph
   TileB tb;
   const int nk = (K + BK - 1) / BK;
   if (nk > 0) {
-    ta.template load<VEC>(A, lda, m0, 0, M, K);
-    tb.template load<VEC>(B, ldb, n0, 0, N, K);
+    ta.load(A, lda, m0, 0, M, K);
+    tb.load(B, ldb, n0, 0, N, K);
     ta.store(sA[0]);
     tb.store(sB[0]);
   }
@@ -200,8 +198,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm(int M, int N, int K, float alph
   for (int kt = 0; kt < nk; ++kt) {
     const int cur = kt & 1;
     if (kt + 1 < nk) {  // next step's tiles in flight during this step's MFMAs
-      ta.template load<VEC>(A, lda, m0, BK * (kt + 1), M, K);
-      tb.template load<VEC>(B, ldb, n0, BK * (kt + 1), N, K);
+      ta.load(A, lda, m0, BK * (kt + 1), M, K);
+      tb.load(B, ldb, n0, BK * (kt + 1), N, K);
     }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -238,10 +236,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(int M, int N, int K, float alph
       for (int r = 0; r < 16; ++r) {
         const int m = m0 + wm + 32 * i + acc_row(r, l >> 5);
         if (m >= M) continue;
-        T* p = C + (int64_t)m * N + n;
-        float v = alpha * acc[i][j][r];
-        if (beta != 0.f) v += beta * G::to_f(*p);
-        *p = G::from_f(v);
+        ep(m, n, acc[i][j][r]);
       }
     }
 }
@@ -310,10 +305,8 @@ __device__ __forceinline__ bf16x8 dma_operand(const u16* s, int rbase, int ks) {
 }
 
 template <bool TA, bool TB>
-__global__ __launch_bounds__(256, 3) void k_gemm_dma(int M, int N, int K, float alpha, const u16* __restrict__ A,
-                                                    int64_t lda, const u16* __restrict__ B, int64_t ldb,
-                                                    float beta, u16* C) {
-  using G = GemmT<u16>;
+__global__ __launch_bounds__(256, 3) void k_gemm_dma(int M, int N, int K, const u16* __restrict__ A, int64_t lda,
+                                                    const u16* __restrict__ B, int64_t ldb, MatrixEpilogue<u16> ep) {
   constexpr int GN = kDmaGN, NB = GN / 64, BK = 32, KS = BK / 16, S = kDmaStages;
   using TileA = DmaTile<GM, !TA>;
   using TileB = DmaTile<GN, TB>;
@@ -371,17 +364,35 @@ __global__ __launch_bounds__(256, 3) void k_gemm_dma(int M, int N, int K, float 
       for (int r = 0; r < 16; ++r) {
         const int m = m0 + wm + 32 * i + acc_row(r, l >> 5);
         if (m >= M) continue;
-        u16* p = C + (int64_t)m * N + n;
-        float v = alpha * acc[i][j][r];
-        if (beta != 0.f) v += beta * G::to_f(*p);
-        *p = G::from_f(v);
+        ep(m, n, acc[i][j][r]);
       }
     }
 }
 
+// Whether the 64 x 64 split kernel (gemm_split.h) takes this product instead
+// of the 128-row tiles.  Measured on the MI355X (N(0,1) operands, us, 128-row
+// tiles / 64 x 64 split):
+//   fp32: 512^3 46 / 14, 1024^3 87 / 33, 2048^3 171 / 166, 2560^3 360 / 350,
+//   3072^3 620 / 550, 4096^3 1090 / 1250, 6000 x 6000 x 200 142 / 168.  The
+//   128 x 128 kernel runs at 128 TF when its tiles fill whole rounds of the
+//   512 workgroup slots (two per CU), the 64 x 64 one at 110 TF whatever
+//   their count: the line is a fill of the rounds below 0.8.
+//   bf16, direct-to-LDS kernel: 1536^3 (72 tiles) 37 / 22, 2048^3 (128) 47 /
+//   34, 2560^3 (200) 59 / 68, 3072 x 3072 x 1024 (288) 34 / 42.
+//   bf16, other shapes: 2047^3 (128) 144 / 71, 3001 x 2001 x 1003 (192) 73 /
+//   50, 4095^3 (512) 331 / 487.
+template <typename T>
+bool use_split_tiles(int64_t m, int64_t n, int64_t k, bool dma) {
+  if (k >= (int64_t(1) << 30)) return false;  // its k indices are 32-bit
+  const int64_t tiles = ((n + GemmT<T>::GN - 1) / GemmT<T>::GN) * ((m + GM - 1) / GM);
+  if (sizeof(T) == 2) return tiles < (dma ? 160 : 256);
+  const int64_t rounds = (tiles + 511) / 512;
+  return 10 * tiles < 8 * 512 * rounds && tiles < 8192;
+}
+
 template <typename T>
 int gemm_launch(const char* fn, int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha, const T* A,
-                const T* B, float beta, T* C, void* stream) {
+                const T* B, float beta, T* C, const T* bias, int64_t bias_step, void* stream) {
   if (m < 0 || n < 0 || k < 0) return fail(TT_ERR_ARG, std::string(fn) + ": negative size");
   if (transa != 0 && transa != 1) return fail(TT_ERR_ARG, std::string(fn) + ": transa must be 0 or 1");
   if (transb != 0 && transb != 1) return fail(TT_ERR_ARG, std::string(fn) + ": transb must be 0 or 1");
@@ -397,16 +408,30 @@ int gemm_launch(const char* fn, int transa, int transb, int64_t m, int64_t n, in
   if (rc) return rc;
   hipStream_t s = stream_or_default(stream);
   const int64_t lda = transa ? m : k, ldb = transb ? k : n;
-  constexpr int EPC = GemmT<T>::EPC;
-  const bool vec = lda % EPC == 0 && ldb % EPC == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)B % 16 == 0;
+  const MatrixEpilogue<T> ep{C, bias, bias_step, alpha, beta, (int)n};
+  // direct-to-LDS kernel: k in whole steps, aligned rows (m, n multiples of 8
+  // where they are the contiguous axis), every per-lane tile offset within 32
+  // bits
+  const bool dma = sizeof(T) == 2 && k % 32 == 0 && lda % 8 == 0 && ldb % 8 == 0 && (uintptr_t)A % 16 == 0 &&
+                   (uintptr_t)B % 16 == 0 && lda < (int64_t(1) << 22) && ldb < (int64_t(1) << 22);
+  if (use_split_tiles<T>(m, n, k, dma)) {
+#define TT_GEMM_S(TA, TB)                                                                                       \
+  return launch_split_gemm<T>(fn, m, n, k, MatrixSource<T, !TA>{A, lda, (int)m, (int)k},                        \
+                              MatrixSource<T, TB>{B, ldb, (int)n, (int)k}, ep, s)
+    switch (transa * 2 + transb) {
+      case 0: TT_GEMM_S(false, false);
+      case 1: TT_GEMM_S(false, true);
+      case 2: TT_GEMM_S(true, false);
+      default: TT_GEMM_S(true, true);
+    }
+#undef TT_GEMM_S
+  }
   const dim3 grid((unsigned)gx, (unsigned)gy), block(256);
   if constexpr (sizeof(T) == 2) {
-    // k in whole steps, aligned rows (m, n multiples of 8 where they are the
-    // contiguous axis: vec), and every per-lane tile offset within 32 bits
-    if (vec && k % 32 == 0 && lda < (int64_t(1) << 22) && ldb < (int64_t(1) << 22)) {
+    if (dma) {
       const dim3 g2((unsigned)((n + kDmaGN - 1) / kDmaGN), (unsigned)gy);
 #define TT_GEMM_D(TA, TB) \
-  hipLaunchKernelGGL((k_gemm_dma<TA, TB>), g2, dim3(256), 0, s, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C)
+  hipLaunchKernelGGL((k_gemm_dma<TA, TB>), g2, dim3(256), 0, s, (int)m, (int)n, (int)k, A, lda, B, ldb, ep)
       switch (transa * 2 + transb) {
         case 0: TT_GEMM_D(false, false); break;
         case 1: TT_GEMM_D(false, true); break;
@@ -418,20 +443,82 @@ int gemm_launch(const char* fn, int transa, int transb, int64_t m, int64_t n, in
       return ok();
     }
   }
-#define TT_GEMM(TA, TB, V)                                                                                   \
-  hipLaunchKernelGGL((k_gemm<T, TA, TB, V>), grid, block, 0, s, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, \
-                     beta, C)
-  switch (transa * 4 + transb * 2 + (vec ? 1 : 0)) {
-    case 0: TT_GEMM(false, false, false); break;
-    case 1: TT_GEMM(false, false, true); break;
-    case 2: TT_GEMM(false, true, false); break;
-    case 3: TT_GEMM(false, true, true); break;
-    case 4: TT_GEMM(true, false, false); break;
-    case 5: TT_GEMM(true, false, true); break;
-    case 6: TT_GEMM(true, true, false); break;
-    default: TT_GEMM(true, true, true); break;
+#define TT_GEMM(TA, TB) \
+  hipLaunchKernelGGL((k_gemm<T, TA, TB>), grid, block, 0, s, (int)m, (int)n, (int)k, A, lda, B, ldb, ep)
+  switch (transa * 2 + transb) {
+    case 0: TT_GEMM(false, false); break;
+    case 1: TT_GEMM(false, true); break;
+    case 2: TT_GEMM(true, false); break;
+    default: TT_GEMM(true, true); break;
   }
 #undef TT_GEMM
+  TT_LAUNCHED(fn, s);
+  return ok();
+}
+
+// Column sums of a row-major [rows][cols] matrix: y[c] = sum over r of
+// x[r][c], the bias gradient of the fully connected layer.  Workgroup (bx,
+// by): 64 columns, rows [by * rpb, (by + 1) * rpb); its 16 waves take rows w,
+// w + 16, ... (64 consecutive elements per load, eight loads in flight) and
+// meet in LDS, all in a fixed order.  With one row block the sums go to y,
+// otherwise to part [blocks][cols], which a second launch over `part` adds.
+// It replaces a product with a row of ones (one 128-row GEMM tile walking
+// all of k, 26-30 us for 256 rows, plus the fill of the ones: 4.5 us).
+constexpr int kColSumRows = 2048;  // rows per row block
+
+template <typename T, typename O>
+__global__ __launch_bounds__(1024) void k_col_sum(const T* __restrict__ x, O* __restrict__ y, int64_t rows,
+                                                  int64_t cols, int64_t rpb) {
+  __shared__ float red[16][64];
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int64_t c = (int64_t)blockIdx.x * 64 + l;
+  const int64_t r1 = min(rows, (int64_t)(blockIdx.y + 1) * rpb);
+  float s = 0.f;
+  if (c < cols) {
+    int64_t r = (int64_t)blockIdx.y * rpb + w;
+    for (; r + 16 * 7 < r1; r += 16 * 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = split_load(x + (r + 16 * u) * cols + c);
+      s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    }
+    for (; r < r1; r += 16) s += split_load(x + r * cols + c);
+  }
+  red[w][l] = s;
+  __syncthreads();
+  if (w == 0 && c < cols) {
+    float t = red[0][l];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) t += red[i][l];
+    split_store(y + blockIdx.y * cols + c, t);
+  }
+}
+
+template <typename T>
+int col_sum_launch(const char* fn, const T* x, T* y, int64_t rows, int64_t cols, hipStream_t s) {
+  const int64_t gx = (cols + 63) / 64;
+  if (!grid_fits(gx, 1024)) return fail(TT_ERR_ARG, std::string(fn) + ": too many columns");
+  int64_t blocks = (rows + kColSumRows - 1) / kColSumRows;
+  if (blocks > kColSumRows) blocks = kColSumRows;  // the second launch adds at most that many partials
+  float* part = nullptr;
+  std::optional<WorkspaceLease> ws;  // held until the second launch is queued
+  // the partials share the split products' buffer; without it one block takes every row
+  if (blocks > 1 && ((size_t)(blocks * cols) * sizeof(float) > kSplitWorkBytes || stream_capturing(s) ||
+                     ws.emplace().get(s, kWsGemmSplits, kSplitWorkBytes, (void**)&part) != TT_OK)) {
+    blocks = 1;
+    part = nullptr;
+  }
+  if (blocks <= 1) {
+    hipLaunchKernelGGL((k_col_sum<T, T>), dim3((unsigned)gx), dim3(1024), 0, s, x, y, rows, cols, rows);
+    TT_LAUNCHED(fn, s);
+    return ok();
+  }
+  const int64_t rpb = (rows + blocks - 1) / blocks;
+  hipLaunchKernelGGL((k_col_sum<T, float>), dim3((unsigned)gx, (unsigned)blocks), dim3(1024), 0, s, x, part, rows,
+                     cols, rpb);
+  TT_LAUNCHED(fn, s);
+  hipLaunchKernelGGL((k_col_sum<float, T>), dim3((unsigned)gx), dim3(1024), 0, s, (const float*)part, y, blocks, cols,
+                     blocks);
   TT_LAUNCHED(fn, s);
   return ok();
 }
@@ -442,12 +529,39 @@ int gemm_launch(const char* fn, int transa, int transb, int64_t m, int64_t n, in
 
 using namespace tt;
 
+extern "C" int tt_fc_forward(int dtype, int64_t batch, int64_t fin, int64_t fout, const void* in, const void* weight,
+                             const void* bias, int bias_scalar, void* out, void* stream) {
+  const char* fn = "tt_fc_forward";
+  if (batch > 0 && fout > 0 && !bias) return fail(TT_ERR_ARG, std::string(fn) + ": null pointer");
+  const int64_t step = bias_scalar ? 0 : 1;
+  if (dtype == TT_F32)
+    return gemm_launch<float>(fn, 0, 0, batch, fout, fin, 1.f, (const float*)in, (const float*)weight, 0.f,
+                              (float*)out, (const float*)bias, step, stream);
+  if (dtype == TT_BF16)
+    return gemm_launch<u16>(fn, 0, 0, batch, fout, fin, 1.f, (const u16*)in, (const u16*)weight, 0.f, (u16*)out,
+                            (const u16*)bias, step, stream);
+  return fail(TT_ERR_ARG, std::string(fn) + ": dtype must be TT_F32 or TT_BF16");
+}
+
+extern "C" int tt_col_sum(int dtype, const void* x, void* y, int64_t rows, int64_t cols, void* stream) {
+  const char* fn = "tt_col_sum";
+  if (rows < 0 || cols < 0) return fail(TT_ERR_ARG, std::string(fn) + ": negative size");
+  if (dtype != TT_F32 && dtype != TT_BF16) return fail(TT_ERR_ARG, std::string(fn) + ": dtype must be TT_F32 or TT_BF16");
+  if (cols == 0) return ok();
+  if (!y || (rows > 0 && !x)) return fail(TT_ERR_ARG, std::string(fn) + ": null pointer");
+  int rc = ensure_init();
+  if (rc) return rc;
+  hipStream_t s = stream_or_default(stream);
+  if (dtype == TT_F32) return col_sum_launch<float>(fn, (const float*)x, (float*)y, rows, cols, s);
+  return col_sum_launch<u16>(fn, (const u16*)x, (u16*)y, rows, cols, s);
+}
+
 extern "C" int tt_gemm_f32(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha, const float* A,
                            const float* B, float beta, float* C, void* stream) {
-  return gemm_launch<float>("tt_gemm_f32", transa, transb, m, n, k, alpha, A, B, beta, C, stream);
+  return gemm_launch<float>("tt_gemm_f32", transa, transb, m, n, k, alpha, A, B, beta, C, nullptr, 0, stream);
 }
 
 extern "C" int tt_gemm_bf16(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha, const uint16_t* A,
                             const uint16_t* B, float beta, uint16_t* C, void* stream) {
-  return gemm_launch<u16>("tt_gemm_bf16", transa, transb, m, n, k, alpha, A, B, beta, C, stream);
+  return gemm_launch<u16>("tt_gemm_bf16", transa, transb, m, n, k, alpha, A, B, beta, C, nullptr, 0, stream);
 }

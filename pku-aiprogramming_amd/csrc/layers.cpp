@@ -165,6 +165,11 @@ void SoftmaxForward(const TinyTensor<T>& input, TinyTensor<T>& output) {
 
 namespace {
 
+template <typename T>
+int dtype_code() {
+  return std::is_same<T, float>::value ? TT_F32 : TT_BF16;
+}
+
 // C = alpha op(A) op(B) + beta C on the library GEMM (row-major, tt_gemm_*).
 template <typename T>
 void gemm(const char* fn, bool ta, bool tb, int64_t m, int64_t n, int64_t k, float alpha, const T* A, const T* B,
@@ -222,18 +227,10 @@ void FcForward(const TinyTensor<T>& input, TinyTensor<T>& output, const TinyTens
   oshape.push_back((int)f.fout);
   output.resize(oshape);
   if (f.batch == 0 || f.fout == 0) return;
-  gemm<T>(fn.c_str(), false, false, f.batch, f.fout, f.fin, 1.f, input.p_data, weight.p_data, 0.f, output.p_data);
-  TinyTensor<T> ones(std::vector<int>{(int)f.batch, 1}, "gpu");
-  ones.ones();
-  if (f.scalar_bias) {
-    TinyTensor<T> row(std::vector<int>{1, (int)f.fout}, "gpu");
-    row.floatks((float)bias.get_data()[0]);
-    gemm<T>(fn.c_str(), false, false, f.batch, f.fout, 1, 1.f, ones.p_data, row.p_data, 1.f, output.p_data);
-    tt_check(tt_sync(), fn.c_str());
-  } else {
-    gemm<T>(fn.c_str(), false, false, f.batch, f.fout, 1, 1.f, ones.p_data, bias.p_data, 1.f, output.p_data);
-    tt_check(tt_sync(), fn.c_str());
-  }
+  tt_check(tt_fc_forward(dtype_code<T>(), f.batch, f.fin, f.fout, input.p_data, weight.p_data, bias.p_data,
+                         f.scalar_bias ? 1 : 0, output.p_data, nullptr),
+           fn.c_str());
+  tt_check(tt_sync(), fn.c_str());
 }
 
 template <typename T>
@@ -273,18 +270,13 @@ void FcBackward(const TinyTensor<T>& input, const TinyTensor<T>& output, const T
           grad_input.p_data);
   gemm<T>(fn.c_str(), true, false, f.fin, f.fout, f.batch, 1.f, input.p_data, grad_output.p_data, 0.f,
           grad_weight.p_data);
-  TinyTensor<T> ones(std::vector<int>{1, (int)f.batch}, "gpu");
-  ones.ones();
   if (f.scalar_bias) {
     TinyTensor<T> row(std::vector<int>{1, (int)f.fout}, "gpu");
-    gemm<T>(fn.c_str(), false, false, 1, f.fout, f.batch, 1.f, ones.p_data, grad_output.p_data, 0.f, row.p_data);
-    TinyTensor<T> col(std::vector<int>{(int)f.fout, 1}, "gpu");
-    col.ones();
-    gemm<T>(fn.c_str(), false, false, 1, 1, f.fout, 1.f, row.p_data, col.p_data, 0.f, grad_bias.p_data);
+    tt_check(tt_col_sum(dtype_code<T>(), grad_output.p_data, row.p_data, f.batch, f.fout, nullptr), fn.c_str());
+    tt_check(tt_col_sum(dtype_code<T>(), row.p_data, grad_bias.p_data, f.fout, 1, nullptr), fn.c_str());
     tt_check(tt_sync(), fn.c_str());
   } else {
-    gemm<T>(fn.c_str(), false, false, 1, f.fout, f.batch, 1.f, ones.p_data, grad_output.p_data, 0.f,
-            grad_bias.p_data);
+    tt_check(tt_col_sum(dtype_code<T>(), grad_output.p_data, grad_bias.p_data, f.batch, f.fout, nullptr), fn.c_str());
     tt_check(tt_sync(), fn.c_str());
   }
 }
@@ -311,11 +303,6 @@ int conv_out(const std::string& fn, int in, int k, int pad, int stride) {
     throw std::invalid_argument(fn + ": kernel sizes >= 1, pads >= 0 and strides >= 1 required");
   if ((int64_t)in + 2 * (int64_t)pad < k) throw std::invalid_argument(fn + ": the kernel is larger than the padded image");
   return (int)((in + 2 * (int64_t)pad - k) / stride + 1);
-}
-
-template <typename T>
-int dtype_code() {
-  return std::is_same<T, float>::value ? TT_F32 : TT_BF16;
 }
 
 template <typename T>

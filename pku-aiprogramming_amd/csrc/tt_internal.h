@@ -28,6 +28,10 @@ int device_cu_count();
 // kernel launch on `s`; a no-op unless instrumentation is enabled.
 void after_launch(hipStream_t s);
 
+// Whether `s` is being captured into a graph (then a launcher allocates
+// nothing and leaves no scratch address behind).
+bool stream_capturing(hipStream_t s);
+
 // The allocation-free backward's scratch: a static device array of
 // kNoAllocScratchBytes whose device address tt_init looks up once per
 // device.  Returns nullptr before tt_init; *bytes gets the array's size.
@@ -38,7 +42,7 @@ void* noalloc_scratch(size_t* bytes);
 // grown on demand and kept for reuse.  A lease holds the workspace lock from
 // get() until it is destroyed: keep it alive until every kernel that reads
 // the buffer has been launched on that stream.
-enum { kWsBackwardRows = 0, kWsDecodePartials = 1, kWsForwardSplits = 2, kWsSoftmaxPartials = 3 };
+enum { kWsBackwardRows = 0, kWsDecodePartials = 1, kWsForwardSplits = 2, kWsSoftmaxPartials = 3, kWsGemmSplits = 4 };
 class WorkspaceLease {
  public:
   WorkspaceLease();

@@ -58,6 +58,15 @@ hipStream_t stream_or_default(void* s) {
   return s ? static_cast<hipStream_t>(s) : g_stream;
 }
 
+bool stream_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;  // unknown: take the path that allocates nothing
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
 // ---------------------------------------------------------------- allocator
 // hipMalloc / hipFree / hipStreamSynchronize as the backend of the caching
 // allocator and the workspace cache (device_cache.h).  Allocation failures,
