@@ -321,6 +321,17 @@ int tt_im2col(int dtype, const void* im, void* col, int64_t N, int C, int H, int
  * col entries that im2col fills from it; every element of im is written. */
 int tt_col2im(int dtype, const void* col, void* im, int64_t N, int C, int H, int W, int kh, int kw, int pad_h,
               int pad_w, int stride_h, int stride_w, void* stream);
+/* The convolution itself (ConvForward / ConvBackward, src/Layers.cu:160-252,
+ * which run im2col, one GEMM per image and col2im): in[N][C][H][W] with
+ * weight[Cout][C][kh][kw] gives out[N][Cout][OH][OW]; the backward writes
+ * grad_in (every element) and grad_weight.  The products gather their
+ * operands from the images (no column matrix) and split long sums over
+ * workgroups like tt_gemm_*, through the same per-stream workspace. */
+int tt_conv_forward(int dtype, const void* in, const void* weight, void* out, int64_t N, int C, int H, int W,
+                    int cout, int kh, int kw, int pad_h, int pad_w, int stride_h, int stride_w, void* stream);
+int tt_conv_backward(int dtype, const void* in, const void* weight, const void* grad_out, void* grad_in,
+                     void* grad_weight, int64_t N, int C, int H, int W, int cout, int kh, int kw, int pad_h,
+                     int pad_w, int stride_h, int stride_w, void* stream);
 
 /* Max pooling over `planes` images [H][W] (batch x channels): out and mask
  * [planes][OH][OW] (OH, OW as for im2col); the window is clipped to the

@@ -1,5 +1,7 @@
-// im2col / col2im: the data movement of the convolution layer on the library
-// GEMM (reference src/Layers.cu:81-158, kernels src/Layers_kernels.cu:32-105).
+// The convolution: its products, which gather their operands from the images
+// (tt_conv_forward / tt_conv_backward, reference src/Layers.cu:160-252), the
+// column matrix on its own (im2col / col2im, src/Layers.cu:81-158, kernels
+// src/Layers_kernels.cu:32-105) and max pooling.
 //
 // Layout (the reference's): an image batch im[N][C][H][W] and its column
 // matrix col[N][P][C][kh][kw], P = OH * OW output pixels in row-major order,
@@ -10,8 +12,10 @@
 // order of the sums, no atomics), the whole batch in one launch.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
+#include "gemm_split.h"
 #include "tt_internal.h"
 
 namespace tt {
@@ -188,6 +192,376 @@ int conv_entry(const char* fn, int dtype, const void* src, void* dst, int64_t N,
   return fail(TT_ERR_ARG, std::string(fn) + ": dtype must be TT_F32 or TT_BF16");
 }
 
+// ---------------------------------------------------------------- the convolution products
+// The convolution's three products as split-k MFMA products (gemm_split.h)
+// whose operands are gathered from the image, so that no column matrix is
+// written:
+//   forward  out[co, q]  = sum over kk of W[co, kk] X(kk, q)     q = (n, oy, ox), kk = (c, ky, kx)
+//   dW       gW[co, kk]  = sum over q of  gO[co, q] X(kk, q)
+//   dX       gX[c, p]    = sum over (co, ky, kx) of W[co, c, ky, kx] gO(co, ky, kx, p)   p = (n, y, x)
+// with X(kk, q) the image element under kernel position kk of output pixel q
+// and gO(.., p) the output gradient that position reads p from (zero where
+// there is none).  One launch covers the whole batch.
+//
+// They replace im2col, one GEMM per image and col2im: at small images the
+// launches dominated (a product per image at 5-76 us each), at large ones the
+// dW product, one or a few tiles walking every pixel.  Forward / backward
+// through myLayer, us, before -> now: 64 x 8 x 14 x 14, 16 kernels 5 x 5 fp32
+// 1557 / 2212 -> 28 / 55; 64 x 64 x 56 x 56, 64 kernels 3 x 3 fp32 4128 /
+// 22291 -> 293 / 693 (51 / 43 TF), bf16 1683 / 7425 -> 179 / 495; 8 x 512 x
+// 28 x 28, 512 kernels 3 x 3 fp32 3468 / 1648 -> 691 / 1490; 1 x 3 x 224 x 224,
+// 768 kernels 16 x 16 stride 16 fp32 85 / 123 -> 29 / 46.  What bounds the
+// large ones now is the gather (index arithmetic and 4- to 16-byte loads).
+
+// n / d for 0 <= n < 2^31 by a multiplication (Granlund and Montgomery's
+// round-up method).
+struct FastDiv {
+  uint32_t d, mul, shift;
+  FastDiv() = default;
+  __host__ __device__ explicit FastDiv(uint32_t d_) : d(d_) {
+    shift = 0;
+    while ((uint64_t(1) << shift) < d) ++shift;
+    mul = (uint32_t)(((uint64_t(1) << 32) * ((uint64_t(1) << shift) - d)) / d + 1);
+  }
+  __device__ __forceinline__ int div(int n) const { return (int)((__umulhi(mul, (uint32_t)n) + (uint32_t)n) >> shift); }
+  __device__ __forceinline__ int divmod(int n, int& rem) const {
+    const int q = div(n);
+    rem = n - q * (int)d;
+    return q;
+  }
+};
+
+struct ConvDivs {
+  FastDiv kk, kw, P, ow;  // kh * kw, kw, oh * ow, ow
+};
+
+// Chunks of EPC consecutive positions of one row of a [planes][h][w] image.
+// X(kk, q): kKC = false puts q on the tile rows (forward), true on k (dW).
+template <typename T, bool KC>
+struct ColumnSource {
+  static constexpr bool kKC = KC, kPhased = false;
+  const T* im;
+  ConvGeom g;
+  ConvDivs dv;
+  int K, Q;
+  __device__ __forceinline__ split_u32x4 chunk(int row, int k) const {
+    constexpr int EPC = SplitT<T>::EPC;
+    const int kk = KC ? row : k, q = KC ? k : row;
+    T v[EPC];
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) v[e] = T(0);
+    if (kk < K && q < Q) {
+      int r, kx, p, ox;
+      const int c = dv.kk.divmod(kk, r), ky = dv.kw.divmod(r, kx);
+      int n = dv.P.divmod(q, p), oy = dv.ow.divmod(p, ox);
+      int y = oy * g.sh - g.ph + ky, x = ox * g.sw - g.pw + kx;
+      const T* pl = im + ((int64_t)n * g.C + c) * g.H * g.W;
+      if (g.sw == 1 && ox + EPC <= g.ow && x >= 0 && x + EPC <= g.W) {  // one image row, inside
+        if (y >= 0 && y < g.H) return *reinterpret_cast<const split_u32x4_any*>(pl + (int64_t)y * g.W + x);
+      } else {
+        const int left = Q - q;
+#pragma unroll
+        for (int e = 0; e < EPC; ++e) {
+          if (e < left && y >= 0 && y < g.H && x >= 0 && x < g.W) v[e] = pl[(int64_t)y * g.W + x];
+          x += g.sw;
+          if (++ox == g.ow) {  // next output row, or the next image
+            ox = 0;
+            x = kx - g.pw;
+            y += g.sh;
+            if (++oy == g.oh) {
+              oy = 0;
+              y = ky - g.ph;
+              pl += (int64_t)g.C * g.H * g.W;
+            }
+          }
+        }
+      }
+    }
+    return __builtin_bit_cast(split_u32x4, v);
+  }
+};
+
+// gO[co, q] of the [N][Cout][P] output gradient: kKC = true rows co, k = q;
+// false rows q, k = co.
+template <typename T, bool KC>
+struct GradRowSource {
+  static constexpr bool kKC = KC, kPhased = false;
+  const T* go;
+  FastDiv P;
+  int cout, Q;
+  __device__ __forceinline__ split_u32x4 chunk(int row, int k) const {
+    constexpr int EPC = SplitT<T>::EPC;
+    const int co = KC ? row : k, q0 = KC ? k : row;
+    T v[EPC];
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) v[e] = T(0);
+    if (co < cout && q0 < Q) {
+      int p;
+      const int n = P.divmod(q0, p), np = (int)P.d;
+      const T* q = go + ((int64_t)n * cout + co) * np;
+      if (p + EPC <= np) return *reinterpret_cast<const split_u32x4_any*>(q + p);
+      const int left = Q - q0;
+#pragma unroll
+      for (int e = 0; e < EPC; ++e) {
+        if (e < left) v[e] = q[p];
+        if (++p == np) {  // the next image
+          p = 0;
+          q += (int64_t)cout * np;
+        }
+      }
+    }
+    return __builtin_bit_cast(split_u32x4, v);
+  }
+};
+
+// dX by phases.  With strides sh x sw an image row y is only reached by the
+// kernel rows ky = (y + ph) mod sh + sh i, so the pixels are taken by phase
+// (y mod sh, x mod sw): within one phase the product is a stride-1 one over
+// ny x nx pixels and nky x nkx taps, with no zero taps to multiply, and
+//   oy = by + j - i   for pixel row y = fy + sh j and tap ky = ky0 + sh i.
+// Stride 1 is the one phase (0, 0) with all taps.
+struct ConvPhase {
+  int fy, fx, ky0, kx0, ny, nx, nky, nkx, by, bx;
+  __device__ __forceinline__ ConvPhase(const ConvGeom& g, int z, int phases_x) {
+    fy = z / phases_x, fx = z - fy * phases_x;
+    ky0 = (fy + g.ph) % g.sh, kx0 = (fx + g.pw) % g.sw;
+    ny = (g.H - fy + g.sh - 1) / g.sh, nx = (g.W - fx + g.sw - 1) / g.sw;
+    nky = ky0 < g.kh ? (g.kh - ky0 + g.sh - 1) / g.sh : 0;
+    nkx = kx0 < g.kw ? (g.kw - kx0 + g.sw - 1) / g.sw : 0;
+    by = (fy + g.ph - ky0) / g.sh, bx = (fx + g.pw - kx0) / g.sw;
+  }
+};
+
+// W[co, c, ky, kx]: rows c, k = (co, i, j) over the phase's taps.
+template <typename T>
+struct WeightSource {
+  static constexpr bool kKC = true;
+  const T* w;
+  ConvGeom g;
+  int cout, z0, phases_x;
+  FastDiv taps, nkx;  // nky * nkx, nkx (of the phase; at least 1)
+  int K;
+  __device__ __forceinline__ void enter(int z) {
+    const ConvPhase f(g, z0 + z, phases_x);
+    taps = FastDiv(max(1, f.nky * f.nkx)), nkx = FastDiv(max(1, f.nkx));
+    K = cout * f.nky * f.nkx;
+    w += (int64_t)f.ky0 * g.kw + f.kx0;
+  }
+  __device__ __forceinline__ split_u32x4 chunk(int row, int k) const {
+    constexpr int EPC = SplitT<T>::EPC;
+    T v[EPC];
+    int r, j;
+    const int co = taps.divmod(k, r), kk = g.kh * g.kw;
+    int i = nkx.divmod(r, j);
+    const T* p = w + ((int64_t)co * g.C + row) * kk;
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) {
+      v[e] = (row < g.C && k + e < K) ? p[(int64_t)i * g.sh * g.kw + (int64_t)j * g.sw] : T(0);
+      if (++j == (int)nkx.d) {  // next tap row, or the next output channel
+        j = 0;
+        if (++i * (int)nkx.d == (int)taps.d) {
+          i = 0;
+          p += (int64_t)g.C * kk;
+        }
+      }
+    }
+    return __builtin_bit_cast(split_u32x4, v);
+  }
+};
+
+// gO(co, i, j, p): rows p = (n, pixel of the phase), k = (co, i, j).
+template <typename T>
+struct GradImageSource {
+  static constexpr bool kKC = false, kPhased = true;
+  const T* go;
+  ConvGeom g;
+  int cout, images, z0, phases_x;
+  FastDiv taps, nkx, pix, nx;  // nky * nkx, nkx, ny * nx, nx
+  int by, bx, ny, K, Q;
+  __device__ __forceinline__ void enter(int z) {
+    const ConvPhase f(g, z0 + z, phases_x);
+    taps = FastDiv(max(1, f.nky * f.nkx)), nkx = FastDiv(max(1, f.nkx));
+    pix = FastDiv(f.ny * f.nx), nx = FastDiv(f.nx);
+    by = f.by, bx = f.bx, ny = f.ny;
+    K = cout * f.nky * f.nkx;
+    Q = images * f.ny * f.nx;
+  }
+  __device__ __forceinline__ split_u32x4 chunk(int row, int k) const {
+    constexpr int EPC = SplitT<T>::EPC;
+    T v[EPC];
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) v[e] = T(0);
+    if (k < K && row < Q) {
+      int r, j, p, x;
+      const int co = taps.divmod(k, r), i = nkx.divmod(r, j), n = pix.divmod(row, p);
+      int y = nx.divmod(p, x);
+      const int64_t P = (int64_t)g.oh * g.ow;
+      const T* pl = go + ((int64_t)n * cout + co) * P;
+      int oy = by + y - i, ox = bx + x - j;
+      if (x + EPC <= (int)nx.d && ox >= 0 && ox + EPC <= g.ow) {  // one gradient row, inside
+        if (oy >= 0 && oy < g.oh) return *reinterpret_cast<const split_u32x4_any*>(pl + (int64_t)oy * g.ow + ox);
+      } else {
+        const int left = Q - row;
+#pragma unroll
+        for (int e = 0; e < EPC; ++e) {
+          if (e < left && oy >= 0 && oy < g.oh && ox >= 0 && ox < g.ow) v[e] = pl[(int64_t)oy * g.ow + ox];
+          ++ox;
+          if (++x == (int)nx.d) {  // next pixel row, or the next image
+            x = 0;
+            ox = bx - j;
+            ++oy;
+            if (++y == ny) {
+              y = 0;
+              oy = by - i;
+              pl += cout * P;
+            }
+          }
+        }
+      }
+    }
+    return __builtin_bit_cast(split_u32x4, v);
+  }
+};
+
+// gX[n][c][y][x] for product column p = (n, pixel of the phase).
+template <typename T>
+struct PhaseEpilogue {
+  T* gx;
+  ConvGeom g;
+  int images, z0, phases_x;
+  FastDiv pix, nx;
+  __device__ __forceinline__ int columns() const { return images * (int)pix.d; }
+  __device__ __forceinline__ void enter(int z) {
+    const ConvPhase f(g, z0 + z, phases_x);
+    pix = FastDiv(f.ny * f.nx), nx = FastDiv(f.nx);
+    gx += (int64_t)f.fy * g.W + f.fx;
+  }
+  __device__ __forceinline__ void operator()(int m, int q, float acc) const {
+    int p, x;
+    const int n = pix.divmod(q, p), y = nx.divmod(p, x);
+    split_store(gx + ((int64_t)n * g.C + m) * g.H * g.W + (int64_t)y * g.sh * g.W + (int64_t)x * g.sw, acc);
+  }
+};
+
+// dX where the windows do not overlap (sh >= kh and sw >= kw): every pixel is
+// under at most one kernel position, so the product of W^T (rows kk = (c, ky,
+// kx)) and gO (columns q) scatters straight into the image.
+template <typename T>
+struct WindowEpilogue {
+  T* gx;
+  ConvGeom g;
+  FastDiv kk, kw, P, ow;
+  __device__ __forceinline__ void operator()(int m, int q, float acc) const {
+    int r, kx, p, ox;
+    const int c = kk.divmod(m, r), ky = kw.divmod(r, kx), n = P.divmod(q, p), oy = ow.divmod(p, ox);
+    const int y = oy * g.sh - g.ph + ky, x = ox * g.sw - g.pw + kx;
+    if (y >= 0 && y < g.H && x >= 0 && x < g.W)
+      split_store(gx + (((int64_t)n * g.C + c) * g.H + y) * g.W + x, acc);
+  }
+};
+
+// y[n][m][p] for product column q = (n, p): [N][M][P] planes.
+template <typename T>
+struct PlaneEpilogue {
+  T* y;
+  FastDiv P;
+  int M;
+  __device__ __forceinline__ void operator()(int m, int q, float acc) const {
+    int p;
+    const int n = P.divmod(q, p);
+    split_store(y + ((int64_t)n * M + m) * P.d + p, acc);
+  }
+};
+
+ConvDivs conv_divs(const ConvGeom& g) {
+  return ConvDivs{FastDiv(g.kh * g.kw), FastDiv(g.kw), FastDiv(g.oh * g.ow), FastDiv(g.ow)};
+}
+
+constexpr int64_t kConvPhases = 32768;  // phases per launch (the grid's z extent is 16 bits)
+
+// Images per launch: the product's columns (n, pixel) stay below 2^30.
+int64_t conv_slab(int64_t N, int64_t pixels) { return std::min(N, std::max<int64_t>(1, (int64_t(1) << 30) / pixels)); }
+
+template <typename T>
+int conv_forward(const char* fn, const T* in, const T* w, T* out, int64_t N, int cout, const ConvGeom& g,
+                 hipStream_t s) {
+  const int64_t P = (int64_t)g.oh * g.ow, K = (int64_t)g.C * g.kh * g.kw, slab = conv_slab(N, P);
+  const ConvDivs dv = conv_divs(g);
+  for (int64_t n = 0; n < N; n += slab) {
+    const int64_t Q = std::min(slab, N - n) * P;
+    const int rc = launch_split_gemm<T>(
+        fn, cout, Q, K, MatrixSource<T, true>{w, K, cout, (int)K},
+        ColumnSource<T, false>{in + n * g.C * g.H * g.W, g, dv, (int)K, (int)Q},
+        PlaneEpilogue<T>{out + n * cout * P, dv.P, cout}, s);
+    if (rc) return rc;
+  }
+  return ok();
+}
+
+template <typename T>
+int conv_backward(const char* fn, const T* in, const T* w, const T* go, T* gin, T* gw, int64_t N, int cout,
+                  const ConvGeom& g, hipStream_t s) {
+  const int64_t P = (int64_t)g.oh * g.ow, K = (int64_t)g.C * g.kh * g.kw, HW = (int64_t)g.H * g.W;
+  const ConvDivs dv = conv_divs(g);
+  int64_t slab = conv_slab(N, P);
+  for (int64_t n = 0; n < N; n += slab) {
+    const int64_t Q = std::min(slab, N - n) * P;
+    const int rc = launch_split_gemm<T>(
+        fn, cout, K, Q, GradRowSource<T, true>{go + n * cout * P, dv.P, cout, (int)Q},
+        ColumnSource<T, true>{in + n * g.C * HW, g, dv, (int)K, (int)Q},
+        MatrixEpilogue<T>{gw, nullptr, 0, 1.f, n == 0 ? 0.f : 1.f, (int)K}, s);
+    if (rc) return rc;
+  }
+  if (g.sh >= g.kh && g.sw >= g.kw) {
+    // pixels outside every window are not written by the product
+    const bool tiled = g.sh == g.kh && g.sw == g.kw && g.ph == 0 && g.pw == 0 && g.oh * g.kh == g.H && g.ow * g.kw == g.W;
+    if (!tiled) {
+      const int rc = tt_elementwise(TT_EW_FILL, sizeof(T) == 2 ? TT_BF16 : TT_F32, gin, nullptr, nullptr,
+                                    N * g.C * HW, 0.0, 0.0, 0, s);
+      if (rc) return rc;
+    }
+    for (int64_t n = 0; n < N; n += slab) {
+      const int64_t Q = std::min(slab, N - n) * P;
+      const int rc = launch_split_gemm<T>(
+          fn, K, Q, cout, MatrixSource<T, false>{w, K, (int)K, cout},
+          GradRowSource<T, false>{go + n * cout * P, dv.P, cout, (int)Q},
+          WindowEpilogue<T>{gin + n * g.C * HW, g, dv.kk, dv.kw, dv.P, dv.ow}, s);
+      if (rc) return rc;
+    }
+    return ok();
+  }
+  slab = conv_slab(N, HW);
+  const int phases_x = std::min(g.sw, g.W);
+  const int64_t phases = (int64_t)std::min(g.sh, g.H) * phases_x;
+  const int64_t pixels = (int64_t)((g.H + g.sh - 1) / g.sh) * ((g.W + g.sw - 1) / g.sw);  // of the largest phase
+  const int64_t taps = (int64_t)((g.kh + g.sh - 1) / g.sh) * ((g.kw + g.sw - 1) / g.sw);    // likewise
+  for (int64_t n = 0; n < N; n += slab) {
+    const int64_t images = std::min(slab, N - n);
+    for (int64_t z0 = 0; z0 < phases; z0 += kConvPhases) {
+      const int rc = launch_split_gemm<T>(
+          fn, g.C, images * pixels, cout * taps, WeightSource<T>{w, g, cout, (int)z0, phases_x},
+          GradImageSource<T>{go + n * cout * P, g, cout, (int)images, (int)z0, phases_x},
+          PhaseEpilogue<T>{gin + n * g.C * HW, g, (int)images, (int)z0, phases_x}, s,
+          (int)std::min<int64_t>(kConvPhases, phases - z0));
+      if (rc) return rc;
+    }
+  }
+  return ok();
+}
+
+// Clamps strides to the padded extent (a longer one also leaves one output)
+// and returns whether the products' 32-bit indices and grids cover the shape.
+bool conv_fits(ConvGeom& g, int cout) {
+  const int64_t lim = int64_t(1) << 30, kk = (int64_t)g.kh * g.kw;
+  const int64_t eh = (int64_t)g.H + 2 * (int64_t)g.ph, ew = (int64_t)g.W + 2 * (int64_t)g.pw;
+  if (eh >= lim / 2 || ew >= lim / 2 || (int64_t)g.oh * g.ow > lim || (int64_t)g.H * g.W > lim || kk > lim ||
+      g.C * kk > lim || cout * kk > lim)
+    return false;
+  g.sh = std::min(g.sh, (int)eh + 1);
+  g.sw = std::min(g.sw, (int)ew + 1);
+  return true;
+}
+
 }  // namespace
 
 }  // namespace tt
@@ -197,6 +571,45 @@ using namespace tt;
 extern "C" int tt_im2col(int dtype, const void* im, void* col, int64_t N, int C, int H, int W, int kh, int kw,
                          int pad_h, int pad_w, int stride_h, int stride_w, void* stream) {
   return conv_entry<true>("tt_im2col", dtype, im, col, N, C, H, W, kh, kw, pad_h, pad_w, stride_h, stride_w, stream);
+}
+
+extern "C" int tt_conv_forward(int dtype, const void* in, const void* weight, void* out, int64_t N, int C, int H,
+                               int W, int cout, int kh, int kw, int pad_h, int pad_w, int stride_h, int stride_w,
+                               void* stream) {
+  const char* fn = "tt_conv_forward";
+  ConvGeom g;
+  int rc = conv_geom(fn, N, C, H, W, kh, kw, pad_h, pad_w, stride_h, stride_w, g);
+  if (rc) return rc;
+  if (cout < 0) return fail(TT_ERR_ARG, std::string(fn) + ": negative output channels");
+  if (dtype != TT_F32 && dtype != TT_BF16) return fail(TT_ERR_ARG, std::string(fn) + ": dtype must be TT_F32 or TT_BF16");
+  if (N == 0 || cout == 0) return ok();
+  if (!in || !weight || !out) return fail(TT_ERR_ARG, std::string(fn) + ": null pointer");
+  if (!conv_fits(g, cout)) return fail(TT_ERR_UNSUPPORTED, std::string(fn) + ": image or kernel above 2^29 elements an axis or 2^30 in all");
+  if ((rc = ensure_init())) return rc;
+  hipStream_t s = stream_or_default(stream);
+  if (dtype == TT_F32) return conv_forward(fn, (const float*)in, (const float*)weight, (float*)out, N, cout, g, s);
+  return conv_forward(fn, (const uint16_t*)in, (const uint16_t*)weight, (uint16_t*)out, N, cout, g, s);
+}
+
+extern "C" int tt_conv_backward(int dtype, const void* in, const void* weight, const void* grad_out, void* grad_in,
+                                void* grad_weight, int64_t N, int C, int H, int W, int cout, int kh, int kw,
+                                int pad_h, int pad_w, int stride_h, int stride_w, void* stream) {
+  const char* fn = "tt_conv_backward";
+  ConvGeom g;
+  int rc = conv_geom(fn, N, C, H, W, kh, kw, pad_h, pad_w, stride_h, stride_w, g);
+  if (rc) return rc;
+  if (N < 1 || cout < 1) return fail(TT_ERR_ARG, std::string(fn) + ": N and output channels >= 1 required");
+  if (dtype != TT_F32 && dtype != TT_BF16) return fail(TT_ERR_ARG, std::string(fn) + ": dtype must be TT_F32 or TT_BF16");
+  if (!in || !weight || !grad_out || !grad_in || !grad_weight)
+    return fail(TT_ERR_ARG, std::string(fn) + ": null pointer");
+  if (!conv_fits(g, cout)) return fail(TT_ERR_UNSUPPORTED, std::string(fn) + ": image or kernel above 2^29 elements an axis or 2^30 in all");
+  if ((rc = ensure_init())) return rc;
+  hipStream_t s = stream_or_default(stream);
+  if (dtype == TT_F32)
+    return conv_backward(fn, (const float*)in, (const float*)weight, (const float*)grad_out, (float*)grad_in,
+                         (float*)grad_weight, N, cout, g, s);
+  return conv_backward(fn, (const uint16_t*)in, (const uint16_t*)weight, (const uint16_t*)grad_out,
+                       (uint16_t*)grad_in, (uint16_t*)grad_weight, N, cout, g, s);
 }
 
 extern "C" int tt_col2im(int dtype, const void* col, void* im, int64_t N, int C, int H, int W, int kh, int kw,

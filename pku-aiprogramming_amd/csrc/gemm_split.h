@@ -18,6 +18,9 @@
 //   kKC  = true:  chunk(row, k) = elements (row, k .. k + EPC - 1)
 //   kKC  = false: chunk(row, k) = elements (row .. row + EPC - 1, k)
 // so a source can be a stored matrix of either orientation or a gather.
+// A phased product (SB::kPhased) is several products in one launch: enter(z)
+// of the sources and the epilogue sets them up for product z, whose N and K
+// are then B.Q and B.K (M is common).  blockIdx.z = phase * nsplit + split.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -32,7 +35,8 @@
 namespace tt {
 
 // Tile rows TM: 64 (64 x 64, waves 2 x 2) or 32 (32 x 128, waves side by
-// side) for products of at most 32 rows.
+// side) for products of at most 32 rows.  (A 128 x 128 variant for large
+// gathered products measured slower at every convolution size tried.)
 constexpr int split_tile_cols(int tm) { return 4096 / tm; }
 
 template <typename T>
@@ -127,7 +131,7 @@ __device__ __forceinline__ bf16x8 split_operand(const u16* s, int rbase, int j) 
 // else stored [k][row].
 template <typename T, bool KC>
 struct MatrixSource {
-  static constexpr bool kKC = KC;
+  static constexpr bool kKC = KC, kPhased = false;
   const T* p;
   int64_t ld;
   int rows, K;
@@ -168,7 +172,7 @@ struct MatrixEpilogue {
 };
 
 template <typename T, int TM, class SA, class SB, class EP>
-__global__ __launch_bounds__(256) void k_split_gemm(int M, int N, int K, int kper, SA A, SB B, EP ep,
+__global__ __launch_bounds__(256) void k_split_gemm(int M, int N, int K, int nsplit, SA A, SB B, EP ep,
                                                     float* __restrict__ part) {
   constexpr int BK = SplitT<T>::BK, GROUPS = sizeof(T) == 2 ? BK / 16 : BK / 8;
   constexpr int TN = split_tile_cols(TM);
@@ -178,8 +182,22 @@ __global__ __launch_bounds__(256) void k_split_gemm(int M, int N, int K, int kpe
   __shared__ __align__(16) T sB[2][TileB::ELEMS];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int wm = TM == 64 ? 32 * (w >> 1) : 0, wn = TM == 64 ? 32 * (w & 1) : 32 * w;
-  const int kbeg = blockIdx.z * kper, kend = min(K, kbeg + kper);
+  const int wm = TM == 32 ? 0 : 32 * (w >> 1), wn = TM == 32 ? 32 * w : 32 * (w & 1);
+  int split = blockIdx.z;
+  if (part) part += (int64_t)blockIdx.z * M * N;
+  const int pitch = N;  // of a row of partial sums: the columns of the largest phase
+  if constexpr (SB::kPhased) {
+    const int phase = blockIdx.z / nsplit;
+    split = blockIdx.z - phase * nsplit;
+    A.enter(phase);
+    B.enter(phase);
+    ep.enter(phase);
+    N = B.Q;
+    K = B.K;
+    if (n0 >= N) return;  // uniform: the grid covers the largest phase
+  }
+  const int kper = ((K + BK - 1) / BK + nsplit - 1) / nsplit * BK;  // whole steps; a late split may be empty
+  const int kbeg = min(K, split * kper), kend = min(K, kbeg + kper);
   f32x16 acc = f32x16{};
   TileA ta;
   TileB tb;
@@ -220,24 +238,33 @@ __global__ __launch_bounds__(256) void k_split_gemm(int M, int N, int K, int kpe
     const int m = m0 + wm + acc_row(r, l >> 5);
     if (m >= M) continue;
     if (part)
-      part[((int64_t)blockIdx.z * M + m) * N + n] = acc[r];
+      part[(int64_t)m * pitch + n] = acc[r];
     else
       ep(m, n, acc[r]);
   }
 }
 
-// Adds the splits' sums in a fixed order and runs the epilogue.  64 outputs
-// per wave; G waves of the workgroup take the splits w, w + G, ... of the same
-// outputs and meet in LDS, 4 / G (G < 4) groups of outputs per workgroup.
-template <int G, class EP>
+// Adds the splits' sums in a fixed order and runs the epilogue, phase by
+// blockIdx.y.  64 outputs per wave; G waves of the workgroup take the splits
+// w, w + G, ... of the same outputs and meet in LDS, 4 / G (G < 4) groups of
+// outputs per workgroup.  Columns past a phase's own (PHASED) are skipped.
+template <int G, bool PHASED, class EP>
 __global__ __launch_bounds__(64 * (G < 4 ? 4 : G)) void k_split_reduce(const float* __restrict__ part, int M, int N,
                                                                        int nsplit, EP ep) {
   constexpr int W = G < 4 ? 4 : G, OUT = 64 * (W / G);  // waves and outputs per workgroup
   __shared__ float red[W][64];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = w % G;
   const int64_t total = (int64_t)M * N, i = (int64_t)blockIdx.x * OUT + 64 * (w / G) + l;
+  const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
+  int cols = N;
+  if constexpr (PHASED) {
+    ep.enter(blockIdx.y);
+    cols = ep.columns();
+    part += blockIdx.y * nsplit * total;
+  }
+  const bool in = i < total && n < cols;
   float s = 0.f;
-  if (i < total) {
+  if (in) {
 #pragma unroll 8
     for (int z = g; z < nsplit; z += G) s += part[z * total + i];
   }
@@ -248,11 +275,13 @@ __global__ __launch_bounds__(64 * (G < 4 ? 4 : G)) void k_split_reduce(const flo
 #pragma unroll
     for (int k = 1; k < G; ++k) s += red[w + k][l];
   }
-  if (i < total) ep((int)(i / N), (int)(i % N), s);
+  if (in) ep(m, n, s);
 }
 
 // Splits of the contraction for a grid of `tiles` tiles and nk BK-steps:
-// about two workgroups per CU in all, each with at least two steps.
+// about two workgroups per CU in all, each with at least two steps.  (Three
+// or four per CU: bf16 1536^3 22 -> 31 us, fp32 1500^3 106 -> 93 us, most sizes
+// within 5 %.)
 inline int split_count(int64_t tiles, int64_t nk) {
   int64_t s = (512 + tiles - 1) / (tiles > 0 ? tiles : 1);
   if (s > nk / 2) s = nk / 2;
@@ -265,17 +294,20 @@ inline int split_count(int64_t tiles, int64_t nk) {
 // below 1024; a tile is 16 KB).  One fixed size per stream, so the buffer is allocated once.
 constexpr size_t kSplitWorkBytes = size_t(16) << 20;
 
-// Launches the product on s.  Without scratch (a refused allocation, or a
-// stream under capture, where nothing may be allocated and a captured
-// address must not outlive the buffer) the contraction is not split.
+// Launches the product on s: N columns and K contraction values (of the
+// largest phase), `phases` phases (1 unless SB::kPhased).  Without scratch (a
+// refused allocation, or a stream under capture, where nothing may be
+// allocated and a captured address must not outlive the buffer) the
+// contraction is not split.
 template <typename T, int TM, class SA, class SB, class EP>
-int launch_split_tiles(const char* fn, int64_t M, int64_t N, int64_t K, const SA& A, const SB& B, const EP& ep,
-                      hipStream_t s) {
+int launch_split_tiles(const char* fn, int64_t M, int64_t N, int64_t K, int phases, const SA& A, const SB& B,
+                       const EP& ep, hipStream_t s) {
   constexpr int BK = SplitT<T>::BK, TN = split_tile_cols(TM);
   const int64_t gx = (N + TN - 1) / TN, gy = (M + TM - 1) / TM;
-  if (!grid_fits(gx, 256) || gy > 65535) return fail(TT_ERR_ARG, std::string(fn) + ": too large");
   const int64_t nk = (K + BK - 1) / BK;
-  int nsplit = split_count(gx * gy, nk);
+  int nsplit = split_count(gx * gy * phases, nk);
+  if (!grid_fits(gx, 256) || gy > 65535 || (int64_t)phases * nsplit > 65535)
+    return fail(TT_ERR_ARG, std::string(fn) + ": too large");
   float* part = nullptr;
   std::optional<WorkspaceLease> ws;  // held until the reduction is queued
   if (nsplit > 1 &&
@@ -283,33 +315,31 @@ int launch_split_tiles(const char* fn, int64_t M, int64_t N, int64_t K, const SA
     nsplit = 1;
     part = nullptr;
   }
-  const int64_t per = (nk + nsplit - 1) / nsplit;
-  if (nsplit > 1) nsplit = (int)((nk + per - 1) / per);
-  const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)nsplit);
-  hipLaunchKernelGGL((k_split_gemm<T, TM, SA, SB, EP>), grid, dim3(256), 0, s, (int)M, (int)N, (int)K, (int)(per * BK),
-                     A, B, ep, part);
+  hipLaunchKernelGGL((k_split_gemm<T, TM, SA, SB, EP>), dim3((unsigned)gx, (unsigned)gy, (unsigned)(phases * nsplit)),
+                     dim3(256), 0, s, (int)M, (int)N, (int)K, nsplit, A, B, ep, part);
   TT_LAUNCHED(fn, s);
   if (nsplit > 1) {
     const int64_t waves = (M * N + 63) / 64;
     const float* p = part;
+    constexpr bool PH = SB::kPhased;
     if (nsplit >= 64)
-      hipLaunchKernelGGL((k_split_reduce<16, EP>), dim3((unsigned)waves), dim3(1024), 0, s, p, (int)M, (int)N, nsplit,
-                         ep);
+      hipLaunchKernelGGL((k_split_reduce<16, PH, EP>), dim3((unsigned)waves, (unsigned)phases), dim3(1024), 0, s, p,
+                         (int)M, (int)N, nsplit, ep);
     else if (nsplit >= 16)
-      hipLaunchKernelGGL((k_split_reduce<4, EP>), dim3((unsigned)waves), dim3(256), 0, s, p, (int)M, (int)N, nsplit,
-                         ep);
+      hipLaunchKernelGGL((k_split_reduce<4, PH, EP>), dim3((unsigned)waves, (unsigned)phases), dim3(256), 0, s, p,
+                         (int)M, (int)N, nsplit, ep);
     else
-      hipLaunchKernelGGL((k_split_reduce<1, EP>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, p, (int)M,
-                         (int)N, nsplit, ep);
+      hipLaunchKernelGGL((k_split_reduce<1, PH, EP>), dim3((unsigned)((waves + 3) / 4), (unsigned)phases), dim3(256),
+                         0, s, p, (int)M, (int)N, nsplit, ep);
     TT_LAUNCHED(fn, s);
   }
   return ok();
 }
 template <typename T, class SA, class SB, class EP>
 int launch_split_gemm(const char* fn, int64_t M, int64_t N, int64_t K, const SA& A, const SB& B, const EP& ep,
-                      hipStream_t s) {
-  if (M <= 32) return launch_split_tiles<T, 32>(fn, M, N, K, A, B, ep, s);
-  return launch_split_tiles<T, 64>(fn, M, N, K, A, B, ep, s);
+                      hipStream_t s, int phases = 1) {
+  if (M <= 32) return launch_split_tiles<T, 32>(fn, M, N, K, phases, A, B, ep, s);
+  return launch_split_tiles<T, 64>(fn, M, N, K, phases, A, B, ep, s);
 }
 
 }  // namespace tt

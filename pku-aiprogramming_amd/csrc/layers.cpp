@@ -403,12 +403,18 @@ void ConvForward(const TinyTensor<T>& input, TinyTensor<T>& output, const TinyTe
   oshape.insert(oshape.end(), {d.cout, d.oh, d.ow});
   output.resize(oshape);
   if (d.in.batch == 0 || d.cout == 0) return;
-  const int64_t P = d.P(), K = d.K();
-  TinyTensor<T> col(std::vector<int>{(int)d.in.batch, (int)P, (int)K}, "gpu");
-  im2col_call(fn, input.p_data, col.p_data, d.in, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w);
-  for (int64_t n = 0; n < d.in.batch; ++n)
-    gemm<T>(fn.c_str(), false, true, d.cout, P, K, 1.f, weight.p_data, col.p_data + n * P * K, 0.f,
-            output.p_data + n * d.cout * P);
+  const int rc = tt_conv_forward(dtype_code<T>(), input.p_data, weight.p_data, output.p_data, d.in.batch, d.in.C,
+                                 d.in.H, d.in.W, d.cout, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w, nullptr);
+  if (rc == TT_ERR_UNSUPPORTED) {  // planes past its 32-bit indices: column matrix and one product per image
+    const int64_t P = d.P(), K = d.K();
+    TinyTensor<T> col(std::vector<int>{(int)d.in.batch, (int)P, (int)K}, "gpu");
+    im2col_call(fn, input.p_data, col.p_data, d.in, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w);
+    for (int64_t n = 0; n < d.in.batch; ++n)
+      gemm<T>(fn.c_str(), false, true, d.cout, P, K, 1.f, weight.p_data, col.p_data + n * P * K, 0.f,
+              output.p_data + n * d.cout * P);
+  } else {
+    tt_check(rc, fn.c_str());
+  }
   tt_check(tt_sync(), fn.c_str());
 }
 
@@ -435,16 +441,23 @@ void ConvBackward(const TinyTensor<T>& input, const TinyTensor<T>& output, const
     tt_check(tt_sync(), fn.c_str());
     return;
   }
-  TinyTensor<T> col(std::vector<int>{(int)d.in.batch, (int)P, (int)K}, "gpu");
-  im2col_call(fn, input.p_data, col.p_data, d.in, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w);
-  TinyTensor<T> grad_col(std::vector<int>{(int)d.in.batch, (int)P, (int)K}, "gpu");
-  for (int64_t n = 0; n < d.in.batch; ++n) {
-    const T* go = grad_output.p_data + n * d.cout * P;
-    gemm<T>(fn.c_str(), false, false, d.cout, K, P, 1.f, go, col.p_data + n * P * K, n == 0 ? 0.f : 1.f,
-            grad_weight.p_data);
-    gemm<T>(fn.c_str(), true, false, P, K, d.cout, 1.f, go, weight.p_data, 0.f, grad_col.p_data + n * P * K);
+  const int rc = tt_conv_backward(dtype_code<T>(), input.p_data, weight.p_data, grad_output.p_data, grad_input.p_data,
+                                  grad_weight.p_data, d.in.batch, d.in.C, d.in.H, d.in.W, d.cout, d.kh, d.kw, pad_h,
+                                  pad_w, stride_h, stride_w, nullptr);
+  if (rc == TT_ERR_UNSUPPORTED) {  // as in ConvForward
+    TinyTensor<T> col(std::vector<int>{(int)d.in.batch, (int)P, (int)K}, "gpu");
+    im2col_call(fn, input.p_data, col.p_data, d.in, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w);
+    TinyTensor<T> grad_col(std::vector<int>{(int)d.in.batch, (int)P, (int)K}, "gpu");
+    for (int64_t n = 0; n < d.in.batch; ++n) {
+      const T* go = grad_output.p_data + n * d.cout * P;
+      gemm<T>(fn.c_str(), false, false, d.cout, K, P, 1.f, go, col.p_data + n * P * K, n == 0 ? 0.f : 1.f,
+              grad_weight.p_data);
+      gemm<T>(fn.c_str(), true, false, P, K, d.cout, 1.f, go, weight.p_data, 0.f, grad_col.p_data + n * P * K);
+    }
+    col2im_call(fn, grad_col.p_data, grad_input.p_data, d.in, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w);
+  } else {
+    tt_check(rc, fn.c_str());
   }
-  col2im_call(fn, grad_col.p_data, grad_input.p_data, d.in, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w);
   tt_check(tt_sync(), fn.c_str());
 }
 

@@ -1,0 +1,77 @@
+"""GPU tests of the gathered convolution products (tt_conv_forward /
+tt_conv_backward, csrc/conv.hip) where they can go wrong: channel counts
+around the 32- and 64-row tiles, chunks that cross image rows and images,
+strides with uneven phases, phases without taps, windows that do not overlap
+or leave pixels uncovered, sums split over workgroups.  Reference: numpy
+float64 on the same (for bf16: bf16-rounded) values.  Bars (normwise
+max|x - ref| / max|ref|): fp32 1e-5 (fp32 products and sums), bf16 8e-3 (one
+rounding of the result)."""
+import numpy as np
+import pytest
+
+from oracle import attn_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+TOL = {"float": 1e-5, "bf16": 8e-3}
+
+# (N, Cin, H, W, Cout, kh, kw, pad_h, pad_w, stride_h, stride_w)
+CASES = [
+    (3, 1, 5, 5, 1, 1, 1, 0, 0, 1, 1),       # 1 x 1: windows do not overlap
+    (2, 33, 6, 7, 31, 3, 3, 1, 1, 1, 1),     # rows past the 32-row tile, rows of 7 pixels
+    (2, 65, 5, 3, 64, 3, 1, 1, 0, 1, 1),     # past the 64-row tile
+    (5, 3, 11, 13, 6, 5, 5, 2, 2, 2, 2),     # uneven phases
+    (2, 4, 10, 9, 5, 3, 2, 0, 1, 2, 1),      # stride in one axis
+    (2, 3, 13, 13, 4, 3, 3, 1, 1, 4, 3),     # gaps between windows in one axis
+    (2, 3, 16, 12, 5, 4, 3, 0, 0, 4, 3),     # windows tile the image
+    (2, 3, 17, 14, 5, 4, 3, 1, 0, 4, 3),     # windows tile it with a pad and a remainder
+    (1, 2, 4, 4, 3, 2, 2, 0, 0, 9, 9),       # stride past the image: one output pixel
+    (1, 2, 6, 5, 3, 6, 5, 0, 0, 2, 2),       # kernel as large as the image
+    (4, 2, 40, 40, 3, 3, 3, 1, 1, 1, 1),     # dW sums 6400 pixels over many splits
+    (1, 200, 7, 7, 40, 3, 3, 1, 1, 1, 1),    # dX splits its contraction
+    (1, 40, 14, 14, 200, 3, 3, 1, 1, 2, 2),  # and by phases
+]
+
+
+def _ref(x, w, go, ph, pw, sh, sw):
+    N, C, H, W = x.shape
+    Co, _, kh, kw = w.shape
+    oh, ow = (H + 2 * ph - kh) // sh + 1, (W + 2 * pw - kw) // sw + 1
+    xp = np.zeros((N, C, H + 2 * ph, W + 2 * pw))
+    xp[:, :, ph:ph + H, pw:pw + W] = x
+    out, gw, gxp = np.zeros((N, Co, oh, ow)), np.zeros(w.shape), np.zeros(xp.shape)
+    for ky in range(kh):
+        for kx in range(kw):
+            at = (slice(None), slice(None), slice(ky, ky + sh * (oh - 1) + 1, sh), slice(kx, kx + sw * (ow - 1) + 1, sw))
+            out += np.einsum("oc,ncyx->noyx", w[:, :, ky, kx], xp[at])
+            gw[:, :, ky, kx] = np.einsum("noyx,ncyx->oc", go, xp[at])
+            gxp[at] += np.einsum("oc,noyx->ncyx", w[:, :, ky, kx], go)
+    return out, gw, gxp[:, :, ph:ph + H, pw:pw + W]
+
+
+@pytest.mark.parametrize("dt", ["float", "bf16"])
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_conv_products(dt, case):
+    import myLayer as ml
+    import myTensor as mt
+
+    T = getattr(mt, "Tensor_" + dt)
+    N, C, H, W, Co, kh, kw, ph, pw, sh, sw = case
+    rng = np.random.default_rng(sum(case))
+    oh, ow = (H + 2 * ph - kh) // sh + 1, (W + 2 * pw - kw) // sw + 1
+    x, w, go = (rng.standard_normal(s).astype(np.float32) for s in ((N, C, H, W), (Co, C, kh, kw), (N, Co, oh, ow)))
+    if dt == "bf16":
+        x, w, go = orc.bf16_round(x), orc.bf16_round(w), orc.bf16_round(go)
+    X, Wt, GO = (T(a, "gpu") for a in (x, w, go))
+    out, gx, gw = (T([1], "gpu") for _ in range(3))
+    ml.ConvForward(X, out, Wt, ph, pw, sh, sw)
+    ml.ConvBackward(X, out, Wt, gx, GO, gw, ph, pw, sh, sw)
+    ref = _ref(x.astype(np.float64), w.astype(np.float64), go.astype(np.float64), ph, pw, sh, sw)
+    for name, got, r in zip(("out", "grad_weight", "grad_input"), (out, gw, gx), ref):
+        a = np.asarray(got.numpy()).reshape(r.shape)
+        if r.size == 0 or not np.any(r):
+            assert not np.any(a)
+            continue
+        e = orc.max_rel_err(a, r)
+        print(f"  {name} {e:.2e}", flush=True)
+        assert e <= TOL[dt], (name, e)
