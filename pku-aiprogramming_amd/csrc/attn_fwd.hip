@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <optional>
 #include <type_traits>
 
 #include "attn_common.h"
@@ -51,11 +52,18 @@ constexpr int FWD_F32_BM = 128;  // queries per workgroup of the fp32 kernel
 // body (an explicit sched_group_barrier pattern measured 3 % slower).
 constexpr int FWDP_NW = 4;
 
-template <int D, bool CAUSAL, int NW>
+//
+// SPLIT: the key tiles of each query tile are shared out over nsplit
+// workgroups (workgroup id = split * nqt * BH + tile id), each writing its
+// unnormalised fp32 O, running max and row sum to `part` for the combine
+// kernel: few query tiles against many keys (B = 2, H = 16, 77 queries, 4099
+// keys: 32 tiles) then fill the chip.  A causal workgroup's last split takes
+// both diagonal tiles, so every wave has a key tile in every non-empty split.
+template <int D, bool CAUSAL, int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
     const u16* __restrict__ Q, const u16* __restrict__ K, const u16* __restrict__ V,
     u16* __restrict__ O, float* __restrict__ LSE, int Lq, int Lk, int BH, int nqt, int order,
-    float sl2) {
+    float sl2, int nsplit, float* __restrict__ part) {
   using Tile = SwzTile<D>;
   constexpr int BM = 32 * NW, BN = 64;
   constexpr int NC = D / 16, ND = D / 32;
@@ -68,10 +76,31 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63, g = l >> 5, r32 = l & 31;
   int qt, bh;
-  map_tile(blockIdx.x, nqt, BH, order, qt, bh, CAUSAL);
+  const int split = SPLIT ? blockIdx.x / (nqt * BH) : 0;
+  map_tile(SPLIT ? blockIdx.x - split * (nqt * BH) : blockIdx.x, nqt, BH, order, qt, bh, CAUSAL);
   const int q0 = qt * BM, wq0 = q0 + 32 * w, qrow = wq0 + r32;
   const int64_t qbase = (int64_t)bh * Lq * D;
-  const int64_t kbase = (int64_t)bh * Lk * D;
+  int64_t kbase = (int64_t)bh * Lk * D;
+  // SPLIT: keys from here on are counted from this split's first one
+  int k_first = 0;
+  if constexpr (SPLIT) {
+    const int kend = CAUSAL ? min(Lk, q0 + BM) : Lk;
+    // units of one tile, the last of a causal range two (its diagonal tiles)
+    const int units = max(1, (kend + BN - 1) / BN - (CAUSAL ? 1 : 0));
+    const int lo = (int)((int64_t)units * split / nsplit), hi = (int)((int64_t)units * (split + 1) / nsplit);
+    if (lo == hi) {  // uniform: no keys for this split
+      if (threadIdx.x < BM && q0 + (int)threadIdx.x < Lq) {
+        float* ml = part + (int64_t)nsplit * BH * Lq * D + 2 * (((int64_t)split * BH + bh) * Lq + q0 + threadIdx.x);
+        ml[0] = -INFINITY;
+        ml[1] = -1.f;  // marks O_s as unset
+      }
+      return;
+    }
+    k_first = BN * lo;
+    kbase += (int64_t)k_first * D;
+    if (hi < units) Lk = min(Lk, BN * hi);  // keys of later splits do not exist here
+    Lk -= k_first;
+  }
 
   bf16x8 qf[NC];
   {
@@ -81,12 +110,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
       qf[c] = __builtin_bit_cast(bf16x8, ldg16(Q + qbase + (int64_t)qr * D + 16 * c + 8 * g));
   }
 
-  const int kend = CAUSAL ? min(Lk, q0 + BM) : Lk;  // >= 1: Lk >= 1, and q0 < Lq = Lk when causal
+  const int kend = CAUSAL ? min(Lk, q0 + BM - k_first) : Lk;  // >= 1: Lk >= 1, and q0 < Lq = Lk when causal
   const int ntiles = (kend + BN - 1) / BN;
   // Last tile this wave computes: its diagonal tile (causal) or the last
   // tile.  Every earlier tile lies inside Lk and before every query of the
   // wave, so only the last one can need a mask.
-  const int last = CAUSAL ? min(wq0 / BN, ntiles - 1) : ntiles - 1;
+  const int last = CAUSAL ? min((wq0 - k_first) / BN, ntiles - 1) : ntiles - 1;
   const bool mask_last = CAUSAL || (Lk % BN) != 0;
 
   // Per-lane LDS element offsets.  K operand of chunk c: key row r32 (+32
@@ -136,7 +165,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int key = kb + 32 * t + acc_row(r, g);
-        if (key >= Lk || (CAUSAL && key > qrow)) s[t][r] = -INFINITY;
+        if (key >= Lk || (CAUSAL && key > qrow - k_first)) s[t][r] = -INFINITY;
       }
   };
   // Running max per query, in the log2 domain.  It moves only when some
@@ -316,6 +345,24 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
   wait_vmem_le<0>();  // nothing may be in flight into LDS when the workgroup exits
 
   const float ls = sum_xor32(lsum);
+  if constexpr (SPLIT) {
+    if (qrow < Lq) {
+      const int64_t row = ((int64_t)split * BH + bh) * Lq + qrow;
+      float* orow = part + row * D;
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4)
+          *reinterpret_cast<f32x4*>(orow + 32 * dt + acc_row(r, g)) =
+              f32x4{o[dt][r], o[dt][r + 1], o[dt][r + 2], o[dt][r + 3]};
+      if (g == 0) {
+        float* ml = part + (int64_t)nsplit * BH * Lq * D + 2 * row;
+        ml[0] = m;
+        ml[1] = ls;
+      }
+    }
+    return;
+  }
   const float inv = ls > 0.f ? 1.f / ls : 0.f;
   if (qrow < Lq && g == 0 && LSE) LSE[(int64_t)bh * Lq + qrow] = (m + __log2f(ls)) * kLn2;
   if constexpr (D >= 128) {
@@ -522,52 +569,83 @@ __global__ __launch_bounds__(256, (D >= 128 ? 1 : 2)) void attn_fwd_f32_kernel(
   }
 }
 
-// Merges the nsplit partial results of the split fp32 forward: per query
-// row, with M = max of the splits' running maxima, O = sum_s 2^(m_s - M) O_s /
-// sum_s 2^(m_s - M) l_s and LSE = (M + log2 of that denominator) ln 2.  A split
-// with no keys for the row has m_s = -inf and weight 0; split 0 always holds
-// key 0, which every query sees.  D / 4 threads per row, one float4 each.
-template <int D>
-__global__ __launch_bounds__(256) void attn_fwd_f32_combine_kernel(const float* __restrict__ part,
-                                                                   float* __restrict__ O, float* __restrict__ LSE,
-                                                                   int64_t rows, int nsplit) {
+// Merges the nsplit partial results of a split forward: per query row, with
+// M = max of the splits' running maxima, O = sum_s 2^(m_s - M) O_s / sum_s
+// 2^(m_s - M) l_s and LSE = (M + log2 of that denominator) ln 2.  A split
+// without keys has m_s = -inf; l_s < 0 marks its O_s as unset.  NaN maxima
+// propagate.  D / 4 threads per row, four columns each.
+__device__ __forceinline__ void store4(float* p, float a, float b, float c, float d) {
+  *reinterpret_cast<f32x4*>(p) = f32x4{a, b, c, d};
+}
+__device__ __forceinline__ void store4(u16* p, float a, float b, float c, float d) {
+  *reinterpret_cast<uint2*>(p) = uint2{pack_bf16x2(a, b), pack_bf16x2(c, d)};
+}
+// U splits' loads are in flight at a time.
+template <typename T, int D, int U>
+__global__ __launch_bounds__(256) void attn_fwd_combine_kernel(const float* __restrict__ part, T* __restrict__ O,
+                                                               float* __restrict__ LSE, int64_t rows, int nsplit) {
   constexpr int TPR = D / 4;
   const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
   const int c = threadIdx.x % TPR;
   if (row >= rows) return;
   const float* ml = part + (int64_t)nsplit * rows * D;
   float mx = -INFINITY;
-  for (int sp = 0; sp < nsplit; ++sp) mx = fmaxf(mx, ml[2 * (sp * rows + row)]);
+#pragma unroll U
+  for (int sp = 0; sp < nsplit; ++sp) mx = vmax(mx, ml[2 * (sp * rows + row)]);
+  const float mb = mx == -INFINITY ? 0.f : mx;
   float den = 0.f;
-  float4 num = {0.f, 0.f, 0.f, 0.f};
-  for (int sp = 0; sp < nsplit; ++sp) {
-    const int64_t pr = sp * rows + row;
-    const float wgt = fast_exp2(ml[2 * pr] - mx);  // 0 for an empty split (m = -inf)
-    den += wgt * ml[2 * pr + 1];
-    const float4 o = *reinterpret_cast<const float4*>(part + pr * D + 4 * c);
-    num.x += wgt * o.x;
-    num.y += wgt * o.y;
-    num.z += wgt * o.z;
-    num.w += wgt * o.w;
+  f32x4 num = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < nsplit; s0 += U) {
+    f32x4 o[U];
+    float ms[U], ls[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t pr = min(s0 + u, nsplit - 1) * rows + row;
+      ms[u] = ml[2 * pr];
+      ls[u] = ml[2 * pr + 1];
+      o[u] = *reinterpret_cast<const f32x4*>(part + pr * D + 4 * c);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s0 + u >= nsplit || ls[u] < 0.f) continue;
+      const float wgt = fast_exp2(ms[u] - mb);
+      den += wgt * ls[u];
+      num += wgt * o[u];
+    }
   }
   const float inv = den > 0.f ? 1.f / den : 0.f;
-  *reinterpret_cast<float4*>(O + row * D + 4 * c) = float4{num.x * inv, num.y * inv, num.z * inv, num.w * inv};
+  store4(O + row * D + 4 * c, num.x * inv, num.y * inv, num.z * inv, num.w * inv);
   if (c == 0 && LSE) LSE[row] = (mx + __log2f(den)) * kLn2;
 }
 
-template <typename T, typename KernelPtr>
-static int launch_fwd(KernelPtr kern, int bm, int threads, int wg_per_cu, int light_div, const T* q, const T* k,
-                      const T* v, T* o, float* lse, int64_t BH, int64_t Lq, int64_t Lk, float scale, hipStream_t s) {
-  const int64_t nqt = (Lq + bm - 1) / bm;
-  const int64_t nblk = nqt * BH;
-  if (!grid_fits(nblk, threads)) return fail(TT_ERR_ARG, "attention forward: grid too large");
-  // heads in flight per XCD: enough tiles for the resident workgroups of its
-  // 32 CUs
-  const int order = tile_order(BH, nqt, 32 * wg_per_cu, light_div);
-  hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(threads), 0, s, q, k, v, o, lse, (int)Lq, (int)Lk,
-                     (int)BH, (int)nqt, order, scale * kLog2e);
-  TT_LAUNCHED("attention forward launch", s);
+template <typename T, int D>
+static int launch_fwd_combine(const float* part, T* o, float* lse, int64_t rows, int nsplit, hipStream_t st) {
+  constexpr int RPB = 256 / (D / 4);  // rows per workgroup
+  const dim3 grid((unsigned)((rows + RPB - 1) / RPB));
+  if (nsplit <= 4)
+    hipLaunchKernelGGL((attn_fwd_combine_kernel<T, D, 4>), grid, dim3(256), 0, st, part, o, lse, rows, nsplit);
+  else
+    hipLaunchKernelGGL((attn_fwd_combine_kernel<T, D, 8>), grid, dim3(256), 0, st, part, o, lse, rows, nsplit);
+  TT_LAUNCHED("attention forward combine launch", st);
   return ok();
+}
+
+// Key splits of the bf16 forward: a workgroup takes about 0.8-1 us per key
+// tile, so with few query tiles and many keys the time is one workgroup's
+// chain; a split costs about 8 us more (a partial O of 4 D bytes a row and
+// split, written, read back and merged by a second launch).  Measured
+// (unsplit / split, us): [2,16] 77 x 4099 d = 64 (32 tiles) 53 / 17; [1,8] 128
+// x 8192 d = 128 (8) 120 / 20; [1,32] 256 x 4096 d = 128 (64) 63 / 32; causal
+// [1,8,2048] d = 128 (128) 35 / 34; but [1,12,1000] d = 64 (96) 15.9 / 16.9,
+// [1,32,512] d = 128 (128) 13.5 / 19.6, [1,16,2048] d = 64 (256) 26 / 33.  About
+// one workgroup per CU measured as fast as two, with half the partials, and
+// 16 splits as fast as 32.
+static int fwd_bf16_splits(int64_t tiles, int64_t ktiles) {
+  if (tiles > 128 || ktiles < (tiles <= 32 ? 16 : 32)) return 1;
+  int64_t n = (256 + tiles - 1) / tiles;
+  if (n > ktiles / 4) n = ktiles / 4;
+  if (n > 16) n = 16;
+  return n < 1 ? 1 : (int)n;
 }
 
 template <int D, bool CAUSAL>
@@ -577,9 +655,30 @@ static int fwd_bf16(const u16* q, const u16* k, const u16* v, u16* o, float* lse
   // kernel measured 5-10 % faster than the simpler two-stage kernel it
   // replaced there, non-causal and at L = 4096, and the same at
   // [16,16,1024,32] causal)
-  constexpr int NW = FWDP_NW;
-  return launch_fwd(attn_fwd_bf16_pipe_kernel<D, CAUSAL, NW>, 32 * NW, 64 * NW, 8 / NW,
-                    attention_light_div(CAUSAL, D), q, k, v, o, lse, BH, Lq, Lk, scale, st);
+  constexpr int NW = FWDP_NW, BM = 32 * NW;
+  const int64_t nqt = (Lq + BM - 1) / BM, tiles = nqt * BH;
+  if (!grid_fits(tiles, 64 * NW)) return fail(TT_ERR_ARG, "attention forward: grid too large");
+  // heads in flight per XCD: enough tiles for the resident workgroups of its
+  // 32 CUs
+  const int order = tile_order(BH, nqt, 32 * (8 / NW), attention_light_div(CAUSAL, D));
+  const float sl2 = scale * kLog2e;
+  const int nsplit = fwd_bf16_splits(tiles, (Lk + 63) / 64);
+  float* part = nullptr;
+  std::optional<WorkspaceLease> lease;  // held until both kernels are launched
+  if (nsplit > 1 && !stream_capturing(st) &&
+      lease.emplace().get(st, kWsForwardSplits, (size_t)(nsplit * BH * Lq) * (D + 2) * sizeof(float),
+                          (void**)&part) == TT_OK) {
+    hipLaunchKernelGGL((attn_fwd_bf16_pipe_kernel<D, CAUSAL, NW, true>), dim3((unsigned)(tiles * nsplit)),
+                       dim3(64 * NW), 0, st, q, k, v, o, lse, (int)Lq, (int)Lk, (int)BH, (int)nqt, order, sl2, nsplit,
+                       part);
+    TT_LAUNCHED("attention forward split launch", st);
+    return launch_fwd_combine<u16, D>(part, o, lse, BH * Lq, nsplit, st);
+  }
+  // without scratch (refused, or under capture) the keys are not split
+  hipLaunchKernelGGL((attn_fwd_bf16_pipe_kernel<D, CAUSAL, NW, false>), dim3((unsigned)tiles), dim3(64 * NW), 0, st, q,
+                     k, v, o, lse, (int)Lq, (int)Lk, (int)BH, (int)nqt, order, sl2, 1, nullptr);
+  TT_LAUNCHED("attention forward launch", st);
+  return ok();
 }
 
 template <int D, bool CAUSAL>
@@ -613,11 +712,7 @@ static int fwd_f32(const float* q, const float* k, const float* v, float* o, flo
   hipLaunchKernelGGL((attn_fwd_f32_kernel<D, CAUSAL>), dim3((unsigned)(ntq * nsplit)), dim3(256), 0, st, q, k, v,
                      o, lse, (int)Lq, (int)Lk, (int)BH, (int)nqt, order, sl2, (int)nsplit, part);
   TT_LAUNCHED("attention forward split launch", st);
-  constexpr int RPB = 256 / (D / 4);  // rows per combine workgroup
-  hipLaunchKernelGGL((attn_fwd_f32_combine_kernel<D>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st,
-                     (const float*)part, o, lse, rows, (int)nsplit);
-  TT_LAUNCHED("attention forward combine launch", st);
-  return ok();
+  return launch_fwd_combine<float, D>(part, o, lse, rows, (int)nsplit, st);
 }
 
 }  // namespace tt
