@@ -6,8 +6,9 @@
 // HBM bandwidth and is built to stream K and V exactly once.
 //
 // Split-KV: workgroup id = bh * nsplit + split owns keys [split*chunk, (split+1)*chunk)
-// of one head.  Phase 1 streams its K rows (16-byte non-temporal loads, TPR
-// threads per row, several rows in flight per thread) and writes the log2-domain scores
+// of one head.  (attn_decode_short_kernel below takes the problems with too
+// few heads and keys to fill the chip that way.)  Phase 1 streams its K rows
+// (16-byte non-temporal loads, TPR threads per row, several rows in flight per thread) and writes the log2-domain scores
 // to LDS; phase 2 reduces max and sum over the chunk; phase 3 streams the V
 // rows and accumulates sum_j p_j V_j.  Each split writes a normalised partial
 // (o_c, lse_c) in fp32; a combine kernel merges them by LSE rescaling:
@@ -17,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <optional>
 
 #include "attn_common.h"
 #include "attn_tiles.h"
@@ -176,29 +178,158 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_split_kernel(
   }
 }
 
-// One workgroup of D threads per (b, h): merge the nsplit partials.
+// Short splits: every K and V row of the split is loaded at once (ROWS = 8
+// rows of each per thread: 32 KB of K and of V per workgroup, the same for
+// every D and type), so that a split costs one memory latency instead of the
+// three phases above in series.  Each wave keeps its own running softmax of its rows
+// and the waves meet once, in LDS.
+constexpr int kDecRows = 8;
 template <typename T, int D>
-__global__ __launch_bounds__(D) void attn_decode_combine_kernel(const float* __restrict__ part_o,
-                                                                const float* __restrict__ part_lse,
-                                                                T* __restrict__ o, float* __restrict__ lse,
-                                                                int nsplit) {
-  const int64_t bh = blockIdx.x;
-  const int dd = threadIdx.x;
-  const float* pl = part_lse + bh * nsplit;
-  float mx = -INFINITY;
-  for (int c = 0; c < nsplit; ++c) mx = fmaxf(mx, pl[c]);
-  float sw = 0.f, acc = 0.f;
-  for (int c = 0; c < nsplit; ++c) {
-    const float wgt = fast_exp2(pl[c] - mx);
-    sw += wgt;
-    acc += wgt * part_o[(bh * nsplit + c) * D + dd];
+constexpr int dec_short_chunk() { return kDecRows * DEC_THREADS / (D / Vec16<T>::N); }
+
+template <typename T, int D>
+__global__ __launch_bounds__(DEC_THREADS) void attn_decode_short_kernel(
+    const T* __restrict__ q, const T* __restrict__ K, const T* __restrict__ V, float* __restrict__ part_o,
+    float* __restrict__ part_lse, T* __restrict__ o, float* __restrict__ lse, int Lkv, int nsplit, float sl2) {
+  constexpr int EPT = Vec16<T>::N, TPR = D / EPT, RPP = DEC_THREADS / TPR, R = kDecRows;
+  constexpr int NW = DEC_THREADS / 64;
+  __shared__ __align__(16) float s_acc[NW][D];
+  __shared__ float s_m[NW], s_l[NW];
+  const int split = blockIdx.x % nsplit;
+  const int64_t bh = blockIdx.x / nsplit;
+  const int tid = threadIdx.x, col = tid % TPR, rsub = tid / TPR, w = tid >> 6;
+  const int kbeg = split * (R * RPP), n = min(R * RPP, Lkv - kbeg);
+  const T* Kh = K + (bh * Lkv + kbeg) * D + col * EPT;
+  const T* Vh = V + (bh * Lkv + kbeg) * D + col * EPT;
+  const uint4 qx = ldg16(q + bh * D + col * EPT);
+  uint4 kx[R], vx[R];
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int j = rsub + u * RPP;
+    kx[u] = j < n ? ldg16_stream(Kh + (int64_t)j * D) : uint4{0, 0, 0, 0};
   }
-  const float val = acc / sw;
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int j = rsub + u * RPP;
+    vx[u] = j < n ? ldg16_stream(Vh + (int64_t)j * D) : uint4{0, 0, 0, 0};
+  }
+  float qv[EPT];
+  Vec16<T>::cvt(qx, qv);
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) qv[e] *= sl2;
+  float sc[R], m = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    float kf[EPT], dot = 0.f;
+    Vec16<T>::cvt(kx[u], kf);
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) dot += qv[e] * kf[e];
+#pragma unroll
+    for (int off = TPR / 2; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+    sc[u] = rsub + u * RPP < n ? dot : -INFINITY;
+    m = vmax(m, sc[u]);  // NaN scores propagate
+  }
+#pragma unroll
+  for (int off = TPR; off < 64; off <<= 1) m = vmax(m, __shfl_xor(m, off, 64));
+  const float mb = m == -INFINITY ? 0.f : m;  // no row (or none finite): every weight 0
+  float l = 0.f, acc[EPT];
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const float p = fast_exp2(sc[u] - mb);
+    float vf[EPT];
+    Vec16<T>::cvt(vx[u], vf);
+    l += p;
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) acc[e] += p * vf[e];
+  }
+#pragma unroll
+  for (int off = TPR; off < 64; off <<= 1) {
+    l += __shfl_xor(l, off, 64);
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
+  }
+  if ((tid & 63) < TPR) {
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) s_acc[w][col * EPT + e] = acc[e];
+    if (col == 0) {
+      s_m[w] = m;
+      s_l[w] = l;
+    }
+  }
+  __syncthreads();
+  if (tid >= D) return;
+  float M = s_m[0];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) M = vmax(M, s_m[i]);
+  const float Mb = M == -INFINITY ? 0.f : M;
+  float num = 0.f, den = 0.f;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    const float wgt = fast_exp2(s_m[i] - Mb);
+    den += wgt * s_l[i];
+    num += wgt * s_acc[i][tid];
+  }
+  const int64_t pidx = bh * nsplit + split;
+  if (nsplit > 1) {
+    // a split whose scores are all -inf: lse = -inf and o = 0, weight 0 in the merge
+    part_o[pidx * D + tid] = den == 0.f ? 0.f : num / den;
+    if (tid == 0) part_lse[pidx] = M + __log2f(den);
+    return;
+  }
+  const float inv = 1.f / den;
   if constexpr (sizeof(T) == 2)
-    o[bh * D + dd] = f32_to_bf16(val);
+    o[bh * D + tid] = f32_to_bf16(num * inv);
   else
-    o[bh * D + dd] = val;
-  if (dd == 0 && lse) lse[bh] = (mx + __log2f(sw)) * kLn2;
+    o[bh * D + tid] = num * inv;
+  if (tid == 0 && lse) lse[bh] = (M + __log2f(den)) * kLn2;
+}
+
+// One workgroup of 4 waves per (b, h) merges the nsplit partials: D / 4 threads
+// per partial row, 1024 / D rows side by side, which meet in LDS.  (One thread
+// per column walking the splits in turn took 6 us for 17 splits and 40 us for
+// 128.)
+template <typename T, int D>
+__global__ __launch_bounds__(256) void attn_decode_combine_kernel(const float* __restrict__ part_o,
+                                                                  const float* __restrict__ part_lse,
+                                                                  T* __restrict__ o, float* __restrict__ lse,
+                                                                  int nsplit) {
+  constexpr int TPR = D / 4, G = 256 / TPR;
+  __shared__ __align__(16) float s_acc[G][D];
+  __shared__ float s_w[G];
+  const int64_t bh = blockIdx.x;
+  const int tid = threadIdx.x, c = tid % TPR, g = tid / TPR;
+  const float* pl = part_lse + bh * nsplit;
+  const float* po = part_o + bh * nsplit * D + 4 * c;
+  float mx = -INFINITY;  // every wave forms the maximum by itself
+  for (int s = tid & 63; s < nsplit; s += 64) mx = vmax(mx, pl[s]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mx = vmax(mx, __shfl_xor(mx, off, 64));
+  float sw = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = g; s < nsplit; s += G) {
+    const float wgt = fast_exp2(pl[s] - mx);
+    sw += wgt;
+    acc += wgt * *reinterpret_cast<const f32x4*>(po + (int64_t)s * D);
+  }
+  *reinterpret_cast<f32x4*>(&s_acc[g][4 * c]) = acc;
+  if (c == 0) s_w[g] = sw;
+  __syncthreads();
+  if (tid >= D) return;
+  float num = 0.f, den = 0.f;
+#pragma unroll
+  for (int i = 0; i < G; ++i) {
+    num += s_acc[i][tid];
+    den += s_w[i];
+  }
+  const float val = num / den;
+  if constexpr (sizeof(T) == 2)
+    o[bh * D + tid] = f32_to_bf16(val);
+  else
+    o[bh * D + tid] = val;
+  if (tid == 0 && lse) lse[bh] = (mx + __log2f(den)) * kLn2;
 }
 
 template <typename T, int D>
@@ -216,13 +347,38 @@ static int launch_decode(const T* q, const T* k, const T* v, T* o, float* lse, i
       chunk = c;
       break;
     }
+  // Fewer than 1024 such workgroups: short splits, which cost one memory
+  // latency.  Measured (256-key splits / short, us, both with the parallel
+  // merge): bf16 d = 128 [1,8] x 1024 11.4 / 6.6, [1,8] x 8192 14.0 / 9.6, [1,32] x
+  // 4097 17.5 / 14.0 (544 workgroups); beyond the line [1,8] x 32768 25.0 /
+  // 27.6, [8,32] x 1024 23.1 / 23.2 (1024), [4,32] x 4096 44.8 / 43.7 (2048);
+  // and at [64,32] x 1024 160 / 175 against 1024-key splits.
+  bool is_short = chunk == 256 && splits(256) < 1024;
   if (Lkv < chunk) chunk = (int)((Lkv + 63) / 64 * 64);
-  const int64_t nsplit = (Lkv + chunk - 1) / chunk;
+  const int64_t long_splits = (Lkv + chunk - 1) / chunk;
+  int64_t nsplit = is_short ? (Lkv + dec_short_chunk<T, D>() - 1) / dec_short_chunk<T, D>() : long_splits;
   if (!grid_fits(BH * nsplit, DEC_THREADS)) return fail(TT_ERR_ARG, "attention decode: grid too large");
   const float sl2 = scale * kLog2e;
+  void* ws = nullptr;
+  std::optional<WorkspaceLease> lease;  // held until both kernels are launched
+  if (nsplit > 1) {
+    // A head that one long split covers runs without scratch where none may be
+    // allocated (a stream under capture, a refused allocation).
+    int rc = long_splits == 1 && stream_capturing(st)
+                 ? TT_ERR_NOMEM
+                 : lease.emplace().get(st, kWsDecodePartials, (size_t)(BH * nsplit) * (D + 1) * sizeof(float), &ws);
+    if (rc && long_splits > 1) return rc;
+    if (rc) {
+      is_short = false;
+      nsplit = 1;
+    }
+  }
   const dim3 grid((unsigned)(nsplit * BH)), block(DEC_THREADS);
   if (nsplit == 1) {  // one split per head: no partials, no combine
-    if (chunk <= DEC_SMALL_CHUNK)
+    if (is_short)
+      hipLaunchKernelGGL((attn_decode_short_kernel<T, D>), grid, block, 0, st, q, k, v, nullptr, nullptr, o, lse,
+                         (int)Lkv, 1, sl2);
+    else if (chunk <= DEC_SMALL_CHUNK)
       hipLaunchKernelGGL((attn_decode_split_kernel<T, D, 8, DEC_SMALL_CHUNK, true>), grid, block, 0, st, q, k, v,
                          nullptr, nullptr, o, lse, (int)Lkv, 1, chunk, sl2);
     else
@@ -231,21 +387,19 @@ static int launch_decode(const T* q, const T* k, const T* v, T* o, float* lse, i
     TT_LAUNCHED("attention decode launch", st);
     return ok();
   }
-  void* ws = nullptr;
-  const size_t need = (size_t)(BH * nsplit) * (D + 1) * sizeof(float);
-  WorkspaceLease lease;  // held until both kernels are launched
-  int rc = lease.get(st, kWsDecodePartials, need, &ws);
-  if (rc) return rc;
   float* part_o = (float*)ws;
   float* part_lse = part_o + BH * nsplit * D;
-  if (chunk <= DEC_SMALL_CHUNK)
+  if (is_short)
+    hipLaunchKernelGGL((attn_decode_short_kernel<T, D>), grid, block, 0, st, q, k, v, part_o, part_lse, nullptr,
+                       nullptr, (int)Lkv, (int)nsplit, sl2);
+  else if (chunk <= DEC_SMALL_CHUNK)
     hipLaunchKernelGGL((attn_decode_split_kernel<T, D, 8, DEC_SMALL_CHUNK, false>), grid, block, 0, st, q, k, v,
                        part_o, part_lse, nullptr, nullptr, (int)Lkv, (int)nsplit, chunk, sl2);
   else
     hipLaunchKernelGGL((attn_decode_split_kernel<T, D, 8, DEC_MAX_CHUNK, false>), grid, block, 0, st, q, k, v,
                        part_o, part_lse, nullptr, nullptr, (int)Lkv, (int)nsplit, chunk, sl2);
   TT_LAUNCHED("attention decode split launch", st);
-  hipLaunchKernelGGL((attn_decode_combine_kernel<T, D>), dim3((unsigned)BH), dim3(D), 0, st, part_o,
+  hipLaunchKernelGGL((attn_decode_combine_kernel<T, D>), dim3((unsigned)BH), dim3(256), 0, st, part_o,
                      part_lse, o, lse, (int)nsplit);
   TT_LAUNCHED("attention decode combine launch", st);
   return ok();
