@@ -286,16 +286,18 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_short_kernel(
   if (tid == 0 && lse) lse[bh] = (M + __log2f(den)) * kLn2;
 }
 
-// One workgroup of 4 waves per (b, h) merges the nsplit partials: D / 4 threads
-// per partial row, 1024 / D rows side by side, which meet in LDS.  (One thread
-// per column walking the splits in turn took 6 us for 17 splits and 40 us for
-// 128.)
-template <typename T, int D>
-__global__ __launch_bounds__(256) void attn_decode_combine_kernel(const float* __restrict__ part_o,
+// One workgroup of NT threads per (b, h) merges the nsplit partials: D / 4
+// threads per partial row, 4 NT / D rows side by side, which meet in LDS.
+// (One thread per column walking the splits in turn took 6 us for 17 splits
+// and 40 us for 128.)  NT = 256, or max(64, D) for up to 8 splits: a decode of
+// 928 heads in two splits each took 15.3 us with 256 threads a head, 14.9 with
+// D.
+template <typename T, int D, int NT>
+__global__ __launch_bounds__(NT) void attn_decode_combine_kernel(const float* __restrict__ part_o,
                                                                   const float* __restrict__ part_lse,
                                                                   T* __restrict__ o, float* __restrict__ lse,
                                                                   int nsplit) {
-  constexpr int TPR = D / 4, G = 256 / TPR;
+  constexpr int TPR = D / 4, G = NT / TPR;
   __shared__ __align__(16) float s_acc[G][D];
   __shared__ float s_w[G];
   const int64_t bh = blockIdx.x;
@@ -332,6 +334,8 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(const float* _
   if (tid == 0 && lse) lse[bh] = (mx + __log2f(den)) * kLn2;
 }
 
+constexpr int64_t kDecShortBytes = int64_t(56) << 20;
+
 template <typename T, int D>
 static int launch_decode(const T* q, const T* k, const T* v, T* o, float* lse, int64_t BH, int64_t Lkv,
                          float scale, hipStream_t st) {
@@ -347,16 +351,25 @@ static int launch_decode(const T* q, const T* k, const T* v, T* o, float* lse, i
       chunk = c;
       break;
     }
-  // Fewer than 1024 such workgroups: short splits, which cost one memory
-  // latency.  Measured (256-key splits / short, us, both with the parallel
-  // merge): bf16 d = 128 [1,8] x 1024 11.4 / 6.6, [1,8] x 8192 14.0 / 9.6, [1,32] x
-  // 4097 17.5 / 14.0 (544 workgroups); beyond the line [1,8] x 32768 25.0 /
-  // 27.6, [8,32] x 1024 23.1 / 23.2 (1024), [4,32] x 4096 44.8 / 43.7 (2048);
-  // and at [64,32] x 1024 160 / 175 against 1024-key splits.
-  bool is_short = chunk == 256 && splits(256) < 1024;
+  // Short splits, which cost one memory latency, where 256-key ones would be
+  // few or (bf16) the keys are small.  Measured (256-key splits / short, us, both
+  // with the parallel merge): bf16 d = 128 [1,8] x 1024 11.4 / 6.6, [1,8] x 8192
+  // 14.0 / 9.6, [1,32] x 4097 17.5 / 14.0 (544 workgroups), [16,32] x 300 18.4 /
+  // 15.0 (39 MB of K), d = 32 [29,32] x 512 12.9 / 9.5 (30 MB); fp32 d = 128 [1,32] x
+  // 4097 28.2 / 24.3 (544).  Beyond the line: bf16 d = 128 [1,8] x 32768 25.0 /
+  // 27.6 (1024, 67 MB), [64,32] x 1024 160 / 175 against 1024-key splits; fp32 d = 64
+  // [16,16] x 700 16.2 / 16.5 (768), d = 32 [40,16] x 500 13.5 / 14.6 (more
+  // cross-lane steps per byte than bf16).  Nor where a head's last short split
+  // is mostly empty (bf16 d = 32 [16,32] x 513 10.7 / 11.8), or two replace one
+  // long split, no merge, of many heads (d = 128 [30,32] x 129 12.3 / 17.5).
+  const int64_t kbytes = BH * Lkv * D * (int64_t)sizeof(T);
+  bool is_short = chunk == 256 && (sizeof(T) == 2 ? splits(256) < 1024 || kbytes < kDecShortBytes : splits(256) < 640);
+  const int64_t short_splits = (Lkv + dec_short_chunk<T, D>() - 1) / dec_short_chunk<T, D>();
+  if (Lkv <= 256 && short_splits > 1 && BH >= 256) is_short = false;
+  if (short_splits > 1 && BH >= 64 && 10 * Lkv < 6 * short_splits * dec_short_chunk<T, D>()) is_short = false;
   if (Lkv < chunk) chunk = (int)((Lkv + 63) / 64 * 64);
   const int64_t long_splits = (Lkv + chunk - 1) / chunk;
-  int64_t nsplit = is_short ? (Lkv + dec_short_chunk<T, D>() - 1) / dec_short_chunk<T, D>() : long_splits;
+  int64_t nsplit = is_short ? short_splits : long_splits;
   if (!grid_fits(BH * nsplit, DEC_THREADS)) return fail(TT_ERR_ARG, "attention decode: grid too large");
   const float sl2 = scale * kLog2e;
   void* ws = nullptr;
@@ -399,8 +412,13 @@ static int launch_decode(const T* q, const T* k, const T* v, T* o, float* lse, i
     hipLaunchKernelGGL((attn_decode_split_kernel<T, D, 8, DEC_MAX_CHUNK, false>), grid, block, 0, st, q, k, v,
                        part_o, part_lse, nullptr, nullptr, (int)Lkv, (int)nsplit, chunk, sl2);
   TT_LAUNCHED("attention decode split launch", st);
-  hipLaunchKernelGGL((attn_decode_combine_kernel<T, D>), dim3((unsigned)BH), dim3(256), 0, st, part_o,
-                     part_lse, o, lse, (int)nsplit);
+  constexpr int kFew = D > 64 ? D : 64;
+  if (nsplit <= 8)
+    hipLaunchKernelGGL((attn_decode_combine_kernel<T, D, kFew>), dim3((unsigned)BH), dim3(kFew), 0, st, part_o,
+                       part_lse, o, lse, (int)nsplit);
+  else
+    hipLaunchKernelGGL((attn_decode_combine_kernel<T, D, 256>), dim3((unsigned)BH), dim3(256), 0, st, part_o,
+                       part_lse, o, lse, (int)nsplit);
   TT_LAUNCHED("attention decode combine launch", st);
   return ok();
 }
