@@ -83,6 +83,13 @@ int tt_malloc(void** ptr, size_t bytes);
  * on a caller stream that still reads or writes the block must have
  * finished (tt_stream_sync) before the block is freed. */
 int tt_free(void* ptr);
+/* The same for memory whose every use is ordered on the library stream, such
+ * as the myTensor tensors': work queued there may still use a block when it
+ * is freed, and the next tt_malloc_ordered may hand it out at once, since its
+ * owner's work follows on that stream.  tt_malloc hands such a block out only
+ * after waiting for the library stream. */
+int tt_malloc_ordered(void** ptr, size_t bytes);
+int tt_free_ordered(void* ptr);
 int tt_empty_cache(void);
 /* Bytes currently handed out / held in the cache. */
 int tt_mem_stats(size_t* in_use, size_t* cached);

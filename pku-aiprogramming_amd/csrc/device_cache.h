@@ -84,18 +84,60 @@ class BlockCache {
     const size_t cls = block_size_class(bytes);
     {
       std::lock_guard<std::mutex> lk(mu_);
-      auto it = free_.lower_bound(cls);
-      if (it != free_.end() && it->first <= 2 * cls) {
-        void* p = it->second;
-        const size_t c = it->first;
-        free_.erase(it);
-        live_[p] = c;
-        cached_ -= c;
-        in_use_ += c;
-        *ptr = p;
-        return 0;
-      }
+      if (take(free_, cls, ptr)) return 0;
     }
+    return alloc_new(cls, ptr);
+  }
+  // The same for a block of which every use is ordered on the stream that
+  // release_ordered blocks were used on.
+  int alloc_ordered(size_t bytes, void** ptr) {
+    const size_t cls = block_size_class(bytes);
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (take(ordered_, cls, ptr) || take(free_, cls, ptr)) return 0;
+    }
+    return alloc_new(cls, ptr);
+  }
+  // Whether alloc(bytes) would need a new block although settle could free one.
+  bool wants_settle(size_t bytes) {
+    const size_t cls = block_size_class(bytes);
+    std::lock_guard<std::mutex> lk(mu_);
+    return !fits(free_, cls) && fits(ordered_, cls);
+  }
+  // Make the release_ordered blocks of before this call available to alloc,
+  // after `wait` (0 = success) has waited for their stream.
+  template <class Wait>
+  int settle(Wait&& wait) {
+    std::multimap<size_t, void*> blocks;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      blocks.swap(ordered_);
+    }
+    const int rc = wait();
+    std::lock_guard<std::mutex> lk(mu_);
+    (rc ? ordered_ : free_).insert(blocks.begin(), blocks.end());
+    return rc;
+  }
+
+ private:
+  using Blocks = std::multimap<size_t, void*>;
+  static bool fits(const Blocks& list, size_t cls) {
+    auto it = list.lower_bound(cls);
+    return it != list.end() && it->first <= 2 * cls;
+  }
+  bool take(Blocks& list, size_t cls, void** ptr) {
+    auto it = list.lower_bound(cls);
+    if (it == list.end() || it->first > 2 * cls) return false;
+    void* p = it->second;
+    const size_t c = it->first;
+    list.erase(it);
+    live_[p] = c;
+    cached_ -= c;
+    in_use_ += c;
+    *ptr = p;
+    return true;
+  }
+  int alloc_new(size_t cls, void** ptr) {
     void* p = nullptr;
     int rc = be_.alloc(cls, &p);
     if (rc != 0) {
@@ -110,8 +152,13 @@ class BlockCache {
     return 0;
   }
 
+ public:
   // false if `p` is not a live block of this cache (nullptr is fine).
-  bool release(void* p) {
+  bool release(void* p) { return release_to(free_, p); }
+  bool release_ordered(void* p) { return release_to(ordered_, p); }
+
+ private:
+  bool release_to(Blocks& list, void* p) {
     if (!p) return true;
     std::lock_guard<std::mutex> lk(mu_);
     auto it = live_.find(p);
@@ -119,17 +166,21 @@ class BlockCache {
     const size_t c = it->second;
     live_.erase(it);
     in_use_ -= c;
-    free_.emplace(c, p);
+    list.emplace(c, p);
     cached_ += c;
     return true;
   }
 
-  // Return every cached (free) block to the device.
+ public:
+  // Return every cached (free) block to the device, whose release waits for
+  // work that may still use it.
   void trim() {
     std::multimap<size_t, void*> blocks;
     {
       std::lock_guard<std::mutex> lk(mu_);
       blocks.swap(free_);
+      blocks.insert(ordered_.begin(), ordered_.end());
+      ordered_.clear();
       cached_ = 0;
     }
     for (auto& kv : blocks) be_.release(kv.second);
@@ -144,7 +195,7 @@ class BlockCache {
  private:
   Backend& be_;
   std::mutex mu_;
-  std::multimap<size_t, void*> free_;
+  Blocks free_, ordered_;
   std::unordered_map<void*, size_t> live_;  // block -> class size
   size_t in_use_ = 0, cached_ = 0;
 };

@@ -18,6 +18,7 @@
 #include <sstream>
 #include <stdexcept>
 #include <type_traits>
+#include <utility>
 
 namespace py = pybind11;
 
@@ -65,7 +66,7 @@ void TinyTensor<T>::allocate() {
     p_data = new T[size > 0 ? size : 1];
   } else {
     void* p = nullptr;
-    tt_check(tt_malloc(&p, std::max<size_t>(size, 1) * sizeof(T)), "TinyTensor allocation");
+    tt_check(tt_malloc_ordered(&p, std::max<size_t>(size, 1) * sizeof(T)), "TinyTensor allocation");
     p_data = static_cast<T*>(p);
   }
 }
@@ -76,7 +77,7 @@ void TinyTensor<T>::release() {
   if (device == "cpu")
     delete[] p_data;
   else
-    tt_free(p_data);
+    tt_free_ordered(p_data);
   p_data = nullptr;
 }
 
@@ -130,6 +131,14 @@ TinyTensor<T>::TinyTensor(const TinyTensor<T>& other) : shape(other.shape), devi
     std::copy(other.p_data, other.p_data + size, p_data);
   else
     tt_check(tt_memcpy_d2d(p_data, other.p_data, size * sizeof(T)), "TinyTensor copy");
+}
+
+template <typename T>
+TinyTensor<T>::TinyTensor(TinyTensor<T>&& other) noexcept
+    : shape(std::move(other.shape)), device(other.device), p_data(other.p_data), size(other.size) {
+  other.shape.clear();
+  other.p_data = nullptr;
+  other.size = 0;
 }
 
 template <typename T>
@@ -274,7 +283,7 @@ TinyTensor<T>& TinyTensor<T>::cpu() {
       delete[] host;
       tt_check(rc, "TinyTensor.cpu");
     }
-    tt_free(p_data);
+    tt_free_ordered(p_data);
     p_data = host;
     device = "cpu";
   }
@@ -285,10 +294,10 @@ template <typename T>
 TinyTensor<T>& TinyTensor<T>::gpu() {
   if (device == "cpu") {
     void* d = nullptr;
-    tt_check(tt_malloc(&d, std::max<size_t>(size, 1) * sizeof(T)), "TinyTensor.gpu");
+    tt_check(tt_malloc_ordered(&d, std::max<size_t>(size, 1) * sizeof(T)), "TinyTensor.gpu");
     int rc = tt_memcpy_h2d(d, p_data, size * sizeof(T));
     if (rc != TT_OK) {
-      tt_free(d);
+      tt_free_ordered(d);
       tt_check(rc, "TinyTensor.gpu");
     }
     delete[] p_data;
@@ -367,50 +376,66 @@ TinyTensor<T>& TinyTensor<T>::resize(const std::vector<int>& new_shape) {
     p_data = nd;
   } else {
     void* nd = nullptr;
-    tt_check(tt_malloc(&nd, std::max<size_t>(new_size, 1) * sizeof(T)), "TinyTensor.resize");
+    tt_check(tt_malloc_ordered(&nd, std::max<size_t>(new_size, 1) * sizeof(T)), "TinyTensor.resize");
     int rc = tt_memcpy_d2d(nd, p_data, keep * sizeof(T));
     if (rc != TT_OK) {
-      tt_free(nd);
+      tt_free_ordered(nd);
       tt_check(rc, "TinyTensor.resize");
     }
-    tt_free(p_data);
+    tt_free_ordered(p_data);
     p_data = static_cast<T*>(nd);
   }
   return *this;
 }
 
 template <typename T>
+TinyTensor<T>& TinyTensor<T>::resize_output(const std::vector<int>& new_shape) {
+  const size_t new_size = shape_size(new_shape);
+  if (new_size != size) {
+    TinyTensor<T> fresh(new_shape, device);  // before the old storage goes: a refused allocation keeps it
+    std::swap(p_data, fresh.p_data);
+    size = new_size;
+  }
+  shape = new_shape;
+  return *this;
+}
+
+template <typename T>
 TinyTensor<T> TinyTensor<T>::ReluForward() const {
-  TinyTensor<T> result{*this};
-  result.apply(TT_EW_RELU, &result, nullptr, 0, 0, 0);
+  TinyTensor<T> result{shape, device};
+  result.apply(TT_EW_RELU, this, nullptr, 0, 0, 0);
+  return result;
+}
+
+template <typename T>
+TinyTensor<T> TinyTensor<T>::gradient_op(int op, const TinyTensor<T>& grad) const {
+  if (grad.size != size) throw std::invalid_argument("Shape mismatch");
+  TinyTensor<T> result{shape, device};
+  if (grad.device == device) {
+    result.apply(op, this, &grad, 0, 0, 0);
+  } else {
+    TinyTensor<T> g{grad};
+    if (device == "gpu") g.gpu(); else g.cpu();
+    result.apply(op, this, &g, 0, 0, 0);
+  }
   return result;
 }
 
 template <typename T>
 TinyTensor<T> TinyTensor<T>::ReluBackward(const TinyTensor<T>& grad) const {
-  if (grad.size != size) throw std::invalid_argument("Shape mismatch");
-  TinyTensor<T> result{*this};
-  TinyTensor<T> g{grad};
-  if (device == "gpu") g.gpu(); else g.cpu();
-  result.apply(TT_EW_RELU_BWD, &result, &g, 0, 0, 0);
-  return result;
+  return gradient_op(TT_EW_RELU_BWD, grad);
 }
 
 template <typename T>
 TinyTensor<T> TinyTensor<T>::SigmoidForward() const {
-  TinyTensor<T> result{*this};
-  result.apply(TT_EW_SIGMOID, &result, nullptr, 0, 0, 0);
+  TinyTensor<T> result{shape, device};
+  result.apply(TT_EW_SIGMOID, this, nullptr, 0, 0, 0);
   return result;
 }
 
 template <typename T>
 TinyTensor<T> TinyTensor<T>::SigmoidBackward(const TinyTensor<T>& grad) const {
-  if (grad.size != size) throw std::invalid_argument("Shape mismatch");
-  TinyTensor<T> result{*this};
-  TinyTensor<T> g{grad};
-  if (device == "gpu") g.gpu(); else g.cpu();
-  result.apply(TT_EW_SIGMOID_BWD, &result, &g, 0, 0, 0);
-  return result;
+  return gradient_op(TT_EW_SIGMOID_BWD, grad);
 }
 
 template <typename T>

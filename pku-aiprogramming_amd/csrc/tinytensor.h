@@ -99,6 +99,7 @@ class TinyTensor {
   TinyTensor(const std::vector<int>& shape, const std::string& device, const std::vector<Host>& data);
   TinyTensor(const pybind11::array_t<Host>& data, const std::string& device);
   TinyTensor(const TinyTensor<Type>& other);
+  TinyTensor(TinyTensor<Type>&& other) noexcept;  // takes the storage
   ~TinyTensor();
 
   size_t Size() const;
@@ -123,6 +124,9 @@ class TinyTensor {
   TinyTensor<Type>& mults(Host scalar);
   TinyTensor<Type>& floatks(float k);
   TinyTensor<Type>& resize(const std::vector<int>& new_shape);
+  // Sizes an output that its caller overwrites whole: as resize, without
+  // keeping the old elements.
+  TinyTensor<Type>& resize_output(const std::vector<int>& new_shape);
 
   TinyTensor<Type> ReluForward() const;
   TinyTensor<Type> ReluBackward(const TinyTensor<Type>& grad) const;
@@ -132,6 +136,7 @@ class TinyTensor {
   bool on_gpu() const { return device == "gpu"; }
 
  private:
+  TinyTensor<Type> gradient_op(int op, const TinyTensor<Type>& grad) const;
   void allocate();
   void release();
   // Elementwise op via the C-ABI (gpu) or a host loop (cpu); writes into *this.

@@ -456,9 +456,34 @@ int tt_malloc(void** ptr, size_t bytes) {
   *ptr = nullptr;
   int rc = ensure_init();
   if (rc) return rc;
+  // Blocks of freed tensors may still be in use on the library stream: before
+  // one of them goes to a caller who may use it on any stream, wait.
+  if (g_blocks.wants_settle(bytes) && !stream_capturing(g_stream)) {
+    rc = g_blocks.settle([] {
+      const hipError_t e = hipStreamSynchronize(g_stream);
+      return e == hipSuccess ? TT_OK : hip_fail(e, "hipStreamSynchronize (tt_malloc)");
+    });
+    if (rc) return rc;
+  }
   rc = g_blocks.alloc(bytes, ptr);
   if (rc) return rc;
   return ok();
+}
+
+int tt_malloc_ordered(void** ptr, size_t bytes) {
+  if (!ptr) return fail(TT_ERR_ARG, "tt_malloc_ordered: null pointer");
+  *ptr = nullptr;
+  int rc = ensure_init();
+  if (rc) return rc;
+  rc = g_blocks.alloc_ordered(bytes, ptr);
+  if (rc) return rc;
+  return ok();
+}
+
+int tt_free_ordered(void* ptr) {
+  if (!ptr) return TT_OK;
+  if (!g_blocks.release_ordered(ptr)) return fail(TT_ERR_ARG, "tt_free_ordered: pointer not from tt_malloc");
+  return TT_OK;
 }
 
 int tt_free(void* ptr) {

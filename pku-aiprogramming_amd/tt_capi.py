@@ -38,6 +38,8 @@ _SIGS = {
     "tt_stream_destroy": (C.c_int, [_p]),
     "tt_malloc": (C.c_int, [C.POINTER(_p), C.c_size_t]),
     "tt_free": (C.c_int, [_p]),
+    "tt_malloc_ordered": (C.c_int, [C.POINTER(_p), C.c_size_t]),
+    "tt_free_ordered": (C.c_int, [_p]),
     "tt_empty_cache": (C.c_int, []),
     "tt_mem_stats": (C.c_int, [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]),
     "tt_memcpy_h2d": (C.c_int, [_p, _p, C.c_size_t]),

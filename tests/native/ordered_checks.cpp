@@ -1,0 +1,52 @@
+// BlockCache's stream-ordered blocks (csrc/device_cache.h) over a malloc
+// backend: only alloc_ordered hands a release_ordered block out before
+// settle, a failed wait keeps it apart, trim returns it, counts stay whole.
+#include <cstdio>
+#include <cstdlib>
+
+#include "device_cache.h"
+
+using namespace tt;
+
+static int g_failures = 0;
+#define CHECK(cond) \
+  do { \
+    if (!(cond)) { std::fprintf(stderr, "line %d: %s\n", __LINE__, #cond); ++g_failures; } \
+  } while (0)
+
+struct Backend {
+  int releases = 0;
+  int alloc(size_t bytes, void** p) { return (*p = std::malloc(bytes)) ? 0 : 4; }
+  void release(void* p) { std::free(p), ++releases; }
+};
+
+int main() {
+  Backend be;
+  BlockCache<Backend> bc(be);
+  void *a = nullptr, *b = nullptr, *c = nullptr;
+  CHECK(bc.alloc_ordered(4096, &a) == 0);
+  CHECK(!bc.wants_settle(4096));
+  CHECK(bc.release_ordered(a) && !bc.release_ordered(a) && !bc.release(a));
+  CHECK(bc.wants_settle(4096) && !bc.wants_settle(1 << 20));
+  CHECK(bc.alloc(4096, &b) == 0 && b != a);          // never before settle
+  CHECK(bc.settle([] { return 5; }) == 5);           // a failed wait
+  CHECK(bc.alloc(4096, &c) == 0 && c != a);
+  CHECK(bc.release(c));
+  CHECK(!bc.wants_settle(4096));                     // an ordinary block serves it
+  CHECK(bc.alloc_ordered(4096, &c) == 0 && c == a);  // the ordered block first
+  CHECK(bc.release_ordered(c));
+  CHECK(bc.settle([] { return 0; }) == 0);
+  size_t used = 0, cached = 0;
+  bc.stats(&used, &cached);
+  CHECK(used == 4096 && cached == 8192);
+  CHECK(bc.alloc(4096, &a) == 0 && bc.alloc(4096, &c) == 0);  // both cached blocks
+  bc.stats(&used, &cached);
+  CHECK(used == 3 * 4096 && cached == 0);
+  CHECK(bc.release_ordered(a) && bc.release(b) && bc.release_ordered(c));
+  bc.trim();
+  CHECK(be.releases == 3);
+  bc.stats(&used, &cached);
+  CHECK(used == 0 && cached == 0);
+  if (!g_failures) std::puts("ordered checks passed");
+  return g_failures ? 1 : 0;
+}
