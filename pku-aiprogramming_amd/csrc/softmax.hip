@@ -14,10 +14,10 @@
 //   cols <= 64:   G = the next power of two >= cols lanes per row, 64 / G
 //                 rows per wave, one element per lane;
 //   cols <= 2048: one wave per row, up to 32 elements per lane in registers;
-//   cols <= 8192 (and longer rows that are not 16-byte aligned, up to 65536):
-//                 one workgroup of 4 or 16 waves per row, up to 64 elements
-//                 per lane in registers, partials through LDS;
-//   longer aligned rows, up to 2 M columns: the row is split over up to 64
+//   cols <= 8192 (up to 65536 where rows are not split, below): one workgroup
+//                 of 4 or 16 waves per row, up to 64 elements per lane in
+//                 registers, partials through LDS;
+//   longer rows, up to 2 M columns: the row is split over up to 64
 //                 workgroups that each hold their chunk in registers and
 //                 exchange (max, sum) partials through device memory (one
 //                 HBM read and one write per element);
@@ -27,6 +27,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <optional>
 
 #include "tt_internal.h"
 
@@ -243,8 +244,13 @@ __global__ __launch_bounds__(64 * W) void k_softmax_stream(const float* __restri
 // already read, so x == y (in place) is fine.
 constexpr int kSplitMaxChunks = 64;
 typedef float f32x4v __attribute__((ext_vector_type(4)));
+// four floats at any float alignment (the target reads and writes unaligned
+// global words)
+typedef f32x4v f32x4u __attribute__((aligned(4)));
 
-template <int NE4>
+// ALIGNED: cols % 4 == 0 and 16-byte aligned x and y.  Otherwise rows begin
+// at any float and a row's last vector may be partial.
+template <int NE4, bool ALIGNED>
 __global__ __launch_bounds__(kBlock) void k_softmax_split(const float* x, float* y, int64_t cols, int nchunk,
                                                          unsigned long long* slots, unsigned gen) {
   constexpr int CW = 1024 * NE4;  // columns per chunk
@@ -259,9 +265,17 @@ __global__ __launch_bounds__(kBlock) void k_softmax_split(const float* x, float*
   f32x4v v[NE4];
 #pragma unroll
   for (int k = 0; k < NE4; ++k) {
-    const int c = 4 * t + 1024 * k;  // cols % 4 == 0: a vector is wholly inside or outside the row
-    v[k] = c < rem ? __builtin_nontemporal_load(reinterpret_cast<const f32x4v*>(xr + c))
-                   : f32x4v{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    const int c = 4 * t + 1024 * k;  // ALIGNED: a vector is wholly inside or outside the row
+    v[k] = f32x4v{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    if constexpr (ALIGNED) {
+      if (c < rem) v[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4v*>(xr + c));
+    } else if (c + 4 <= rem) {
+      v[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(xr + c));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < rem) v[k][e] = ld(xr + c + e);
+    }
   }
   float m = -INFINITY;
 #pragma unroll
@@ -329,7 +343,16 @@ __global__ __launch_bounds__(kBlock) void k_softmax_split(const float* x, float*
 #pragma unroll
   for (int k = 0; k < NE4; ++k) {
     const int c = 4 * t + 1024 * k;
-    if (c < rem) __builtin_nontemporal_store(v[k] * f, reinterpret_cast<f32x4v*>(yr + c));
+    const f32x4v r = v[k] * f;
+    if constexpr (ALIGNED) {
+      if (c < rem) __builtin_nontemporal_store(r, reinterpret_cast<f32x4v*>(yr + c));
+    } else if (c + 4 <= rem) {
+      __builtin_nontemporal_store(r, reinterpret_cast<f32x4u*>(yr + c));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < rem) st(yr + c + e, r[e]);
+    }
   }
 }
 
@@ -352,31 +375,44 @@ extern "C" int tt_softmax_rows_f32(const float* x, float* y, int64_t rows, int64
   int rc = ensure_init();
   if (rc) return rc;
   hipStream_t s = stream_or_default(stream);
-  // Long 16-byte aligned rows: split over workgroups (k_softmax_split), with
-  // chunks of 4096 / 8192 / 16384 / 32768 columns for rows up to 16 Ki /
-  // 64 Ki / 256 Ki / 2 Mi columns (measured best on the MI355X for each).
+  // Long rows: split over workgroups (k_softmax_split), with chunks of 4096 /
+  // 8192 / 16384 / 32768 columns for rows up to 16 Ki / 64 Ki / 256 Ki / 2 Mi
+  // columns (measured best on the MI355X for each).  Rows that begin at any
+  // float take unaligned 16-byte words: 8192 x 10007 136 -> 122 us (one 16-wave
+  // workgroup a row, 4-byte loads, before; 115 us at 10008), 1000 x 65535 142 ->
+  // 87, 64 x 50257 16.1 -> 7.7, 200 x 262143 178 -> 82; only a handful of short
+  // rows is no faster (3 x 10007 5.25 / 5.37).  Not under capture (a
+  // replay would find the generation of its last one in the slots), nor
+  // without scratch: the kernels below take any length.
   const bool aligned = cols % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)y % 16) == 0;
-  if (aligned && cols > 8192 && cols <= int64_t(kSplitMaxChunks) * 32768) {
+  if (cols > 8192 && cols <= int64_t(kSplitMaxChunks) * 32768 && (aligned || cols > 16384 || rows >= 16) &&
+      !stream_capturing(s)) {
     const int ne4 = cols <= 16384 ? 4 : cols <= 65536 ? 8 : cols <= 262144 ? 16 : 32;
     const int64_t cw = 1024 * ne4, nchunk = (cols + cw - 1) / cw;
-    if (grid_fits(rows * nchunk, kBlock)) {  // else the grid-stride kernels below
-      unsigned long long* slots = nullptr;
-      uint64_t uses = 0;
-      const size_t bytes = (size_t)(rows * nchunk) * 2 * sizeof(unsigned long long);
-      WorkspaceLease ws;  // held until the kernel that reads the slots is queued
-      if ((rc = ws.get(s, kWsSoftmaxPartials, bytes, (void**)&slots, &uses))) return rc;
+    unsigned long long* slots = nullptr;
+    uint64_t uses = 0;
+    const size_t bytes = (size_t)(rows * nchunk) * 2 * sizeof(unsigned long long);
+    std::optional<WorkspaceLease> ws;  // held until the kernel that reads the slots is queued
+    if (grid_fits(rows * nchunk, kBlock) &&
+        ws.emplace().get(s, kWsSoftmaxPartials, bytes, (void**)&slots, &uses) == TT_OK) {
       const unsigned gen = (unsigned)(uses % 0xffffffffull) + 1;  // 1 .. 2^32 - 1
       if (gen == 1 &&  // a new buffer (or a wrapped count): no word may hold a live generation
           (rc = tt_elementwise(TT_EW_FILL, TT_F32, slots, nullptr, nullptr, (int64_t)(bytes / 4), 0.0, 0.0, 0, s)))
         return rc;
       const dim3 grid((unsigned)(rows * nchunk)), blk(kBlock);
       const int n = (int)nchunk;
+#define TT_SPLIT(NE)                                                                                             \
+  if (aligned)                                                                                                   \
+    hipLaunchKernelGGL((k_softmax_split<NE, true>), grid, blk, 0, s, x, y, cols, n, slots, gen);                 \
+  else                                                                                                           \
+    hipLaunchKernelGGL((k_softmax_split<NE, false>), grid, blk, 0, s, x, y, cols, n, slots, gen)
       switch (ne4) {
-        case 4: hipLaunchKernelGGL(k_softmax_split<4>, grid, blk, 0, s, x, y, cols, n, slots, gen); break;
-        case 8: hipLaunchKernelGGL(k_softmax_split<8>, grid, blk, 0, s, x, y, cols, n, slots, gen); break;
-        case 16: hipLaunchKernelGGL(k_softmax_split<16>, grid, blk, 0, s, x, y, cols, n, slots, gen); break;
-        default: hipLaunchKernelGGL(k_softmax_split<32>, grid, blk, 0, s, x, y, cols, n, slots, gen); break;
+        case 4: TT_SPLIT(4); break;
+        case 8: TT_SPLIT(8); break;
+        case 16: TT_SPLIT(16); break;
+        default: TT_SPLIT(32); break;
       }
+#undef TT_SPLIT
       TT_LAUNCHED("tt_softmax_rows_f32", s);
       return ok();
     }
