@@ -59,8 +59,31 @@ constexpr int FWDP_NW = 4;
 // kernel: few query tiles against many keys (B = 2, H = 16, 77 queries, 4099
 // keys: 32 tiles) then fill the chip.  A causal workgroup's last split takes
 // both diagonal tiles, so every wave has a key tile in every non-empty split.
-template <int D, bool CAUSAL, int NW, bool SPLIT>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
+//
+// KG = 2: two groups of NW waves share the queries, group g taking the key
+// tiles g, g + 2, ... through a ring of its own, and merge their O, maxima and
+// sums in LDS at the end.  For grids of fewer workgroups than the chip holds
+// (two NW-wave ones per CU), where the time is the longest query tile's chain
+// of key tiles: the same waves per CU walk half of it each.
+// The tile loader of wave `wave` of a group of NW waves.  (TileDma's own init
+// takes the workgroup's wave index; giving it a parameter instead changed the
+// backward kernels' register allocation and cost [16,16,1024] d = 64 1.5 %.)
+template <int D, int ROWS, int NW>
+struct GroupDma : TileDma<D, ROWS, NW> {
+  using Base = TileDma<D, ROWS, NW>;
+  __device__ __forceinline__ void init_group(int wave) {
+    this->w = wave;
+    const int p = wave * 64 + (threadIdx.x & 63);
+#pragma unroll
+    for (int ph = 0; ph < Base::kPh; ++ph) {
+      const int row = p / Base::kCPR + ph * Base::kStep, ch = (p % Base::kCPR) ^ SwzTile<D>::sw(row);
+      this->voff[ph] = 2u * (uint32_t)(row * D + 8 * ch);
+    }
+  }
+};
+
+template <int D, bool CAUSAL, int NW, int KG, bool SPLIT>
+__global__ __launch_bounds__(64 * NW * KG, 8 / (NW * KG)) void attn_fwd_bf16_pipe_kernel(
     const u16* __restrict__ Q, const u16* __restrict__ K, const u16* __restrict__ V,
     u16* __restrict__ O, float* __restrict__ LSE, int Lq, int Lk, int BH, int nqt, int order,
     float sl2, int nsplit, float* __restrict__ part) {
@@ -68,12 +91,15 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
   constexpr int BM = 32 * NW, BN = 64;
   constexpr int NC = D / 16, ND = D / 32;
   constexpr int TE = Tile::kElems(BN);
-  using Dma = TileDma<D, BN, NW>;
-  __shared__ __align__(16) u16 sK[2 * TE];
-  __shared__ __align__(16) u16 sV[2 * TE];
+  using Dma = GroupDma<D, BN, NW>;
+  __shared__ __align__(16) u16 smem_k[KG * 2 * TE];  // the groups' K rings
+  __shared__ __align__(16) u16 smem_v[KG * 2 * TE];  // and V rings
 
   // the wave index is wave-uniform: loop bounds derived from it stay scalar
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w = KG == 1 ? wv : wv % NW, grp = KG == 1 ? 0 : wv / NW;
+  u16* const sK = smem_k + grp * (2 * TE);
+  u16* const sV = smem_v + grp * (2 * TE);
   const int l = threadIdx.x & 63, g = l >> 5, r32 = l & 31;
   int qt, bh;
   const int split = SPLIT ? blockIdx.x / (nqt * BH) : 0;
@@ -111,11 +137,17 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
   }
 
   const int kend = CAUSAL ? min(Lk, q0 + BM - k_first) : Lk;  // >= 1: Lk >= 1, and q0 < Lq = Lk when causal
-  const int ntiles = (kend + BN - 1) / BN;
+  const int ntiles_wg = (kend + BN - 1) / BN;
+  // This group's tiles: n of its ring is tile KG n + grp.  nsteps: the most of
+  // any group (every wave takes part in that many barriers).
+  const int ntiles = (ntiles_wg - grp + KG - 1) / KG, nsteps = (ntiles_wg + KG - 1) / KG;
+  auto krow = [&](int n) { return BN * (KG * n + grp); };
   // Last tile this wave computes: its diagonal tile (causal) or the last
-  // tile.  Every earlier tile lies inside Lk and before every query of the
-  // wave, so only the last one can need a mask.
-  const int last = CAUSAL ? min((wq0 - k_first) / BN, ntiles - 1) : ntiles - 1;
+  // tile, or the group's last one before it (-1: none).  Every earlier tile
+  // lies inside Lk and before every query of the wave, so only the last one
+  // can need a mask.
+  const int last_wg = CAUSAL ? min((wq0 - k_first) / BN, ntiles_wg - 1) : ntiles_wg - 1;
+  const int last = KG == 1 ? last_wg : (last_wg >= grp ? (last_wg - grp) / KG : -1);
   const bool mask_last = CAUSAL || (Lk % BN) != 0;
 
   // Per-lane LDS element offsets.  K operand of chunk c: key row r32 (+32
@@ -231,12 +263,15 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
   };
 
   Dma dma;
-  dma.init();
+  if constexpr (KG == 1)
+    dma.init();
+  else
+    dma.init_group(w);
   auto issue_k = [&](int n) {
-    if (n < ntiles) dma.issue(K + kbase, BN * n, Lk, sK + (n & 1) * TE);
+    if (n < ntiles) dma.issue(K + kbase, krow(n), Lk, sK + (n & 1) * TE);
   };
   auto issue_v = [&](int n) {
-    if (n < ntiles) dma.issue(V + kbase, BN * n, Lk, sV + (n & 1) * TE);
+    if (n < ntiles) dma.issue(V + kbase, krow(n), Lk, sV + (n & 1) * TE);
   };
   auto step = [&](int n) {
     wait_vmem_le<0>();
@@ -260,9 +295,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
     const int kbuf = PAR < 0 ? ((j + 1) & 1) : 1 - PAR, vbuf = PAR < 0 ? (j & 1) : PAR;
     auto load_kv = [&](int c) {
       if (c < kLoads)
-        dma.issue_one(K + kbase, BN * (j + 2), sK + PAR * TE, c);
+        dma.issue_one(K + kbase, krow(j + 2), sK + PAR * TE, c);
       else if (c < 2 * kLoads)
-        dma.issue_one(V + kbase, BN * (j + 1), sV + (1 - PAR) * TE, c - kLoads);
+        dma.issue_one(V + kbase, krow(j + 1), sV + (1 - PAR) * TE, c - kLoads);
     };
     if constexpr (SPREAD) {
       wait_vmem_le<0>();
@@ -283,7 +318,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
     exp_cvt(cur);
     pv(sV + vbuf * TE);
     add_sum();
-    if constexpr (MASK) mask_tile(nx, BN * (j + 1));
+    if constexpr (MASK) mask_tile(nx, krow(j + 1));
     rescale = row_max(nx, false);
   };
 
@@ -296,8 +331,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
   else
     wait_vmem_le<Dma::kLoads>();
   __syncthreads();
+  if (KG == 1 || last >= 0) {
   qk(sK, sa, no_load);
-  if (last == 0 && mask_last) mask_tile(sa, 0);
+  if (last == 0 && mask_last) mask_tile(sa, krow(0));
   row_max(sa, true);
 
   // Unmasked iterations 0 .. last - 2 in pairs (the score tiles swap roles),
@@ -339,14 +375,54 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
   exp_cvt(sa);
   pv(sV + (last & 1) * TE);
   add_sum();
+  } else {
+    m = -INFINITY;  // no tile of this group: nothing to add
+  }
   // Later tiles belong to other waves of the workgroup: take part in their
   // barriers and loads.
-  for (int n = last + 1; n < ntiles; ++n) step(n);
+  for (int n = last + 1; n < nsteps; ++n) step(n);
   wait_vmem_le<0>();  // nothing may be in flight into LDS when the workgroup exits
 
-  const float ls = sum_xor32(lsum);
+  float ls = sum_xor32(lsum);
+  if constexpr (KG == 2) {
+    // group 1 hands its O, max and sum over through its own rings' space: the
+    // first half of O's registers through the K ring's, the rest the V ring's
+    static_assert(2 * TE * sizeof(u16) >= NW * 64 * ND * 8 * sizeof(float), "a ring holds half of the group's O");
+    __shared__ float s_ml[NW * 64 * 2];
+    auto ox = [&](int i) -> f32x4& {  // four registers i of 4 ND, of this wave and lane
+      u16* half = (i < 2 * ND ? smem_k : smem_v) + 2 * TE;
+      return reinterpret_cast<f32x4*>(half)[(w * 2 * ND + i % (2 * ND)) * 64 + l];
+    };
+    float* ml = s_ml + 2 * (64 * w + l);
+    __syncthreads();  // every wave is done with the rings
+    if (grp == 1) {
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4)
+          ox(4 * dt + r / 4) = f32x4{o[dt][r], o[dt][r + 1], o[dt][r + 2], o[dt][r + 3]};
+      ml[0] = m;
+      ml[1] = ls;
+    }
+    __syncthreads();
+    if (grp == 0) {
+      const float m1 = ml[0], mm = vmax(m, m1), mb = mm == -INFINITY ? 0.f : mm;
+      const float a0 = fast_exp2(m - mb), a1 = fast_exp2(m1 - mb);
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+          const f32x4 x = ox(4 * dt + r / 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[dt][r + e] = o[dt][r + e] * a0 + x[e] * a1;
+        }
+      ls = ls * a0 + ml[1] * a1;
+      m = mm;
+    }
+  }
+  const bool out = KG == 1 || grp == 0;  // this group holds the result
   if constexpr (SPLIT) {
-    if (qrow < Lq) {
+    if (out && qrow < Lq) {
       const int64_t row = ((int64_t)split * BH + bh) * Lq + qrow;
       float* orow = part + row * D;
 #pragma unroll
@@ -364,17 +440,17 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_bf16_pipe_kernel(
     return;
   }
   const float inv = ls > 0.f ? 1.f / ls : 0.f;
-  if (qrow < Lq && g == 0 && LSE) LSE[(int64_t)bh * Lq + qrow] = (m + __log2f(ls)) * kLn2;
+  if (out && qrow < Lq && g == 0 && LSE) LSE[(int64_t)bh * Lq + qrow] = (m + __log2f(ls)) * kLn2;
   if constexpr (D >= 128) {
     // O through LDS (the K ring is free once every wave has passed its last
     // wait; 128 rows of D bf16 fit the two K buffers): c5 -0.5 %; at d = 64
     // the two extra barriers cost more than the 8-byte stores (+1.7 % at c3)
     static_assert(2 * TE >= BM * D, "the K ring holds the workgroup's O rows");
     __syncthreads();
-    stage_rows_bf16<D, ND>(sK, 32 * w + r32, g, o, inv);
+    if (out) stage_rows_bf16<D, ND>(smem_k, 32 * w + r32, g, o, inv);
     __syncthreads();
-    store_staged_rows<D>(sK, BM, O + qbase, q0, Lq, 64 * NW);
-  } else if (qrow < Lq) {
+    store_staged_rows<D>(smem_k, BM, O + qbase, q0, Lq, 64 * NW * KG);
+  } else if (out && qrow < Lq) {
     u16* orow = O + qbase + (int64_t)qrow * D;
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt)
@@ -668,15 +744,30 @@ static int fwd_bf16(const u16* q, const u16* k, const u16* v, u16* o, float* lse
   if (nsplit > 1 && !stream_capturing(st) &&
       lease.emplace().get(st, kWsForwardSplits, (size_t)(nsplit * BH * Lq) * (D + 2) * sizeof(float),
                           (void**)&part) == TT_OK) {
-    hipLaunchKernelGGL((attn_fwd_bf16_pipe_kernel<D, CAUSAL, NW, true>), dim3((unsigned)(tiles * nsplit)),
-                       dim3(64 * NW), 0, st, q, k, v, o, lse, (int)Lq, (int)Lk, (int)BH, (int)nqt, order, sl2, nsplit,
-                       part);
+    // two key groups per workgroup at d = 128 (below: [1,32] 256 x 4096 31.8 ->
+    // 29.5 us), one at d <= 64 (two: [2,16] 77 x 4099 14.9 -> 15.5, [2,8] 333 x 2000
+    // d = 32 14.0 -> 17.3)
+    constexpr int KG = D >= 128 ? 2 : 1;
+    hipLaunchKernelGGL((attn_fwd_bf16_pipe_kernel<D, CAUSAL, NW, KG, true>), dim3((unsigned)(tiles * nsplit)),
+                       dim3(64 * NW * KG), 0, st, q, k, v, o, lse, (int)Lq, (int)Lk, (int)BH, (int)nqt, order, sl2,
+                       nsplit, part);
     TT_LAUNCHED("attention forward split launch", st);
     return launch_fwd_combine<u16, D>(part, o, lse, BH * Lq, nsplit, st);
   }
   // without scratch (refused, or under capture) the keys are not split
-  hipLaunchKernelGGL((attn_fwd_bf16_pipe_kernel<D, CAUSAL, NW, false>), dim3((unsigned)tiles), dim3(64 * NW), 0, st, q,
-                     k, v, o, lse, (int)Lq, (int)Lk, (int)BH, (int)nqt, order, sl2, 1, nullptr);
+  // Two key groups per workgroup where fewer query tiles than workgroup slots
+  // (512) walk many key tiles.  Measured (one / two groups, us): causal [1,32,1531]
+  // d = 128 (384 tiles) 37.9 / 32.3, [1,8,4096] d = 128 (256) 64.6 / 51.9,
+  // [1,12,1000] d = 64 (96) 15.5 / 14.0; full [1,16,2048] d = 64 (256) 25.9 / 24.1.  Not
+  // with few key tiles ([3,32,300] d = 64 8.1 / 11.4, [4,16,512] 10.1 / 10.5), nor
+  // full with more tiles than CUs ([1,40,1400] d = 128 (440) 47.9 / 54.6), nor from
+  // 512 tiles on ([2,32,1500] d = 128 49.6 / 56.4).
+  if (Lk >= 768 && tiles < (CAUSAL ? 512 : 257))
+    hipLaunchKernelGGL((attn_fwd_bf16_pipe_kernel<D, CAUSAL, NW, 2, false>), dim3((unsigned)tiles), dim3(64 * NW * 2),
+                       0, st, q, k, v, o, lse, (int)Lq, (int)Lk, (int)BH, (int)nqt, order, sl2, 1, nullptr);
+  else
+    hipLaunchKernelGGL((attn_fwd_bf16_pipe_kernel<D, CAUSAL, NW, 1, false>), dim3((unsigned)tiles), dim3(64 * NW), 0,
+                       st, q, k, v, o, lse, (int)Lq, (int)Lk, (int)BH, (int)nqt, order, sl2, 1, nullptr);
   TT_LAUNCHED("attention forward launch", st);
   return ok();
 }

@@ -1,5 +1,5 @@
-"""GPU tests of the bf16 forward with its keys split over workgroups (few
-query tiles, many keys; csrc/attn_fwd.hip), where splits, tiles and diagonals
+"""GPU tests of the bf16 forward with its keys split over workgroups, or over
+two groups of waves of one workgroup (few query tiles, many keys; csrc/attn_fwd.hip), where splits, tiles and diagonals
 meet, against the float64 oracle at the bf16 bar (2e-2, normwise).  LSE: the
 row sum adds the bf16-rounded weights that the P V product applies, each
 within 2^-9 of its value, so it is within log(1 + 2^-9) < 2^-9 of the exact
@@ -41,7 +41,10 @@ def _inputs(B, H, Lq, Lk, d, seed):
 # 16 key tiles is the shortest split (up to 32 query tiles), 32 beyond; unsplit just below
 CASES = [(1, 1, 1, 961, 64, False), (1, 1, 5, 960, 32, False), (1, 3, 129, 1500, 128, False), (1, 2, 300, 2049, 64, False),
          (1, 1, 1025, 1025, 64, True), (1, 2, 1000, 1000, 128, True), (1, 1, 4097, 4097, 32, True),
-         (1, 8, 1985, 1985, 32, True), (1, 9, 1000, 2047, 32, False)]
+         (1, 8, 1985, 1985, 32, True), (1, 9, 1000, 2047, 32, False),
+         # two key groups without a split: an odd and an even count of key tiles, ragged ends, diagonals
+         (1, 9, 769, 769, 128, True), (1, 9, 833, 833, 64, True), (2, 17, 896, 896, 32, True),
+         (2, 20, 300, 1023, 128, False), (1, 33, 130, 768, 64, False)]
 
 
 @pytest.mark.parametrize("case", CASES, ids=str)
