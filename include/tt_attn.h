@@ -294,7 +294,7 @@ int tt_cross_entropy_backward_f32(const float* p, const int* labels, float* grad
  * 26-77) and ConvForward / ConvBackward (:197, :247-248).  fp32: fp32
  * products and sums on the fp32 MFMA; bf16: bf16 A, B, C with fp32 sums.
  * Products too small to fill the chip split k over workgroups through a
- * 16 MiB per-stream library workspace (allocated on first use); if that
+ * 12 MiB per-stream library workspace (allocated on first use); if that
  * allocation fails, or the stream is being captured into a graph, they run
  * unsplit and allocate nothing. */
 int tt_gemm_f32(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha,

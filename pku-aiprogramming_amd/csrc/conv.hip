@@ -207,12 +207,11 @@ int conv_entry(const char* fn, int dtype, const void* src, void* dst, int64_t N,
 // launches dominated (a product per image at 5-76 us each), at large ones the
 // dW product, one or a few tiles walking every pixel.  Forward / backward
 // through myLayer, us, before -> now: 64 x 8 x 14 x 14, 16 kernels 5 x 5 fp32
-// 1557 / 2212 -> 28 / 55; 64 x 64 x 56 x 56, 64 kernels 3 x 3 fp32 4128 /
-// 22291 -> 293 / 693 (51 / 43 TF), bf16 1683 / 7425 -> 179 / 495; 8 x 512 x
-// 28 x 28, 512 kernels 3 x 3 fp32 3468 / 1648 -> 691 / 1490; 1 x 3 x 224 x 224,
-// 768 kernels 16 x 16 stride 16 fp32 85 / 123 -> 29 / 46.  What bounds the
-// large ones now is the gather (index arithmetic and 4- to 16-byte loads).
-
+// 1557 / 2212 -> 22 / 47; 64 x 64 x 56 x 56, 64 kernels 3 x 3 fp32 4128 /
+// 22291 -> 241 / 566 (61 / 52 TF), bf16 1683 / 7425 -> 109 / 360; 8 x 512 x
+// 28 x 28, 512 kernels 3 x 3 fp32 3468 / 1648 -> 566 / 1248; 1 x 3 x 224 x 224,
+// 768 kernels 16 x 16 stride 16 fp32 85 / 123 -> 27 / 44.  What bounds them now
+// is the gather's index arithmetic, about ten VALU instructions an element.
 // n / d for 0 <= n < 2^31 by a multiplication (Granlund and Montgomery's
 // round-up method).
 struct FastDiv {
@@ -235,83 +234,152 @@ struct ConvDivs {
   FastDiv kk, kw, P, ow;  // kh * kw, kw, oh * ow, ow
 };
 
-// Chunks of EPC consecutive positions of one row of a [planes][h][w] image.
-// X(kk, q): kKC = false puts q on the tile rows (forward), true on k (dW).
-template <typename T, bool KC>
-struct ColumnSource {
-  static constexpr bool kKC = KC, kPhased = false;
-  const T* im;
-  ConvGeom g;
-  ConvDivs dv;
-  int K, Q;
-  __device__ __forceinline__ split_u32x4 chunk(int row, int k) const {
-    constexpr int EPC = SplitT<T>::EPC;
-    const int kk = KC ? row : k, q = KC ? k : row;
+// Gathers.  Every operand is im[base(v) + off(t)] for a vector position v (a
+// pixel, whose EPC neighbours make one chunk) and a tap t (a kernel position
+// or channel), zero unless the tap's step from the position stays inside the
+// image: 0 <= y(v) + dy(t) < ylim and 0 <= x(v) + dx(t) < xlim.  The chunk's
+// elements are loaded one by one without branches (element 0 where there is
+// none, replaced by zero in pack): with branches around the loads (one 16-byte
+// load inside an image row, predicated ones across its edge) each chunk waited
+// for its own loads, 5-10 us a k-step.
+struct Tap {
+  int off, dy, dx;
+};
+template <int N>
+struct Positions {
+  int base[N], y[N], x[N];
+};
+constexpr int kOutside = -(1 << 30);  // a y or dy that no step brings inside
+
+// a b + c for offsets of elements that may not exist
+__device__ __forceinline__ int wrap_mad(int a, int b, int c) {
+  return (int)((unsigned)a * (unsigned)b + (unsigned)c);
+}
+
+// Src: Positions<EPC> positions(v), Tap tap(t), data(), ylim(), xlim().
+// kKC = true: v = k and t = row; false: v = row and t = k.
+template <typename T, bool KC, class Src>
+struct Gather {
+  static constexpr bool kKC = KC;
+  static constexpr int EPC = SplitT<T>::EPC;
+  struct Raw {
+    T v[EPC];
+    bool in[EPC];
+  };
+  using At = std::conditional_t<KC, Tap, Positions<EPC>>;
+  __device__ __forceinline__ const Src& self() const { return static_cast<const Src&>(*this); }
+  __device__ __forceinline__ At at(int row) const {
+    if constexpr (KC)
+      return self().tap(row);
+    else
+      return self().positions(row);
+  }
+  __device__ __forceinline__ Raw chunk(const At& at, int k) const {
+    if constexpr (KC)
+      return load(self().positions(k), at);
+    else
+      return load(at, self().tap(k));
+  }
+  __device__ __forceinline__ Raw load(const Positions<EPC>& p, const Tap& t) const {
+    Raw r;
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) {
+      r.in[e] = ((unsigned)(p.y[e] + t.dy) < (unsigned)self().ylim()) &
+                ((unsigned)(p.x[e] + t.dx) < (unsigned)self().xlim());
+      r.v[e] = self().data()[r.in[e] ? p.base[e] + t.off : 0];
+    }
+    return r;
+  }
+  __device__ __forceinline__ split_u32x4 pack(const Raw& r) const {
     T v[EPC];
 #pragma unroll
-    for (int e = 0; e < EPC; ++e) v[e] = T(0);
-    if (kk < K && q < Q) {
-      int r, kx, p, ox;
-      const int c = dv.kk.divmod(kk, r), ky = dv.kw.divmod(r, kx);
-      int n = dv.P.divmod(q, p), oy = dv.ow.divmod(p, ox);
-      int y = oy * g.sh - g.ph + ky, x = ox * g.sw - g.pw + kx;
-      const T* pl = im + ((int64_t)n * g.C + c) * g.H * g.W;
-      if (g.sw == 1 && ox + EPC <= g.ow && x >= 0 && x + EPC <= g.W) {  // one image row, inside
-        if (y >= 0 && y < g.H) return *reinterpret_cast<const split_u32x4_any*>(pl + (int64_t)y * g.W + x);
-      } else {
-        const int left = Q - q;
-#pragma unroll
-        for (int e = 0; e < EPC; ++e) {
-          if (e < left && y >= 0 && y < g.H && x >= 0 && x < g.W) v[e] = pl[(int64_t)y * g.W + x];
-          x += g.sw;
-          if (++ox == g.ow) {  // next output row, or the next image
-            ox = 0;
-            x = kx - g.pw;
-            y += g.sh;
-            if (++oy == g.oh) {
-              oy = 0;
-              y = ky - g.ph;
-              pl += (int64_t)g.C * g.H * g.W;
-            }
-          }
-        }
-      }
-    }
+    for (int e = 0; e < EPC; ++e) v[e] = r.in[e] ? r.v[e] : T(0);
     return __builtin_bit_cast(split_u32x4, v);
   }
 };
 
-// gO[co, q] of the [N][Cout][P] output gradient: kKC = true rows co, k = q;
-// false rows q, k = co.
+// X(kk, q): v = output pixel q (its window's first row and column), t = kk.
 template <typename T, bool KC>
-struct GradRowSource {
-  static constexpr bool kKC = KC, kPhased = false;
+struct ColumnSource : Gather<T, KC, ColumnSource<T, KC>> {
+  static constexpr bool kPhased = false;
+  const T* im;
+  ConvGeom g;
+  ConvDivs dv;
+  int K, Q;
+  ColumnSource(const T* im_, const ConvGeom& g_, const ConvDivs& dv_, int K_, int Q_)
+      : im(im_), g(g_), dv(dv_), K(K_), Q(Q_) {}
+  __device__ __forceinline__ const T* data() const { return im; }
+  __device__ __forceinline__ int ylim() const { return g.H; }
+  __device__ __forceinline__ int xlim() const { return g.W; }
+  __device__ __forceinline__ Positions<SplitT<T>::EPC> positions(int q) const {
+    Positions<SplitT<T>::EPC> r;
+#pragma unroll
+    for (int e = 0; e < SplitT<T>::EPC; ++e) {
+      int p, ox;
+      const int n = dv.P.divmod(q + e, p), oy = dv.ow.divmod(p, ox);
+      r.y[e] = q + e < Q ? oy * g.sh - g.ph : kOutside;
+      r.x[e] = ox * g.sw - g.pw;
+      r.base[e] = wrap_mad(wrap_mad(n, g.C * g.H, r.y[e]), g.W, r.x[e]);
+    }
+    return r;
+  }
+  __device__ __forceinline__ Tap tap(int kk) const {
+    int r, kx;
+    const int c = dv.kk.divmod(kk, r), ky = dv.kw.divmod(r, kx);
+    return Tap{wrap_mad(wrap_mad(c, g.H, ky), g.W, kx), kk < K ? ky : kOutside, kx};
+  }
+};
+
+// gO[co, q] of the [N][Cout][P] output gradient: v = q, t = co.
+template <typename T, bool KC>
+struct GradRowSource : Gather<T, KC, GradRowSource<T, KC>> {
+  static constexpr bool kPhased = false;
   const T* go;
   FastDiv P;
   int cout, Q;
-  __device__ __forceinline__ split_u32x4 chunk(int row, int k) const {
-    constexpr int EPC = SplitT<T>::EPC;
-    const int co = KC ? row : k, q0 = KC ? k : row;
-    T v[EPC];
+  GradRowSource(const T* go_, const FastDiv& P_, int cout_, int Q_) : go(go_), P(P_), cout(cout_), Q(Q_) {}
+  __device__ __forceinline__ const T* data() const { return go; }
+  __device__ __forceinline__ int ylim() const { return 1; }
+  __device__ __forceinline__ int xlim() const { return 1; }
+  __device__ __forceinline__ Positions<SplitT<T>::EPC> positions(int q) const {
+    Positions<SplitT<T>::EPC> r;
 #pragma unroll
-    for (int e = 0; e < EPC; ++e) v[e] = T(0);
-    if (co < cout && q0 < Q) {
+    for (int e = 0; e < SplitT<T>::EPC; ++e) {
       int p;
-      const int n = P.divmod(q0, p), np = (int)P.d;
-      const T* q = go + ((int64_t)n * cout + co) * np;
-      if (p + EPC <= np) return *reinterpret_cast<const split_u32x4_any*>(q + p);
-      const int left = Q - q0;
-#pragma unroll
-      for (int e = 0; e < EPC; ++e) {
-        if (e < left) v[e] = q[p];
-        if (++p == np) {  // the next image
-          p = 0;
-          q += (int64_t)cout * np;
-        }
-      }
+      const int n = P.divmod(q + e, p);
+      r.base[e] = wrap_mad(n, cout * (int)P.d, p);
+      r.y[e] = q + e < Q ? 0 : kOutside;
+      r.x[e] = 0;
     }
-    return __builtin_bit_cast(split_u32x4, v);
+    return r;
   }
+  __device__ __forceinline__ Tap tap(int co) const { return Tap{wrap_mad(co, (int)P.d, 0), co < cout ? 0 : kOutside, 0}; }
+};
+
+// The same for planes of whole chunks (P % EPC = 0): rows co, k = q, one
+// 16-byte load a chunk.
+template <typename T>
+struct GradPlaneSource {
+  static constexpr bool kKC = true, kPhased = false;
+  const T* go;
+  FastDiv P;
+  int cout, Q;
+  struct Raw {
+    split_u32x4 v;
+    bool in;
+  };
+  struct At {
+    int off;
+    bool in;
+  };
+  __device__ __forceinline__ At at(int co) const { return At{wrap_mad(co, (int)P.d, 0), co < cout}; }
+  __device__ __forceinline__ Raw chunk(const At& at, int q) const {
+    int p;
+    const int n = P.divmod(q, p);
+    const bool in = at.in & (q < Q);
+    return Raw{*reinterpret_cast<const split_u32x4_any*>(go + (in ? wrap_mad(n, cout * (int)P.d, p) + at.off : 0)), in};
+  }
+  __device__ __forceinline__ split_u32x4 pack(const Raw& r) const { return r.in ? r.v : split_u32x4{0, 0, 0, 0}; }
 };
 
 // dX by phases.  With strides sh x sw an image row y is only reached by the
@@ -332,94 +400,78 @@ struct ConvPhase {
   }
 };
 
-// W[co, c, ky, kx]: rows c, k = (co, i, j) over the phase's taps.
+// W[co, c, ky, kx]: v = k = (co, i, j) over the phase's taps, t = row c.
 template <typename T>
-struct WeightSource {
-  static constexpr bool kKC = true;
+struct WeightSource : Gather<T, true, WeightSource<T>> {
   const T* w;
   ConvGeom g;
   int cout, z0, phases_x;
   FastDiv taps, nkx;  // nky * nkx, nkx (of the phase; at least 1)
   int K;
+  WeightSource(const T* w_, const ConvGeom& g_, int cout_, int z0_, int phases_x_)
+      : w(w_), g(g_), cout(cout_), z0(z0_), phases_x(phases_x_) {}
   __device__ __forceinline__ void enter(int z) {
     const ConvPhase f(g, z0 + z, phases_x);
     taps = FastDiv(max(1, f.nky * f.nkx)), nkx = FastDiv(max(1, f.nkx));
     K = cout * f.nky * f.nkx;
     w += (int64_t)f.ky0 * g.kw + f.kx0;
   }
-  __device__ __forceinline__ split_u32x4 chunk(int row, int k) const {
-    constexpr int EPC = SplitT<T>::EPC;
-    T v[EPC];
-    int r, j;
-    const int co = taps.divmod(k, r), kk = g.kh * g.kw;
-    int i = nkx.divmod(r, j);
-    const T* p = w + ((int64_t)co * g.C + row) * kk;
+  __device__ __forceinline__ const T* data() const { return w; }
+  __device__ __forceinline__ int ylim() const { return 1; }
+  __device__ __forceinline__ int xlim() const { return 1; }
+  __device__ __forceinline__ Positions<SplitT<T>::EPC> positions(int k) const {
+    Positions<SplitT<T>::EPC> r;
 #pragma unroll
-    for (int e = 0; e < EPC; ++e) {
-      v[e] = (row < g.C && k + e < K) ? p[(int64_t)i * g.sh * g.kw + (int64_t)j * g.sw] : T(0);
-      if (++j == (int)nkx.d) {  // next tap row, or the next output channel
-        j = 0;
-        if (++i * (int)nkx.d == (int)taps.d) {
-          i = 0;
-          p += (int64_t)g.C * kk;
-        }
-      }
+    for (int e = 0; e < SplitT<T>::EPC; ++e) {
+      int t, j;
+      const int co = taps.divmod(k + e, t), i = nkx.divmod(t, j);
+      r.base[e] = wrap_mad(wrap_mad(co, g.C * g.kh, i * g.sh), g.kw, j * g.sw);
+      r.y[e] = k + e < K ? 0 : kOutside;
+      r.x[e] = 0;
     }
-    return __builtin_bit_cast(split_u32x4, v);
+    return r;
   }
+  __device__ __forceinline__ Tap tap(int c) const { return Tap{wrap_mad(c, g.kh * g.kw, 0), c < g.C ? 0 : kOutside, 0}; }
 };
 
-// gO(co, i, j, p): rows p = (n, pixel of the phase), k = (co, i, j).
+// gO(co, i, j, p): v = row p = (n, pixel of the phase), t = k = (co, i, j).
 template <typename T>
-struct GradImageSource {
-  static constexpr bool kKC = false, kPhased = true;
+struct GradImageSource : Gather<T, false, GradImageSource<T>> {
+  static constexpr bool kPhased = true;
   const T* go;
   ConvGeom g;
   int cout, images, z0, phases_x;
   FastDiv taps, nkx, pix, nx;  // nky * nkx, nkx, ny * nx, nx
-  int by, bx, ny, K, Q;
+  int by, bx, K, Q;
+  GradImageSource(const T* go_, const ConvGeom& g_, int cout_, int images_, int z0_, int phases_x_)
+      : go(go_), g(g_), cout(cout_), images(images_), z0(z0_), phases_x(phases_x_) {}
   __device__ __forceinline__ void enter(int z) {
     const ConvPhase f(g, z0 + z, phases_x);
     taps = FastDiv(max(1, f.nky * f.nkx)), nkx = FastDiv(max(1, f.nkx));
     pix = FastDiv(f.ny * f.nx), nx = FastDiv(f.nx);
-    by = f.by, bx = f.bx, ny = f.ny;
+    by = f.by, bx = f.bx;
     K = cout * f.nky * f.nkx;
     Q = images * f.ny * f.nx;
   }
-  __device__ __forceinline__ split_u32x4 chunk(int row, int k) const {
-    constexpr int EPC = SplitT<T>::EPC;
-    T v[EPC];
+  __device__ __forceinline__ const T* data() const { return go; }
+  __device__ __forceinline__ int ylim() const { return g.oh; }
+  __device__ __forceinline__ int xlim() const { return g.ow; }
+  __device__ __forceinline__ Positions<SplitT<T>::EPC> positions(int row) const {
+    Positions<SplitT<T>::EPC> r;
 #pragma unroll
-    for (int e = 0; e < EPC; ++e) v[e] = T(0);
-    if (k < K && row < Q) {
-      int r, j, p, x;
-      const int co = taps.divmod(k, r), i = nkx.divmod(r, j), n = pix.divmod(row, p);
-      int y = nx.divmod(p, x);
-      const int64_t P = (int64_t)g.oh * g.ow;
-      const T* pl = go + ((int64_t)n * cout + co) * P;
-      int oy = by + y - i, ox = bx + x - j;
-      if (x + EPC <= (int)nx.d && ox >= 0 && ox + EPC <= g.ow) {  // one gradient row, inside
-        if (oy >= 0 && oy < g.oh) return *reinterpret_cast<const split_u32x4_any*>(pl + (int64_t)oy * g.ow + ox);
-      } else {
-        const int left = Q - row;
-#pragma unroll
-        for (int e = 0; e < EPC; ++e) {
-          if (e < left && oy >= 0 && oy < g.oh && ox >= 0 && ox < g.ow) v[e] = pl[(int64_t)oy * g.ow + ox];
-          ++ox;
-          if (++x == (int)nx.d) {  // next pixel row, or the next image
-            x = 0;
-            ox = bx - j;
-            ++oy;
-            if (++y == ny) {
-              y = 0;
-              oy = by - i;
-              pl += cout * P;
-            }
-          }
-        }
-      }
+    for (int e = 0; e < SplitT<T>::EPC; ++e) {
+      int p, x;
+      const int n = pix.divmod(row + e, p), y = nx.divmod(p, x);
+      r.y[e] = row + e < Q ? by + y : kOutside;
+      r.x[e] = bx + x;
+      r.base[e] = wrap_mad(wrap_mad(n, cout * g.oh, by + y), g.ow, bx + x);
     }
-    return __builtin_bit_cast(split_u32x4, v);
+    return r;
+  }
+  __device__ __forceinline__ Tap tap(int k) const {
+    int r, j;
+    const int co = taps.divmod(k, r), i = nkx.divmod(r, j);
+    return Tap{wrap_mad(wrap_mad(co, g.oh, -i), g.ow, -j), k < K ? -i : kOutside, -j};
   }
 };
 
@@ -479,19 +531,23 @@ ConvDivs conv_divs(const ConvGeom& g) {
 
 constexpr int64_t kConvPhases = 32768;  // phases per launch (the grid's z extent is 16 bits)
 
-// Images per launch: the product's columns (n, pixel) stay below 2^30.
-int64_t conv_slab(int64_t N, int64_t pixels) { return std::min(N, std::max<int64_t>(1, (int64_t(1) << 30) / pixels)); }
+// Images per launch: the product's columns (n, pixel) and the offsets of the
+// images' elements stay below 2^30.
+int64_t conv_slab(int64_t N, int cout, const ConvGeom& g) {
+  const int64_t image = std::max((int64_t)g.C * g.H * g.W, (int64_t)cout * g.oh * g.ow);
+  return std::min(N, std::max<int64_t>(1, (int64_t(1) << 30) / image));
+}
 
 template <typename T>
 int conv_forward(const char* fn, const T* in, const T* w, T* out, int64_t N, int cout, const ConvGeom& g,
                  hipStream_t s) {
-  const int64_t P = (int64_t)g.oh * g.ow, K = (int64_t)g.C * g.kh * g.kw, slab = conv_slab(N, P);
+  const int64_t P = (int64_t)g.oh * g.ow, K = (int64_t)g.C * g.kh * g.kw, slab = conv_slab(N, cout, g);
   const ConvDivs dv = conv_divs(g);
   for (int64_t n = 0; n < N; n += slab) {
     const int64_t Q = std::min(slab, N - n) * P;
     const int rc = launch_split_gemm<T>(
         fn, cout, Q, K, MatrixSource<T, true>{w, K, cout, (int)K},
-        ColumnSource<T, false>{in + n * g.C * g.H * g.W, g, dv, (int)K, (int)Q},
+        ColumnSource<T, false>(in + n * g.C * g.H * g.W, g, dv, (int)K, (int)Q),
         PlaneEpilogue<T>{out + n * cout * P, dv.P, cout}, s);
     if (rc) return rc;
   }
@@ -503,13 +559,15 @@ int conv_backward(const char* fn, const T* in, const T* w, const T* go, T* gin, 
                   const ConvGeom& g, hipStream_t s) {
   const int64_t P = (int64_t)g.oh * g.ow, K = (int64_t)g.C * g.kh * g.kw, HW = (int64_t)g.H * g.W;
   const ConvDivs dv = conv_divs(g);
-  int64_t slab = conv_slab(N, P);
+  const int64_t slab = conv_slab(N, cout, g);
   for (int64_t n = 0; n < N; n += slab) {
     const int64_t Q = std::min(slab, N - n) * P;
-    const int rc = launch_split_gemm<T>(
-        fn, cout, K, Q, GradRowSource<T, true>{go + n * cout * P, dv.P, cout, (int)Q},
-        ColumnSource<T, true>{in + n * g.C * HW, g, dv, (int)K, (int)Q},
-        MatrixEpilogue<T>{gw, nullptr, 0, 1.f, n == 0 ? 0.f : 1.f, (int)K}, s);
+    const ColumnSource<T, true> col(in + n * g.C * HW, g, dv, (int)K, (int)Q);
+    const MatrixEpilogue<T> ep{gw, nullptr, 0, 1.f, n == 0 ? 0.f : 1.f, (int)K};
+    const T* gon = go + n * cout * P;
+    const int rc = P % SplitT<T>::EPC == 0
+                       ? launch_split_gemm<T>(fn, cout, K, Q, GradPlaneSource<T>{gon, dv.P, cout, (int)Q}, col, ep, s)
+                       : launch_split_gemm<T>(fn, cout, K, Q, GradRowSource<T, true>(gon, dv.P, cout, (int)Q), col, ep, s);
     if (rc) return rc;
   }
   if (g.sh >= g.kh && g.sw >= g.kw) {
@@ -524,13 +582,12 @@ int conv_backward(const char* fn, const T* in, const T* w, const T* go, T* gin, 
       const int64_t Q = std::min(slab, N - n) * P;
       const int rc = launch_split_gemm<T>(
           fn, K, Q, cout, MatrixSource<T, false>{w, K, (int)K, cout},
-          GradRowSource<T, false>{go + n * cout * P, dv.P, cout, (int)Q},
+          GradRowSource<T, false>(go + n * cout * P, dv.P, cout, (int)Q),
           WindowEpilogue<T>{gin + n * g.C * HW, g, dv.kk, dv.kw, dv.P, dv.ow}, s);
       if (rc) return rc;
     }
     return ok();
   }
-  slab = conv_slab(N, HW);
   const int phases_x = std::min(g.sw, g.W);
   const int64_t phases = (int64_t)std::min(g.sh, g.H) * phases_x;
   const int64_t pixels = (int64_t)((g.H + g.sh - 1) / g.sh) * ((g.W + g.sw - 1) / g.sw);  // of the largest phase
@@ -539,8 +596,8 @@ int conv_backward(const char* fn, const T* in, const T* w, const T* go, T* gin, 
     const int64_t images = std::min(slab, N - n);
     for (int64_t z0 = 0; z0 < phases; z0 += kConvPhases) {
       const int rc = launch_split_gemm<T>(
-          fn, g.C, images * pixels, cout * taps, WeightSource<T>{w, g, cout, (int)z0, phases_x},
-          GradImageSource<T>{go + n * cout * P, g, cout, (int)images, (int)z0, phases_x},
+          fn, g.C, images * pixels, cout * taps, WeightSource<T>(w, g, cout, (int)z0, phases_x),
+          GradImageSource<T>(go + n * cout * P, g, cout, (int)images, (int)z0, phases_x),
           PhaseEpilogue<T>{gin + n * g.C * HW, g, (int)images, (int)z0, phases_x}, s,
           (int)std::min<int64_t>(kConvPhases, phases - z0));
       if (rc) return rc;
@@ -552,10 +609,11 @@ int conv_backward(const char* fn, const T* in, const T* w, const T* go, T* gin, 
 // Clamps strides to the padded extent (a longer one also leaves one output)
 // and returns whether the products' 32-bit indices and grids cover the shape.
 bool conv_fits(ConvGeom& g, int cout) {
-  const int64_t lim = int64_t(1) << 30, kk = (int64_t)g.kh * g.kw;
+  const int64_t lim = int64_t(1) << 30, kk = (int64_t)g.kh * g.kw, P = (int64_t)g.oh * g.ow;
   const int64_t eh = (int64_t)g.H + 2 * (int64_t)g.ph, ew = (int64_t)g.W + 2 * (int64_t)g.pw;
-  if (eh >= lim / 2 || ew >= lim / 2 || (int64_t)g.oh * g.ow > lim || (int64_t)g.H * g.W > lim || kk > lim ||
-      g.C * kk > lim || cout * kk > lim)
+  // (each product below is of factors within 2^31, checked from the left)
+  if (eh >= lim / 2 || ew >= lim / 2 || P > lim || (int64_t)g.H * g.W > lim || kk > lim || g.C * ((int64_t)g.H * g.W) > lim ||
+      cout * P > lim || g.C * kk > lim || cout * (g.C * kk) > lim)
     return false;
   g.sh = std::min(g.sh, (int)eh + 1);
   g.sw = std::min(g.sw, (int)ew + 1);
@@ -584,7 +642,7 @@ extern "C" int tt_conv_forward(int dtype, const void* in, const void* weight, vo
   if (dtype != TT_F32 && dtype != TT_BF16) return fail(TT_ERR_ARG, std::string(fn) + ": dtype must be TT_F32 or TT_BF16");
   if (N == 0 || cout == 0) return ok();
   if (!in || !weight || !out) return fail(TT_ERR_ARG, std::string(fn) + ": null pointer");
-  if (!conv_fits(g, cout)) return fail(TT_ERR_UNSUPPORTED, std::string(fn) + ": image or kernel above 2^29 elements an axis or 2^30 in all");
+  if (!conv_fits(g, cout)) return fail(TT_ERR_UNSUPPORTED, std::string(fn) + ": one image, its output or the weights above 2^30 elements, or an axis above 2^29");
   if ((rc = ensure_init())) return rc;
   hipStream_t s = stream_or_default(stream);
   if (dtype == TT_F32) return conv_forward(fn, (const float*)in, (const float*)weight, (float*)out, N, cout, g, s);
@@ -602,7 +660,7 @@ extern "C" int tt_conv_backward(int dtype, const void* in, const void* weight, c
   if (dtype != TT_F32 && dtype != TT_BF16) return fail(TT_ERR_ARG, std::string(fn) + ": dtype must be TT_F32 or TT_BF16");
   if (!in || !weight || !grad_out || !grad_in || !grad_weight)
     return fail(TT_ERR_ARG, std::string(fn) + ": null pointer");
-  if (!conv_fits(g, cout)) return fail(TT_ERR_UNSUPPORTED, std::string(fn) + ": image or kernel above 2^29 elements an axis or 2^30 in all");
+  if (!conv_fits(g, cout)) return fail(TT_ERR_UNSUPPORTED, std::string(fn) + ": one image, its output or the weights above 2^30 elements, or an axis above 2^29");
   if ((rc = ensure_init())) return rc;
   hipStream_t s = stream_or_default(stream);
   if (dtype == TT_F32)

@@ -13,11 +13,15 @@
 // sums to `part` [nsplit][M][N] and k_split_reduce adds them in split order
 // (a fixed order: results do not depend on timing).
 //
-// A and B are read through sources that return one 16-byte chunk of T at a
+// A and B are read through sources that give one 16-byte chunk of T at a
 // time, zero outside the matrix:
-//   kKC  = true:  chunk(row, k) = elements (row, k .. k + EPC - 1)
-//   kKC  = false: chunk(row, k) = elements (row .. row + EPC - 1, k)
-// so a source can be a stored matrix of either orientation or a gather.
+//   kKC  = true:  chunk(at(row), k) = elements (row, k .. k + EPC - 1)
+//   kKC  = false: chunk(at(row), k) = elements (row .. row + EPC - 1, k)
+// so a source can be a stored matrix of either orientation or a gather.  A
+// thread's rows are the same in every k-step, so at(row), what a source works
+// out from the row alone, is computed once.  chunk returns the loads' raw
+// registers and pack makes the 16 bytes of them only where the tile is
+// written to LDS, after the step's MFMAs: nothing waits for a load in between.
 // A phased product (SB::kPhased) is several products in one launch: enter(z)
 // of the sources and the epilogue sets them up for product z, whose N and K
 // are then B.Q and B.K (M is common).  blockIdx.z = phase * nsplit + split.
@@ -63,7 +67,7 @@ typedef unsigned split_u32x4 __attribute__((ext_vector_type(4)));
 typedef split_u32x4 split_u32x4_any __attribute__((aligned(2)));
 
 // One operand tile: R rows x BK k-values.
-template <typename T, bool KC, int R>
+template <typename T, bool KC, int R, class Raw = split_u32x4>
 struct SplitTile {
   using S = SplitT<T>;
   static constexpr int BK = S::BK, EPC = S::EPC;
@@ -72,8 +76,10 @@ struct SplitTile {
   static constexpr int LD = KC ? BK + S::PAD_K : R + S::PAD_R;
   static constexpr int ELEMS = KC ? R * LD : BK * LD;
   static constexpr int PER = (KC ? BK : R) / EPC;  // chunks per stored row
+  static constexpr int ROWS = KC ? CH : 1;         // rows per thread
+  static_assert(KC || 256 % PER == 0, "one row chunk per thread");
 
-  split_u32x4 reg[CH];
+  Raw reg[CH];
 
   // element offset of chunk c of tile row r (KC)
   __device__ static __forceinline__ int at(int r, int c) {
@@ -81,18 +87,30 @@ struct SplitTile {
     return r * LD + c * EPC;
   }
   template <class Src>
-  __device__ __forceinline__ void load(const Src& src, int r0, int k0) {
+  struct Rows {
+    typename Src::At at[ROWS];
+    __device__ __forceinline__ Rows(const Src& src, int r0) {
+#pragma unroll
+      for (int c = 0; c < ROWS; ++c) {
+        const int id = (int)threadIdx.x + 256 * c;
+        at[c] = src.at(r0 + (KC ? id / PER : (id % PER) * EPC));
+      }
+    }
+  };
+  template <class Src>
+  __device__ __forceinline__ void load(const Src& src, const Rows<Src>& rows, int k0) {
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int id = (int)threadIdx.x + 256 * c, a = id / PER, b = (id % PER) * EPC;
-      reg[c] = KC ? src.chunk(r0 + a, k0 + b) : src.chunk(r0 + b, k0 + a);
+      const int id = (int)threadIdx.x + 256 * c;
+      reg[c] = src.chunk(rows.at[KC ? c : 0], k0 + (KC ? (id % PER) * EPC : id / PER));
     }
   }
-  __device__ __forceinline__ void store(T* s) const {
+  template <class Src>
+  __device__ __forceinline__ void store(const Src& src, T* s) const {
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
       const int id = (int)threadIdx.x + 256 * c, a = id / PER, b = id % PER;
-      *reinterpret_cast<split_u32x4*>(&s[KC ? at(a, b) : a * LD + b * EPC]) = reg[c];
+      *reinterpret_cast<split_u32x4*>(&s[KC ? at(a, b) : a * LD + b * EPC]) = src.pack(reg[c]);
     }
   }
 };
@@ -135,9 +153,15 @@ struct MatrixSource {
   const T* p;
   int64_t ld;
   int rows, K;
-  __device__ __forceinline__ split_u32x4 chunk(int row, int k) const {
+  using Raw = split_u32x4;
+  struct At {
+    int row;
+  };
+  __device__ __forceinline__ At at(int row) const { return At{row}; }
+  __device__ __forceinline__ split_u32x4 pack(const Raw& r) const { return r; }
+  __device__ __forceinline__ Raw chunk(const At& at, int k) const {
     constexpr int EPC = SplitT<T>::EPC;
-    const int a = KC ? row : k, b = KC ? k : row;  // stored row, first stored column
+    const int a = KC ? at.row : k, b = KC ? k : at.row;  // stored row, first stored column
     const int na = KC ? rows : K, nb = KC ? K : rows;
     const T* q = p + (int64_t)a * ld + b;
     if (a < na && b + EPC <= nb) return *reinterpret_cast<const split_u32x4_any*>(q);
@@ -176,8 +200,8 @@ __global__ __launch_bounds__(256) void k_split_gemm(int M, int N, int K, int nsp
                                                     float* __restrict__ part) {
   constexpr int BK = SplitT<T>::BK, GROUPS = sizeof(T) == 2 ? BK / 16 : BK / 8;
   constexpr int TN = split_tile_cols(TM);
-  using TileA = SplitTile<T, SA::kKC, TM>;
-  using TileB = SplitTile<T, SB::kKC, TN>;
+  using TileA = SplitTile<T, SA::kKC, TM, typename SA::Raw>;
+  using TileB = SplitTile<T, SB::kKC, TN, typename SB::Raw>;
   __shared__ __align__(16) T sA[2][TileA::ELEMS];
   __shared__ __align__(16) T sB[2][TileB::ELEMS];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -201,18 +225,20 @@ __global__ __launch_bounds__(256) void k_split_gemm(int M, int N, int K, int nsp
   f32x16 acc = f32x16{};
   TileA ta;
   TileB tb;
+  const typename TileA::template Rows<SA> ra(A, m0);
+  const typename TileB::template Rows<SB> rb(B, n0);
   if (kbeg < kend) {
-    ta.load(A, m0, kbeg);
-    tb.load(B, n0, kbeg);
-    ta.store(sA[0]);
-    tb.store(sB[0]);
+    ta.load(A, ra, kbeg);
+    tb.load(B, rb, kbeg);
+    ta.store(A, sA[0]);
+    tb.store(B, sB[0]);
   }
   __syncthreads();
   for (int k0 = kbeg, cur = 0; k0 < kend; k0 += BK, cur ^= 1) {
     const bool more = k0 + BK < kend;
     if (more) {  // the next step's chunks in flight during this step's MFMAs
-      ta.load(A, m0, k0 + BK);
-      tb.load(B, n0, k0 + BK);
+      ta.load(A, ra, k0 + BK);
+      tb.load(B, rb, k0 + BK);
     }
 #pragma unroll
     for (int j = 0; j < GROUPS; ++j) {
@@ -226,8 +252,8 @@ __global__ __launch_bounds__(256) void k_split_gemm(int M, int N, int K, int nsp
       }
     }
     if (more) {
-      ta.store(sA[cur ^ 1]);
-      tb.store(sB[cur ^ 1]);
+      ta.store(A, sA[cur ^ 1]);
+      tb.store(B, sB[cur ^ 1]);
     }
     __syncthreads();
   }
@@ -278,21 +304,22 @@ __global__ __launch_bounds__(64 * (G < 4 ? 4 : G)) void k_split_reduce(const flo
   if (in) ep(m, n, s);
 }
 
-// Splits of the contraction for a grid of `tiles` tiles and nk BK-steps:
-// about two workgroups per CU in all, each with at least two steps.  (Three
+// Splits of the contraction for a grid of `tiles` tiles and nk BK-steps: to
+// the nearest, two workgroups per CU in all, each with at least two steps.  (Three
 // or four per CU: bf16 1536^3 22 -> 31 us, fp32 1500^3 106 -> 93 us, most sizes
-// within 5 %.)
+// within 5 %; rounded down, fp32 900 x 1100 x 2000, 270 tiles, 76 -> 110 us;
+// rounded up, bf16 300 x 5000 x 600, 395 tiles, 16.8 -> 18.6.)
 inline int split_count(int64_t tiles, int64_t nk) {
-  int64_t s = (512 + tiles - 1) / (tiles > 0 ? tiles : 1);
+  int64_t s = (512 + tiles / 2) / (tiles > 0 ? tiles : 1);
   if (s > nk / 2) s = nk / 2;
   if (s > 256) s = 256;
   return s < 1 ? 1 : (int)s;
 }
 
 // Scratch of one split product: nsplit x M x N floats, at most
-// kSplitWorkBytes (with more than one split, split_count keeps nsplit x tiles
-// below 1024; a tile is 16 KB).  One fixed size per stream, so the buffer is allocated once.
-constexpr size_t kSplitWorkBytes = size_t(16) << 20;
+// kSplitWorkBytes (with more than one split, nsplit x tiles is below 768; a
+// tile is 16 KB).  One fixed size per stream, so the buffer is allocated once.
+constexpr size_t kSplitWorkBytes = size_t(12) << 20;
 
 // Launches the product on s: N columns and K contraction values (of the
 // largest phase), `phases` phases (1 unless SB::kPhased).  Without scratch (a
