@@ -31,6 +31,7 @@
 // inner loops carry no load guards.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -620,6 +621,26 @@ int launch_dkdv_w64(const u16* q, const u16* k, const u16* v, const u16* dout, c
                     u16* dk, u16* dv, int64_t BH, int64_t Lq, int64_t Lk, float sl2, float scale, bool causal,
                     hipStream_t st);
 
+// Whether the fp32 backward runs two groups of waves per workgroup
+// (attn_bwd_f32_kernel).  Measured, pre-pass included (one / two groups, us):
+//   d = 64, where one group leaves one wave per SIMD whatever the grid: causal
+//   [1,4,1024] 170 / 146, [2,16,2048] 657 / 580, [1,8,4096] 679 / 600, [4,16,512]
+//   111 / 103, [16,16,256] 136 / 132; full [1,8,4096] 1046 / 969, [4,16,400] 125 /
+//   118, [8,8,256] 47.8 / 47.4; [2,8] 100 x 3000 350 / 329, 3000 x 100 440 / 407.  Not
+//   with few tiles to share out: [1,8,128] 25.5 / 27.4, [64,8,128] 100 / 103.5,
+//   [1,8,192] 34.2 / 35.4.
+//   d = 32, where two one-group workgroups share a CU: causal [4,8,777] 105 / 69,
+//   [4,16,1024] 199 / 169, [2,16,2048] 387 / 314, [8,16,512] 113 / 103 (two groups
+//   halve the longest workgroup's chain), but [16,16,256] 67 / 71; full only while
+//   the grid has no second workgroup for the CUs: [2,12,700] (288 workgroups) 90 / 86,
+//   [1,2,1999] 157 / 146, [2,16,512] 44.4 / 43.0, but [4,16,1024] 252 / 276, [1,8,4096] 493 / 511.
+static bool bwd_f32_two_groups(int64_t workgroups, int64_t Lq, int64_t Lk, int d, bool causal) {
+  if (std::min(Lq, Lk) <= 64) return false;
+  const int64_t longest = std::max(Lq, Lk);
+  if (d == 64) return longest >= 256;
+  return longest >= 512 && (causal || workgroups <= 288);
+}
+
 // `delta`: device scratch of 2 * BH * Lq floats that the kernels of this call
 // own until they finish: -D (negated row sums of dO o O), then LSE * log2(e).
 template <typename T, int D, bool CAUSAL>
@@ -661,9 +682,17 @@ static int launch_bwd(const T* q, const T* k, const T* v, const T* o, const floa
       const int64_t nqt = (Lq + BWD_F32_BM - 1) / BWD_F32_BM;
       if (!grid_fits((nkt + nqt) * BH, 256)) return fail(TT_ERR_ARG, "attention backward: grid too large");
       const int gk = pick_group(BH, nkt, 32), gq = pick_group(BH, nqt, 32);
-      hipLaunchKernelGGL((attn_bwd_f32_kernel<D, CAUSAL>), dim3((unsigned)((nkt + nqt) * BH)), dim3(256), 0, st,
-                         q, k, v, dout, lse, delta, dq, dk, dv, (int)Lq, (int)Lk, (int)BH, (int)nkt, (int)nqt,
-                         (int)(nkt * BH), gk, gq, sl2, scale);
+      const auto launch = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((nkt + nqt) * BH)), dim3(threads), 0, st, q, k, v, dout, lse,
+                           delta, dq, dk, dv, (int)Lq, (int)Lk, (int)BH, (int)nkt, (int)nqt, (int)(nkt * BH), gk, gq,
+                           sl2, scale);
+      };
+      bool two_groups = false;
+      if constexpr (D <= 64) {
+        two_groups = bwd_f32_two_groups((nkt + nqt) * BH, Lq, Lk, D, CAUSAL);
+        if (two_groups) launch(attn_bwd_f32_kernel<D, CAUSAL, 2>, 512);
+      }
+      if (!two_groups) launch(attn_bwd_f32_kernel<D, CAUSAL, 1>, 256);
       TT_LAUNCHED("attention backward dQ / dK / dV launch", st);
     }
   }

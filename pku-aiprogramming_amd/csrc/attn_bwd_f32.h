@@ -20,36 +20,63 @@ constexpr int BWD_F32_KN = 64;   // keys per LDS step of the dQ kernel
 // accumulators, and the register-staged prefetch of two 64-query tiles (64
 // more) made the causal kernel spill 61 VGPRs to scratch memory (232 bytes
 // per lane); with 32-query tiles no scratch is used (36 VGPRs are parked in
-// unused AGPRs instead).
-template <int D>
-constexpr int bwd_f32_bq() { return D >= 128 ? 32 : 64; }
+// unused AGPRs instead).  32 also at d = 64 with two groups of waves, which have
+// 256 VGPRs a lane and not 512: 64-query tiles spilled 4-7 of them and were 2-4 %
+// slower.
+template <int D, int KG>
+constexpr int bwd_f32_bq() { return D >= 128 || (D == 64 && KG > 1) ? 32 : 64; }
 
 // LDS floats of each role: Q and dO tiles plus their LSE / -D rows; K and V tiles.
-template <int D>
-constexpr int bwd_f32_dkdv_lds() { return 2 * bwd_f32_bq<D>() * (D + 1) + 2 * bwd_f32_bq<D>(); }
+template <int D, int KG>
+constexpr int bwd_f32_dkdv_lds() { return 2 * bwd_f32_bq<D, KG>() * (D + 1) + 2 * bwd_f32_bq<D, KG>(); }
 template <int D>
 constexpr int bwd_f32_dq_lds() { return 2 * BWD_F32_KN * (D + 1); }
 
+// Adds the accumulators of groups 1 .. KG - 1 to those of group 0, through LDS
+// (16 * ND * 256 floats; every thread of the workgroup calls it).
+template <int KG, int ND>
+__device__ __forceinline__ void bwd_f32_meet(float* smem, int grp, int tid, f32x16 (&acc)[ND]) {
+#pragma unroll
+  for (int k = 1; k < KG; ++k) {
+    __syncthreads();
+    if (grp == k) {
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) smem[(16 * dt + r) * 256 + tid] = acc[dt][r];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[dt][r] += smem[(16 * dt + r) * 256 + tid];
+    }
+  }
+}
+
 // dK / dV of the BWD_F32_BN keys of tile `id` (see map_tile), looping over
-// the query tiles.
-template <int D, bool CAUSAL>
+// the query tiles: KG groups of four waves take them in turn, each through
+// LDS tiles of its own (LDS floats apart), and add up in group order at the end.
+template <int D, bool CAUSAL, int KG, int LDS>
 __device__ __forceinline__ void bwd_f32_dkdv(int id, float* smem, const float* __restrict__ Q,
                                              const float* __restrict__ K, const float* __restrict__ V,
                                              const float* __restrict__ dO, const float* __restrict__ LSE,
                                              const float* __restrict__ NDelta, float* __restrict__ dK,
                                              float* __restrict__ dV, int Lq, int Lk, int BH, int nkt, int group,
                                              float sl2, float scale) {
-  constexpr int BN = BWD_F32_BN, BQ = bwd_f32_bq<D>(), MT = BQ / 32;
+  constexpr int BN = BWD_F32_BN, BQ = bwd_f32_bq<D, KG>(), MT = BQ / 32;
   constexpr int P = D + 1;
   constexpr int NC = D / 2, ND = D / 32, CPR = D / 4;
   constexpr int LPT = BQ * CPR / 256;
   static_assert(BQ * CPR % 256 == 0 && BQ <= 256, "a query tile splits evenly over the 256 threads");
-  float* sQ = smem;
+  const int grp = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  float* sQ = smem + grp * LDS;
   float* sdO = sQ + BQ * P;
   float* sL = sdO + BQ * P;
   float* sDl = sL + BQ;
 
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 5, r32 = l & 31;
+  const int tid = KG > 1 ? threadIdx.x & 255 : threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 5, r32 = l & 31;
   int kt, bh;
   map_tile(id, nkt, BH, group, kt, bh, false);
   const int k0 = kt * BN;
@@ -108,13 +135,14 @@ __device__ __forceinline__ void bwd_f32_dkdv(int id, float* smem, const float* _
   };
 
   const int qstart = CAUSAL ? (k0 / BQ) * BQ : 0;
-  if (qstart < Lq) gload(qstart);
-  for (int qb = qstart; qb < Lq; qb += BQ) {
+  if (qstart + BQ * grp < Lq) gload(qstart + BQ * grp);
+  for (int q1 = qstart; q1 < Lq; q1 += BQ * KG) {
+    const int qb = q1 + BQ * grp;
     __syncthreads();
-    sstore();
+    if (KG == 1 || qb < Lq) sstore();
     __syncthreads();
-    if (qb + BQ < Lq) gload(qb + BQ);
-    if (CAUSAL && qb + BQ - 1 < wk_lo) continue;
+    if (qb + BQ * KG < Lq) gload(qb + BQ * KG);
+    if ((CAUSAL && qb + BQ - 1 < wk_lo) || (KG > 1 && qb >= Lq)) continue;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       f32x16 s = f32x16{}, dp = f32x16{};
@@ -144,6 +172,11 @@ __device__ __forceinline__ void bwd_f32_dkdv(int id, float* smem, const float* _
     }
   }
 
+  if constexpr (KG > 1) {
+    bwd_f32_meet<KG>(smem, grp, tid, adk);
+    bwd_f32_meet<KG>(smem, grp, tid, adv);
+    if (grp > 0) return;
+  }
   if (key < Lk) {
     float* dkrow = dK + kbase + (int64_t)key * D;
     float* dvrow = dV + kbase + (int64_t)key * D;
@@ -160,8 +193,9 @@ __device__ __forceinline__ void bwd_f32_dkdv(int id, float* smem, const float* _
   }
 }
 
-// dQ of the BWD_F32_BM queries of tile `id`, looping over the key tiles.
-template <int D, bool CAUSAL>
+// dQ of the BWD_F32_BM queries of tile `id`, looping over the key tiles (KG
+// groups of waves as above).
+template <int D, bool CAUSAL, int KG, int LDS>
 __device__ __forceinline__ void bwd_f32_dq(int id, float* smem, const float* __restrict__ Q,
                                            const float* __restrict__ K, const float* __restrict__ V,
                                            const float* __restrict__ dO, const float* __restrict__ LSE,
@@ -171,10 +205,11 @@ __device__ __forceinline__ void bwd_f32_dq(int id, float* smem, const float* __r
   constexpr int P = D + 1;
   constexpr int NC = D / 2, ND = D / 32, CPR = D / 4;
   constexpr int LPT = BN * CPR / 256;
-  float* sK = smem;
+  const int grp = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  float* sK = smem + grp * LDS;
   float* sV = sK + BN * P;
 
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 5, r32 = l & 31;
+  const int tid = KG > 1 ? threadIdx.x & 255 : threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 5, r32 = l & 31;
   int qt, bh;
   map_tile(id, nqt, BH, group, qt, bh, CAUSAL);
   const int q0 = qt * BM;
@@ -224,13 +259,14 @@ __device__ __forceinline__ void bwd_f32_dq(int id, float* smem, const float* __r
   };
 
   const int kend = CAUSAL ? min(Lk, q0 + BM) : Lk;
-  if (kend > 0) gload(0);
-  for (int kb = 0; kb < kend; kb += BN) {
+  if (BN * grp < kend) gload(BN * grp);
+  for (int k1 = 0; k1 < kend; k1 += BN * KG) {
+    const int kb = k1 + BN * grp;
     __syncthreads();
-    sstore();
+    if (KG == 1 || kb < kend) sstore();
     __syncthreads();
-    if (kb + BN < kend) gload(kb + BN);
-    if (CAUSAL && kb > wq_hi) continue;
+    if (kb + BN * KG < kend) gload(kb + BN * KG);
+    if ((CAUSAL && kb > wq_hi) || (KG > 1 && kb >= kend)) continue;
     const bool need_mask = (kb + BN > Lk) || (CAUSAL && kb + BN - 1 > wq_lo);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -258,6 +294,10 @@ __device__ __forceinline__ void bwd_f32_dq(int id, float* smem, const float* __r
     }
   }
 
+  if constexpr (KG > 1) {
+    bwd_f32_meet<KG>(smem, grp, tid, adq);
+    if (grp > 0) return;
+  }
   if (qrow < Lq) {
     float* row = dQ + qbase + (int64_t)qrow * D;
 #pragma unroll
@@ -276,19 +316,26 @@ __device__ __forceinline__ void bwd_f32_dq(int id, float* smem, const float* __r
 // only part of the CUs with either; together they fill twice as many.
 // nkblk is nkt * BH, a multiple of 8 when BH is, so the dQ workgroups keep
 // their XCD mapping.
-template <int D, bool CAUSAL>
-__global__ __launch_bounds__(256, 1) void attn_bwd_f32_kernel(
+// With one group of waves (KG = 1) the registers of d = 64 and 128 leave one wave
+// per SIMD, whose MFMAs wait for its own exponentials, LDS reads and barriers.
+// KG = 2 (d <= 64) puts a second group on the same 128 rows and every other
+// tile of the other side, within half the registers: d = 64 causal
+// [2,16,2048] 657 -> 580 us (52 -> 59 TFLOP/s charged), full [1,8,4096] 1046 -> 969.
+template <int D, bool CAUSAL, int KG>
+__global__ __launch_bounds__(256 * KG, 1) void attn_bwd_f32_kernel(
     const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
     const float* __restrict__ dO, const float* __restrict__ LSE, const float* __restrict__ NDelta,
     float* __restrict__ dQ, float* __restrict__ dK, float* __restrict__ dV, int Lq, int Lk, int BH, int nkt,
     int nqt, int nkblk, int gk, int gq, float sl2, float scale) {
-  constexpr int kLds = bwd_f32_dkdv_lds<D>() > bwd_f32_dq_lds<D>() ? bwd_f32_dkdv_lds<D>() : bwd_f32_dq_lds<D>();
-  __shared__ float smem[kLds];
+  constexpr int kLds =
+      bwd_f32_dkdv_lds<D, KG>() > bwd_f32_dq_lds<D>() ? bwd_f32_dkdv_lds<D, KG>() : bwd_f32_dq_lds<D>();
+  static_assert(KG == 1 || KG * kLds >= 256 * D / 2, "the groups meet in the tiles' LDS");
+  __shared__ float smem[KG * kLds];
   const int id = blockIdx.x;
   if (id < nkblk)
-    bwd_f32_dkdv<D, CAUSAL>(id, smem, Q, K, V, dO, LSE, NDelta, dK, dV, Lq, Lk, BH, nkt, gk, sl2, scale);
+    bwd_f32_dkdv<D, CAUSAL, KG, kLds>(id, smem, Q, K, V, dO, LSE, NDelta, dK, dV, Lq, Lk, BH, nkt, gk, sl2, scale);
   else
-    bwd_f32_dq<D, CAUSAL>(id - nkblk, smem, Q, K, V, dO, LSE, NDelta, dQ, Lq, Lk, BH, nqt, gq, sl2, scale);
+    bwd_f32_dq<D, CAUSAL, KG, kLds>(id - nkblk, smem, Q, K, V, dO, LSE, NDelta, dQ, Lq, Lk, BH, nqt, gq, sl2, scale);
 }
 
 }  // namespace tt
