@@ -262,7 +262,7 @@ int tt_attn_decode_f32(const float* q, const float* k, const float* v, float* o,
  * Sum, Div of src/Layers_kernels.cu:189-257, the max and the sum each a host
  * loop of thrust calls per row) with one kernel that reads each element once
  * into registers and writes it once: a wave per row up to 2048 columns, a
- * workgroup per row up to 8192 (65536 without the workspace below), and for
+ * workgroup per row up to 12288 (65536 without the workspace below), and for
  * rows of up to 2 Mi columns 2-64 workgroups per row that merge their (max,
  * sum) partials through a per-stream library workspace of rows x chunks x 16
  * bytes (allocated on first use; if that fails, or under graph capture, the

@@ -14,9 +14,11 @@
 //   cols <= 64:   G = the next power of two >= cols lanes per row, 64 / G
 //                 rows per wave, one element per lane;
 //   cols <= 2048: one wave per row, up to 32 elements per lane in registers;
-//   cols <= 8192 (up to 65536 where rows are not split, below): one workgroup
-//                 of 4 or 16 waves per row, up to 64 elements per lane in
-//                 registers, partials through LDS;
+//   cols <= 3328 (12289 to 65536 where rows are not split, below): one
+//                 workgroup of 4 or 16 waves per row, up to 64 elements per
+//                 lane in registers, partials through LDS;
+//   cols <= 12288: the same with 4 or 8 waves and 16-byte vectors that begin on
+//                 128-byte lines whatever the row length;
 //   longer rows, up to 2 M columns: the row is split over up to 64
 //                 workgroups that each hold their chunk in registers and
 //                 exchange (max, sum) partials through device memory (one
@@ -107,6 +109,84 @@ __global__ __launch_bounds__(kBlock) void k_softmax_reg(const float* __restrict_
       const int c = t + 64 * i;
       if (c < cols) st(&yr[c], v[i] / s);
     }
+  }
+}
+
+// The words that the vector kernels below read and write: four floats at any
+// float alignment (the target reads and writes unaligned global words).
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+typedef f32x4v f32x4u __attribute__((aligned(4)));
+
+// One workgroup of W waves per row, NE4 16-byte vectors per lane in
+// registers: 64 W 4 NE4 floats, the row and `shift` floats before it.  `shift`
+// is the distance of the row's first output element from a 128-byte line, so
+// that a wave's 1 KB store covers whole lines whatever the row length.  Only
+// the first vector can begin before the row and only the last two (the host
+// takes the smallest NE4 that holds 31 floats more than the row) can end
+// behind it: those are read by element, the others without a check.
+template <int NE4, int W>
+__global__ __launch_bounds__(64 * W) void k_softmax_vec(const float* x, float* y, int64_t rows, int cols) {
+  constexpr int STEP = 256 * W;
+  __shared__ float red_m[W], red_s[W];
+  const int t = threadIdx.x, w = t >> 6;
+  for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {  // uniform per workgroup
+    const float* xr = x + r * cols;
+    float* yr = y + r * cols;
+    const int shift = (int)(((uintptr_t)yr / sizeof(float)) % 32);
+    auto col = [&](int k) { return 4 * t + STEP * k - shift; };
+    auto whole = [&](int k) {
+      const bool in_front = k > 0 || col(k) >= 0;
+      return in_front && (k < NE4 - 2 || col(k) + 4 <= cols);
+    };
+    f32x4v v[NE4];
+#pragma unroll
+    for (int k = 0; k < NE4; ++k) {
+      const int c = col(k);
+      if (whole(k)) {
+        v[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(xr + c));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[k][e] = c + e >= 0 && c + e < cols ? ld(xr + c + e) : -INFINITY;
+      }
+    }
+    float m = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < NE4; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m = fmaxf(m, v[k][e]);
+    m = group_max<64>(m);
+    if ((t & 63) == 0) red_m[w] = m;
+    __syncthreads();
+    m = red_m[0];
+#pragma unroll
+    for (int i = 1; i < W; ++i) m = fmaxf(m, red_m[i]);
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < NE4; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[k][e] = ex(v[k][e] - m);  // outside the row: exp(-inf) = 0 (NaN if the whole row is -inf, as it should be)
+        s += v[k][e];
+      }
+    s = group_sum<64>(s);
+    if ((t & 63) == 0) red_s[w] = s;
+    __syncthreads();
+    s = red_s[0];
+#pragma unroll
+    for (int i = 1; i < W; ++i) s += red_s[i];
+#pragma unroll
+    for (int k = 0; k < NE4; ++k) {
+      const int c = col(k);
+      const f32x4v o = v[k] / s;
+      if (whole(k)) {
+        __builtin_nontemporal_store(o, reinterpret_cast<f32x4u*>(yr + c));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e >= 0 && c + e < cols) st(yr + c + e, o[e]);
+      }
+    }
+    __syncthreads();  // red_m / red_s are reused by the next row
   }
 }
 
@@ -243,10 +323,6 @@ __global__ __launch_bounds__(64 * W) void k_softmax_stream(const float* __restri
 // and writes NaN for its chunk.  A workgroup writes only the chunk it has
 // already read, so x == y (in place) is fine.
 constexpr int kSplitMaxChunks = 64;
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-// four floats at any float alignment (the target reads and writes unaligned
-// global words)
-typedef f32x4v f32x4u __attribute__((aligned(4)));
 
 // ALIGNED: cols % 4 == 0 and 16-byte aligned x and y.  Otherwise rows begin
 // at any float and a row's last vector may be partial.
@@ -361,6 +437,43 @@ int blocks_for(int64_t rows, int64_t rows_per_block) {
   return (int)(b < 65536 ? b : 65536);  // grid-stride beyond this
 }
 
+// Row lengths of k_softmax_vec.  It is bound by memory; its 16-byte words on
+// whole lines and the missing exchange between workgroups measured against the
+// kernels before it (4-byte words up to 8192 columns, rows split over
+// workgroups beyond; us, before / now): 10000 x 3500 53 / 47, 12000 x 6001 109 /
+// 96, 10000 x 7000 114 / 91, 8000 x 8191 103 / 90 (5.8 TB/s), 8192 x 10007 119.6 / 110.0 (6.0 TB/s), 8192 x 12288 136 / 131, 1000
+// x 5000 9.2 / 8.2, 1 x 8192 4.7 / 3.4; aligned 4096 and 8192 columns equal.
+// Outside the line: 8000 x 3073 36.1 / 37.2, 20000 x 2049 56.6 / 59.1 (a quarter, a
+// third of the lanes idle), 8192 x 16384 169 / 191 (too few rows in flight).
+constexpr int kVecMin = 3328, kVecMax = 12288;
+
+int launch_vec(const float* x, float* y, int64_t rows, int cols, hipStream_t s) {
+  const int over = cols % 32 ? 31 : (int)(((uintptr_t)y / sizeof(float)) % 32);  // the largest shift
+  const dim3 grid(blocks_for(rows, 1));
+#define TT_VEC(NE4, W)                                                                                        \
+  case NE4:                                                                                                   \
+    hipLaunchKernelGGL((k_softmax_vec<NE4, W>), grid, dim3(64 * W), 0, s, x, y, rows, cols);                  \
+    break
+  if (cols + over <= 8192) {
+    switch ((cols + over + 1023) / 1024) {
+      TT_VEC(4, 4);
+      TT_VEC(5, 4);
+      TT_VEC(6, 4);
+      TT_VEC(7, 4);
+      TT_VEC(8, 4);
+    }
+  } else {
+    switch ((cols + over + 2047) / 2048) {
+      TT_VEC(5, 8);
+      TT_VEC(6, 8);
+      TT_VEC(7, 8);
+    }
+  }
+#undef TT_VEC
+  TT_LAUNCHED("tt_softmax_rows_f32", s);
+  return ok();
+}
+
 }  // namespace
 
 }  // namespace tt
@@ -378,14 +491,14 @@ extern "C" int tt_softmax_rows_f32(const float* x, float* y, int64_t rows, int64
   // Long rows: split over workgroups (k_softmax_split), with chunks of 4096 /
   // 8192 / 16384 / 32768 columns for rows up to 16 Ki / 64 Ki / 256 Ki / 2 Mi
   // columns (measured best on the MI355X for each).  Rows that begin at any
-  // float take unaligned 16-byte words: 8192 x 10007 136 -> 122 us (one 16-wave
-  // workgroup a row, 4-byte loads, before; 115 us at 10008), 1000 x 65535 142 ->
-  // 87, 64 x 50257 16.1 -> 7.7, 200 x 262143 178 -> 82; only a handful of short
-  // rows is no faster (3 x 10007 5.25 / 5.37).  Not under capture (a
+  // float take unaligned 16-byte words: 1000 x 65535 142 -> 87 us (one 16-wave
+  // workgroup a row, 4-byte loads, before), 64 x 50257 16.1 -> 7.7, 200 x 262143
+  // 178 -> 82; only a handful of short rows is no faster.  Not under capture (a
   // replay would find the generation of its last one in the slots), nor
   // without scratch: the kernels below take any length.
+  if (cols > kVecMin && cols <= kVecMax) return launch_vec(x, y, rows, (int)cols, s);
   const bool aligned = cols % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)y % 16) == 0;
-  if (cols > 8192 && cols <= int64_t(kSplitMaxChunks) * 32768 && (aligned || cols > 16384 || rows >= 16) &&
+  if (cols > kVecMax && cols <= int64_t(kSplitMaxChunks) * 32768 && (aligned || cols > 16384 || rows >= 16) &&
       !stream_capturing(s)) {
     const int ne4 = cols <= 16384 ? 4 : cols <= 65536 ? 8 : cols <= 262144 ? 16 : 32;
     const int64_t cw = 1024 * ne4, nchunk = (cols + cw - 1) / cw;
@@ -437,8 +550,7 @@ extern "C" int tt_softmax_rows_f32(const float* x, float* y, int64_t rows, int64
   else if (cols <= 512) TT_REG(8);
   else if (cols <= 1024) TT_REG(16);
   else if (cols <= 2048) TT_REG(32);
-  else if (cols <= 4096) TT_BLOCK(16, 4);
-  else if (cols <= 8192) TT_BLOCK(32, 4);
+  else if (cols <= kVecMin) TT_BLOCK(13, 4);
   else if (cols <= 16384) TT_BLOCK(16, 16);
   else if (cols <= 32768) TT_BLOCK(32, 16);
   else if (cols <= 65536) TT_BLOCK(64, 16);

@@ -51,3 +51,22 @@ def test_chunks_without_finite_values(capi):
     keep = np.delete(np.arange(18), bad)
     assert orc.max_rel_err(y[keep], orc.softmax_rows_f64(x[keep])) <= 1e-5
     assert np.all(y[2, :4096] == 0) and np.all(y[3, 12288:] == 0)
+
+
+# one workgroup per row, vectors from 128-byte lines: around its range and the
+# counts of vectors per lane (1024 k and 2048 k floats less the shift of up to 31)
+@pytest.mark.parametrize("cols", [3328, 3329, 4064, 4065, 4096, 4097, 8160, 8161, 8162, 8192, 8193, 10209, 10240, 12257,
+                                  12288])
+@pytest.mark.parametrize("xo,yo", [(0, 0), (1, 2), (3, 31)])
+def test_vector_rows(capi, cols, xo, yo):
+    x = (3 * np.random.default_rng(cols).standard_normal((37, cols))).astype(np.float32)
+    x[3, :] = -np.inf
+    x[4, -1] = np.nan
+    x[5, 0] = np.inf
+    x[6, 1:] = -np.inf
+    keep = np.delete(np.arange(37), [3, 4, 5])
+    ref = orc.softmax_rows_f64(x[keep])
+    for in_place in (False, True):
+        y = _run(capi, x, xo, yo, in_place)
+        assert np.isnan(y[[3, 4]]).all() and np.isnan(y[5, 0])
+        assert orc.max_rel_err(y[keep], ref) <= 1e-5
