@@ -525,6 +525,85 @@ struct PlaneEpilogue {
   }
 };
 
+// dX at stride 1 with few input channels.  The product's rows are the input
+// channels, so that with one of them 31 of 32 rows of its tiles are padding.
+// Here a lane owns a pixel (and all C channels), four groups of lanes of the workgroup take
+// the output channels in turn and meet in LDS, and the weights lie in LDS,
+// read by all lanes of a wave at once.  What is left are the reads of gO: kh kw of
+// them per pixel and output channel, all but the first from the caches.
+constexpr int kFewChannels = 4, kFewWeights = 8192;
+
+template <typename T, int C>
+__global__ __launch_bounds__(256) void k_conv_dx_few(const T* __restrict__ w, const T* __restrict__ go, T* __restrict__ gx,
+                                                     ConvGeom g, int cout, int64_t pixels) {
+  extern __shared__ float s_w[];  // [cout][kh kw][C]
+  __shared__ float red[4][C][64];
+  const int kk = g.kh * g.kw, l = threadIdx.x & 63, grp = threadIdx.x >> 6, P = g.oh * g.ow;
+  for (int i = threadIdx.x; i < cout * C * kk; i += 256) {
+    const int co = i / (C * kk), r = i - co * (C * kk), c = r / kk;
+    s_w[co * C * kk + (r - c * kk) * C + c] = split_load(w + i);
+  }
+  __syncthreads();
+  const int64_t p = (int64_t)blockIdx.x * 64 + l, HW = (int64_t)g.H * g.W;
+  const int64_t n = p / HW;
+  const int q = (int)(p - n * HW), y = q / g.W + g.ph, x = q % g.W + g.pw;
+  float acc[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) acc[c] = 0.f;
+  if (p < pixels) {
+    const T* gon = go + n * cout * P;
+    for (int co = grp; co < cout; co += 4) {
+      const T* plane = gon + (int64_t)co * P;
+      const float* wc = s_w + co * C * kk;
+      for (int ky = 0; ky < g.kh; ++ky) {
+        const int oy = y - ky;
+        const bool row = oy >= 0 && oy < g.oh;
+#pragma unroll 5
+        for (int kx = 0; kx < g.kw; ++kx) {
+          const int ox = x - kx;
+          const bool in = row && ox >= 0 && ox < g.ow;
+          const float v = split_load(plane + (in ? oy * g.ow + ox : 0));
+#pragma unroll
+          for (int c = 0; c < C; ++c) acc[c] = fmaf(wc[(ky * g.kw + kx) * C + c], in ? v : 0.f, acc[c]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c) red[grp][c][l] = acc[c];
+  __syncthreads();
+  if (grp < C && p < pixels)  // C <= 4 groups: one channel each
+    split_store(gx + (n * C + grp) * HW + q, (red[0][grp][l] + red[1][grp][l]) + (red[2][grp][l] + red[3][grp][l]));
+}
+
+// Whether k_conv_dx_few takes the image gradient.  Measured (the whole
+// backward, us, product / this kernel): fp32 64 x 1 x 28 x 28, 8 kernels 5 x 5 46 /
+// 23; 64 x 3 x 32 x 32, 64 3 x 3 78 / 61; 16 x 3 x 224 x 224, 64 3 x 3 730 / 479; 32 x
+// 4 x 64 x 64, 128 3 x 3 248 / 192; one 28 x 28 image 26 / 15; bf16 alike (697 / 417 at
+// 224 x 224).  The error against float64 is half of the product's.  The weights'
+// 32 KB leave four workgroups per CU.
+bool few_channels(const ConvGeom& g, int64_t N, int cout) {
+  const int64_t weights = (int64_t)cout * g.C * g.kh * g.kw;
+  return g.C <= kFewChannels && g.sh == 1 && g.sw == 1 && weights <= kFewWeights &&
+         grid_fits((N * g.H * g.W + 63) / 64, 256);
+}
+
+template <typename T>
+int launch_few_channels(const char* fn, const T* w, const T* go, T* gin, int64_t N, int cout, const ConvGeom& g,
+                        hipStream_t s) {
+  const int64_t pixels = N * g.H * g.W;
+  const dim3 grid((unsigned)((pixels + 63) / 64));
+  const size_t lds = sizeof(float) * cout * g.C * g.kh * g.kw;
+  switch (g.C) {
+    case 1: hipLaunchKernelGGL((k_conv_dx_few<T, 1>), grid, dim3(256), lds, s, w, go, gin, g, cout, pixels); break;
+    case 2: hipLaunchKernelGGL((k_conv_dx_few<T, 2>), grid, dim3(256), lds, s, w, go, gin, g, cout, pixels); break;
+    case 3: hipLaunchKernelGGL((k_conv_dx_few<T, 3>), grid, dim3(256), lds, s, w, go, gin, g, cout, pixels); break;
+    default: hipLaunchKernelGGL((k_conv_dx_few<T, 4>), grid, dim3(256), lds, s, w, go, gin, g, cout, pixels); break;
+  }
+  TT_LAUNCHED(fn, s);
+  return ok();
+}
+
 ConvDivs conv_divs(const ConvGeom& g) {
   return ConvDivs{FastDiv(g.kh * g.kw), FastDiv(g.kw), FastDiv(g.oh * g.ow), FastDiv(g.ow)};
 }
@@ -588,6 +667,7 @@ int conv_backward(const char* fn, const T* in, const T* w, const T* go, T* gin, 
     }
     return ok();
   }
+  if (few_channels(g, N, cout)) return launch_few_channels(fn, w, go, gin, N, cout, g, s);
   const int phases_x = std::min(g.sw, g.W);
   const int64_t phases = (int64_t)std::min(g.sh, g.H) * phases_x;
   const int64_t pixels = (int64_t)((g.H + g.sh - 1) / g.sh) * ((g.W + g.sw - 1) / g.sw);  // of the largest phase
