@@ -531,7 +531,7 @@ struct PlaneEpilogue {
 // the output channels in turn and meet in LDS, and the weights lie in LDS,
 // read by all lanes of a wave at once.  What is left are the reads of gO: kh kw of
 // them per pixel and output channel, all but the first from the caches.
-constexpr int kFewChannels = 4, kFewWeights = 8192;
+constexpr int kFewChannels = 4;
 
 template <typename T, int C>
 __global__ __launch_bounds__(256) void k_conv_dx_few(const T* __restrict__ w, const T* __restrict__ go, T* __restrict__ gx,
@@ -578,20 +578,20 @@ __global__ __launch_bounds__(256) void k_conv_dx_few(const T* __restrict__ w, co
 
 // Whether k_conv_dx_few takes the image gradient.  Measured (the whole
 // backward, us, product / this kernel): fp32 64 x 1 x 28 x 28, 8 kernels 5 x 5 46 /
-// 23; 64 x 3 x 32 x 32, 64 3 x 3 78 / 61; 16 x 3 x 224 x 224, 64 3 x 3 730 / 479; 32 x
-// 4 x 64 x 64, 128 3 x 3 248 / 192; one 28 x 28 image 26 / 15; bf16 alike (697 / 417 at
-// 224 x 224).  The error against float64 is half of the product's.  The weights'
-// 32 KB leave four workgroups per CU.  A lane's loads are one chain, kw of them in
-// flight at a time, where the product splits its contraction: with fewer
-// workgroups than two per CU the chain stays near the longest measured there
-// (75, ten 28 x 28 images with 10 kernels 5 x 5: 25.5 / 17.0), with more near 2000
-// (64 x 1 x 28 x 28, 320 kernels 5 x 5: 814 / 268), and narrow kernels stay on the
-// product.
+// 23; 64 x 3 x 32 x 32, 64 3 x 3 78 / 61; 16 x 3 x 224 x 224, 64 3 x 3 730 / 479; one
+// 28 x 28 image 26 / 15; bf16 alike (697 / 417 at 224 x 224).  The error against
+// float64 is half of the product's.  A lane's loads are one chain, kw of them in
+// flight at a time, where the product splits its contraction: on grids below
+// three workgroups per CU the chain stays near the longest measured there (75, ten
+// 28 x 28 images with 10 kernels 5 x 5: 25.5 / 17.0), beyond near 144 (64 x 3 x 32 x
+// 32 above), or 512 for one channel, where nearly all of the product is padding.  Longer
+// ones lost in bf16 (8 x 4 x 64 x 64, 80 kernels 4 x 4, chain 320, 78 / 95; 8 x 1 x 64 x
+// 64, 512 kernels, chain 2048, 354 / 417), and kernels narrower than three columns
+// stay on the product.  The weights in LDS are then at most 10 KB.
 bool few_channels(const ConvGeom& g, int64_t N, int cout) {
-  const int64_t weights = (int64_t)cout * g.C * g.kh * g.kw, chain = (int64_t)((cout + 3) / 4) * g.kh * g.kw;
-  const int64_t workgroups = (N * g.H * g.W + 63) / 64;
-  return g.C <= kFewChannels && g.sh == 1 && g.sw == 1 && g.kw >= 3 && weights <= kFewWeights &&
-         chain <= (workgroups < 512 ? 96 : 2048) && grid_fits(workgroups, 256);
+  const int64_t chain = (int64_t)((cout + 3) / 4) * g.kh * g.kw, workgroups = (N * g.H * g.W + 63) / 64;
+  return g.C <= kFewChannels && g.sh == 1 && g.sw == 1 && g.kw >= 3 &&
+         chain <= (workgroups < 768 ? 96 : g.C == 1 ? 512 : 160) && grid_fits(workgroups, 256);
 }
 
 template <typename T>

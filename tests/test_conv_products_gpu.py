@@ -32,16 +32,17 @@ CASES = [
     (1, 40, 14, 14, 200, 3, 3, 1, 1, 2, 2),  # and by phases
     # dX of few channels at stride 1: its channel counts, output channels around
     # its four groups, a ragged last workgroup, pads beyond the kernel, the
-    # longest chain of a small grid and beyond, and the most weights its LDS
-    # takes and one channel more
+    # longest chains of a small and a large grid and one output channel more
     (3, 1, 9, 7, 8, 5, 5, 2, 2, 1, 1),
     (2, 2, 8, 8, 3, 3, 4, 1, 0, 1, 1),
     (1, 3, 5, 17, 5, 2, 7, 3, 8, 1, 1),
     (2, 4, 12, 11, 9, 3, 3, 0, 0, 1, 1),
     (1, 4, 6, 9, 24, 4, 4, 1, 2, 1, 1),
     (1, 4, 6, 9, 25, 4, 4, 1, 2, 1, 1),
-    (8, 4, 64, 64, 128, 4, 4, 1, 2, 1, 1),
-    (8, 4, 64, 64, 129, 4, 4, 1, 2, 1, 1),
+    (12, 4, 64, 64, 40, 4, 4, 1, 2, 1, 1),
+    (12, 4, 64, 64, 41, 4, 4, 1, 2, 1, 1),
+    (12, 1, 64, 64, 128, 4, 4, 1, 2, 1, 1),
+    (12, 1, 64, 64, 129, 4, 4, 1, 2, 1, 1),
     (2, 5, 6, 9, 6, 3, 3, 1, 1, 1, 1),
 ]
 
