@@ -26,7 +26,6 @@
 #include <map>
 #include <mutex>
 #include <string>
-#include <unordered_map>
 #include <utility>
 
 namespace tt {
@@ -172,6 +171,16 @@ class BlockCache {
   }
 
  public:
+  // Whether [p, p + bytes) lies inside one live block.
+  bool holds(const void* p, size_t bytes) {
+    std::lock_guard<std::mutex> lk(mu_);
+    auto it = live_.upper_bound(const_cast<void*>(p));
+    if (it == live_.begin()) return false;
+    --it;
+    const size_t at = (size_t)((uintptr_t)p - (uintptr_t)it->first);
+    return at <= it->second && bytes <= it->second - at;
+  }
+
   // Return every cached (free) block to the device, whose release waits for
   // work that may still use it.
   void trim() {
@@ -196,7 +205,7 @@ class BlockCache {
   Backend& be_;
   std::mutex mu_;
   Blocks free_, ordered_;
-  std::unordered_map<void*, size_t> live_;  // block -> class size
+  std::map<void*, size_t> live_;  // block -> class size
   size_t in_use_ = 0, cached_ = 0;
 };
 

@@ -9,9 +9,10 @@
 // one of three pinned buffers while the DMA engine moves the others.  Converting
 // copies (float32 host values <-> bf16 device storage) do the conversion in
 // that same pass, so no intermediate host array is made.  Downloads of up to
-// kSmallMax host bytes are written by a kernel straight into a pinned buffer
-// (widening bf16 on the way).  Other plain copies below kDirectMax, and copies
-// whose host side is already pinned, go straight to hipMemcpyAsync.
+// kSmallMax host bytes from the library's own blocks are written by a kernel
+// straight into a pinned buffer (widening bf16 on the way).  Other plain copies
+// below kDirectMax, and copies whose host side is already pinned, go straight to
+// hipMemcpyAsync.
 #include <hip/hip_runtime.h>
 #include <sched.h>
 #include <unistd.h>
@@ -285,7 +286,9 @@ HostMem host_mem(const void* p) {
 // kernel that stores into mapped pinned memory costs a launch: 4 bytes 20.6 ->
 // 12.1 us, 10 KB 24.8 -> 12.8 us, 313 KB 32.0 -> 24.8 us (numpy(), with the
 // wait); at 800 KB the kernel's stores over the link and the host copy after
-// them lose (41.6 / 44.9 us).
+// them lose (41.6 / 44.9 us).  A kernel reads whatever address it is given, so
+// the source must lie inside a live block of the library's allocator; any other
+// pointer or range goes to the runtime, which checks it.
 constexpr size_t kSmallMax = size_t(512) << 10;  // host bytes
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
@@ -302,12 +305,13 @@ __global__ __launch_bounds__(256) void k_download_bf16(const uint16_t* __restric
 std::mutex g_small_mu;
 void *g_small_host = nullptr, *g_small_dev = nullptr;  // kSmallMax pinned bytes, kept until the process ends
 
-// Download `bytes` host bytes (a kernel launched by `launch(device address of
-// the pinned buffer, workgroups)`), or return -1 where the caller must take
-// another path: too large, no pinned memory, a stream under capture.
+// Download `bytes` host bytes made of the src_bytes at src (a kernel launched by
+// `launch(device address of the pinned buffer, workgroups)`), or return -1 where
+// the caller must take another path: too large, a source that is not known to
+// hold them, no pinned memory, a stream under capture.
 template <class Launch>
-int small_d2h(void* dst, size_t bytes, hipStream_t s, Launch&& launch) {
-  if (bytes > kSmallMax || stream_capturing(s)) return -1;
+int small_d2h(void* dst, size_t bytes, const void* src, size_t src_bytes, hipStream_t s, Launch&& launch) {
+  if (bytes > kSmallMax || !device_block_holds(src, src_bytes) || stream_capturing(s)) return -1;
   std::lock_guard<std::mutex> lk(g_small_mu);
   if (!g_small_host) {
     void *h = nullptr, *d = nullptr;
@@ -369,7 +373,7 @@ int tt_memcpy_d2h(void* dst, const void* src, size_t bytes) {
   if (hm == HostMem::kDevice)
     return fail(TT_ERR_ARG, "tt_memcpy_d2h: destination is device memory (use tt_memcpy_d2d)");
   if (hm == HostMem::kPageable && (uintptr_t)src % 16 == 0) {
-    rc = small_d2h(dst, bytes, s, [&](void* out, unsigned blocks) {
+    rc = small_d2h(dst, bytes, src, bytes, s, [&](void* out, unsigned blocks) {
       hipLaunchKernelGGL(k_download, dim3(blocks), dim3(256), 0, s, (const unsigned char*)src, (unsigned char*)out,
                          (int)bytes);
     });
@@ -404,7 +408,7 @@ int tt_download_bf16_to_f32(float* dst, const void* src, size_t n) {
     return fail(TT_ERR_ARG, "tt_download_bf16_to_f32: destination is device memory");
   hipStream_t s = stream_or_default(nullptr);
   if (n <= kSmallMax / 4) {
-    rc = small_d2h(dst, 4 * n, s, [&](void* out, unsigned blocks) {
+    rc = small_d2h(dst, 4 * n, src, 2 * n, s, [&](void* out, unsigned blocks) {
       hipLaunchKernelGGL(k_download_bf16, dim3(blocks), dim3(256), 0, s, (const uint16_t*)src, (uint32_t*)out, (int)n);
     });
     if (rc >= 0) return rc;

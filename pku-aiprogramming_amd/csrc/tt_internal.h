@@ -32,6 +32,10 @@ void after_launch(hipStream_t s);
 // nothing and leaves no scratch address behind).
 bool stream_capturing(hipStream_t s);
 
+// Whether [p, p + bytes) lies inside one block that tt_malloc or
+// tt_malloc_ordered handed out and that was not freed.
+bool device_block_holds(const void* p, size_t bytes);
+
 // The allocation-free backward's scratch: a static device array of
 // kNoAllocScratchBytes whose device address tt_init looks up once per
 // device.  Returns nullptr before tt_init; *bytes gets the array's size.

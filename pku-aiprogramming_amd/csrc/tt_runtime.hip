@@ -110,6 +110,8 @@ static HipBackend g_backend;
 static BlockCache<HipBackend> g_blocks(g_backend);
 static WorkspaceCache<HipBackend> g_ws(g_backend, g_blocks);
 
+bool device_block_holds(const void* p, size_t bytes) { return g_blocks.holds(p, bytes); }
+
 // ---------------------------------------------------------------- instrumentation
 // Events to record after the next launches (tt_set_launch_events).  The
 // count is read without the lock, so launches pay nothing while none is set.

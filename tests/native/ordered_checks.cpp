@@ -1,6 +1,7 @@
 // BlockCache's stream-ordered blocks (csrc/device_cache.h) over a malloc
 // backend: only alloc_ordered hands a release_ordered block out before
-// settle, a failed wait keeps it apart, trim returns it, counts stay whole.
+// settle, a failed wait keeps it apart, trim returns it, counts stay whole, and
+// holds (which lets a kernel read a caller's range) knows where blocks end.
 #include <cstdio>
 #include <cstdlib>
 
@@ -20,7 +21,26 @@ struct Backend {
   void release(void* p) { std::free(p), ++releases; }
 };
 
+static void holds_checks() {
+  Backend be;
+  BlockCache<Backend> bc(be);
+  char host[64], *a, *b;
+  CHECK(!bc.holds(host, 1));
+  CHECK(bc.alloc(4096, (void**)&a) == 0 && bc.alloc_ordered(1000, (void**)&b) == 0);  // b: a class of 1024
+  for (char* p : {a, b}) {
+    const size_t n = p == a ? 4096 : 1024;
+    CHECK(bc.holds(p, n) && bc.holds(p + 16, n - 16) && bc.holds(p + n - 1, 1) && bc.holds(p, 0));
+    CHECK(!bc.holds(p, n + 1) && !bc.holds(p + 16, n - 15) && !bc.holds(p + n, 1));
+    CHECK(!bc.holds(p, ~size_t(0)) && !bc.holds(p + 16, ~size_t(0)));
+  }
+  CHECK(!bc.holds(nullptr, 1) && !bc.holds(host, 1));
+  CHECK(bc.release(a) && !bc.holds(a, 1) && bc.holds(b, 1));  // cached, not live
+  CHECK(bc.release_ordered(b) && !bc.holds(b, 1));
+  bc.trim();
+}
+
 int main() {
+  holds_checks();
   Backend be;
   BlockCache<Backend> bc(be);
   void *a = nullptr, *b = nullptr, *c = nullptr;
