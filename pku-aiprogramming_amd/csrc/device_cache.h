@@ -97,6 +97,11 @@ class BlockCache {
     }
     return alloc_new(cls, ptr);
   }
+
+  // false if `p` is not a live block of this cache (nullptr is fine).
+  bool release(void* p) { return release_to(free_, p); }
+  bool release_ordered(void* p) { return release_to(ordered_, p); }
+
   // Whether alloc(bytes) would need a new block although settle could free one.
   bool wants_settle(size_t bytes) {
     const size_t cls = block_size_class(bytes);
@@ -104,22 +109,67 @@ class BlockCache {
     return !fits(free_, cls) && fits(ordered_, cls);
   }
   // Make the release_ordered blocks of before this call available to alloc,
-  // after `wait` (0 = success) has waited for their stream.
+  // after `wait` (0 = success) has waited for their stream.  The blocks stay
+  // where they are meanwhile: other threads may take or trim them, and those
+  // released during the wait are not covered by it.
   template <class Wait>
   int settle(Wait&& wait) {
-    std::multimap<size_t, void*> blocks;
+    uint64_t before;
     {
       std::lock_guard<std::mutex> lk(mu_);
-      blocks.swap(ordered_);
+      before = releases_;
     }
     const int rc = wait();
+    if (rc) return rc;
     std::lock_guard<std::mutex> lk(mu_);
-    (rc ? ordered_ : free_).insert(blocks.begin(), blocks.end());
-    return rc;
+    for (auto it = ordered_.begin(); it != ordered_.end();) {
+      if (it->second.released <= before) {
+        free_.insert(*it);
+        it = ordered_.erase(it);
+      } else {
+        ++it;
+      }
+    }
+    return 0;
+  }
+
+  // Return every cached (free) block to the device, whose release waits for
+  // work that may still use it.
+  void trim() {
+    Blocks blocks;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      blocks.swap(free_);
+      blocks.insert(ordered_.begin(), ordered_.end());
+      ordered_.clear();
+      cached_ = 0;
+    }
+    for (auto& kv : blocks) be_.release(kv.second.p);
+  }
+
+  // Whether [p, p + bytes) lies inside one live block.
+  bool holds(const void* p, size_t bytes) {
+    std::lock_guard<std::mutex> lk(mu_);
+    auto it = live_.upper_bound(const_cast<void*>(p));
+    if (it == live_.begin()) return false;
+    --it;
+    const size_t at = (size_t)((uintptr_t)p - (uintptr_t)it->first);
+    return at <= it->second && bytes <= it->second - at;
+  }
+
+  void stats(size_t* in_use, size_t* cached) {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (in_use) *in_use = in_use_;
+    if (cached) *cached = cached_;
   }
 
  private:
-  using Blocks = std::multimap<size_t, void*>;
+  struct Block {
+    void* p;
+    uint64_t released;  // the value of releases_ that its release made
+  };
+  using Blocks = std::multimap<size_t, Block>;  // by class size
+
   static bool fits(const Blocks& list, size_t cls) {
     auto it = list.lower_bound(cls);
     return it != list.end() && it->first <= 2 * cls;
@@ -127,7 +177,7 @@ class BlockCache {
   bool take(Blocks& list, size_t cls, void** ptr) {
     auto it = list.lower_bound(cls);
     if (it == list.end() || it->first > 2 * cls) return false;
-    void* p = it->second;
+    void* p = it->second.p;
     const size_t c = it->first;
     list.erase(it);
     live_[p] = c;
@@ -150,13 +200,6 @@ class BlockCache {
     *ptr = p;
     return 0;
   }
-
- public:
-  // false if `p` is not a live block of this cache (nullptr is fine).
-  bool release(void* p) { return release_to(free_, p); }
-  bool release_ordered(void* p) { return release_to(ordered_, p); }
-
- private:
   bool release_to(Blocks& list, void* p) {
     if (!p) return true;
     std::lock_guard<std::mutex> lk(mu_);
@@ -165,48 +208,17 @@ class BlockCache {
     const size_t c = it->second;
     live_.erase(it);
     in_use_ -= c;
-    list.emplace(c, p);
+    list.emplace(c, Block{p, ++releases_});
     cached_ += c;
     return true;
   }
 
- public:
-  // Whether [p, p + bytes) lies inside one live block.
-  bool holds(const void* p, size_t bytes) {
-    std::lock_guard<std::mutex> lk(mu_);
-    auto it = live_.upper_bound(const_cast<void*>(p));
-    if (it == live_.begin()) return false;
-    --it;
-    const size_t at = (size_t)((uintptr_t)p - (uintptr_t)it->first);
-    return at <= it->second && bytes <= it->second - at;
-  }
-
-  // Return every cached (free) block to the device, whose release waits for
-  // work that may still use it.
-  void trim() {
-    std::multimap<size_t, void*> blocks;
-    {
-      std::lock_guard<std::mutex> lk(mu_);
-      blocks.swap(free_);
-      blocks.insert(ordered_.begin(), ordered_.end());
-      ordered_.clear();
-      cached_ = 0;
-    }
-    for (auto& kv : blocks) be_.release(kv.second);
-  }
-
-  void stats(size_t* in_use, size_t* cached) {
-    std::lock_guard<std::mutex> lk(mu_);
-    if (in_use) *in_use = in_use_;
-    if (cached) *cached = cached_;
-  }
-
- private:
   Backend& be_;
   std::mutex mu_;
   Blocks free_, ordered_;
   std::map<void*, size_t> live_;  // block -> class size
   size_t in_use_ = 0, cached_ = 0;
+  uint64_t releases_ = 0;
 };
 
 // Scratch buffers of the attention launchers, one per (stream, user): two

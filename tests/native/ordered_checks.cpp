@@ -39,8 +39,40 @@ static void holds_checks() {
   bc.trim();
 }
 
+// Another thread's calls while settle waits (made from inside the wait).
+static void settle_window_checks() {
+  Backend be;
+  BlockCache<Backend> bc(be);
+  void *a, *b, *c = nullptr;
+  size_t used, cached;
+  // a trim returns the waiting blocks too, and the counts stay whole
+  CHECK(bc.alloc_ordered(4096, &a) == 0 && bc.release_ordered(a));
+  CHECK(bc.settle([&] { return bc.trim(), 0; }) == 0);
+  CHECK(be.releases == 1);
+  CHECK(bc.alloc(4096, &a) == 0 && bc.release(a) && bc.alloc(4096, &a) == 0);
+  bc.stats(&used, &cached);
+  CHECK(used == 4096 && cached == 0);
+  // one taken meanwhile is gone; one released meanwhile is not covered by the wait
+  CHECK(bc.alloc_ordered(8192, &b) == 0 && bc.alloc_ordered(8192, &c) == 0);
+  CHECK(bc.release_ordered(b));
+  void* d = nullptr;
+  CHECK(bc.settle([&] {
+    CHECK(bc.alloc_ordered(8192, &d) == 0 && d == b);
+    CHECK(bc.release_ordered(c));
+    return 0;
+  }) == 0);
+  bc.stats(&used, &cached);
+  CHECK(used == 4096 + 8192 && cached == 8192);
+  CHECK(bc.wants_settle(8192));  // c waits still
+  CHECK(bc.release(a) && bc.release(d));
+  bc.trim();
+  bc.stats(&used, &cached);
+  CHECK(used == 0 && cached == 0);
+}
+
 int main() {
   holds_checks();
+  settle_window_checks();
   Backend be;
   BlockCache<Backend> bc(be);
   void *a = nullptr, *b = nullptr, *c = nullptr;
