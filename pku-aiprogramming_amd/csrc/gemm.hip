@@ -503,11 +503,9 @@ int col_sum_launch(const char* fn, const T* x, T* y, int64_t rows, int64_t cols,
   float* part = nullptr;
   std::optional<WorkspaceLease> ws;  // held until the second launch is queued
   // the partials share the split products' buffer; without it one block takes every row
-  if (blocks > 1 && ((size_t)(blocks * cols) * sizeof(float) > kSplitWorkBytes || stream_capturing(s) ||
-                     ws.emplace().get(s, kWsGemmSplits, kSplitWorkBytes, (void**)&part) != TT_OK)) {
+  if (blocks > 1 && ((size_t)(blocks * cols) * sizeof(float) > kSplitWorkBytes ||
+                     !ws.emplace().get_optional(s, kWsGemmSplits, kSplitWorkBytes, (void**)&part)))
     blocks = 1;
-    part = nullptr;
-  }
   if (blocks <= 1) {
     hipLaunchKernelGGL((k_col_sum<T, T>), dim3((unsigned)gx), dim3(1024), 0, s, x, y, rows, cols, rows);
     TT_LAUNCHED(fn, s);

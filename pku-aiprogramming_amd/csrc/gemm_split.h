@@ -337,11 +337,7 @@ int launch_split_tiles(const char* fn, int64_t M, int64_t N, int64_t K, int phas
     return fail(TT_ERR_ARG, std::string(fn) + ": too large");
   float* part = nullptr;
   std::optional<WorkspaceLease> ws;  // held until the reduction is queued
-  if (nsplit > 1 &&
-      (stream_capturing(s) || ws.emplace().get(s, kWsGemmSplits, kSplitWorkBytes, (void**)&part) != TT_OK)) {
-    nsplit = 1;
-    part = nullptr;
-  }
+  if (nsplit > 1 && !ws.emplace().get_optional(s, kWsGemmSplits, kSplitWorkBytes, (void**)&part)) nsplit = 1;
   hipLaunchKernelGGL((k_split_gemm<T, TM, SA, SB, EP>), dim3((unsigned)gx, (unsigned)gy, (unsigned)(phases * nsplit)),
                      dim3(256), 0, s, (int)M, (int)N, (int)K, nsplit, A, B, ep, part);
   TT_LAUNCHED(fn, s);

@@ -498,8 +498,7 @@ extern "C" int tt_softmax_rows_f32(const float* x, float* y, int64_t rows, int64
   // without scratch: the kernels below take any length.
   if (cols > kVecMin && cols <= kVecMax) return launch_vec(x, y, rows, (int)cols, s);
   const bool aligned = cols % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)y % 16) == 0;
-  if (cols > kVecMax && cols <= int64_t(kSplitMaxChunks) * 32768 && (aligned || cols > 16384 || rows >= 16) &&
-      !stream_capturing(s)) {
+  if (cols > kVecMax && cols <= int64_t(kSplitMaxChunks) * 32768 && (aligned || cols > 16384 || rows >= 16)) {
     const int ne4 = cols <= 16384 ? 4 : cols <= 65536 ? 8 : cols <= 262144 ? 16 : 32;
     const int64_t cw = 1024 * ne4, nchunk = (cols + cw - 1) / cw;
     unsigned long long* slots = nullptr;
@@ -507,7 +506,7 @@ extern "C" int tt_softmax_rows_f32(const float* x, float* y, int64_t rows, int64
     const size_t bytes = (size_t)(rows * nchunk) * 2 * sizeof(unsigned long long);
     std::optional<WorkspaceLease> ws;  // held until the kernel that reads the slots is queued
     if (grid_fits(rows * nchunk, kBlock) &&
-        ws.emplace().get(s, kWsSoftmaxPartials, bytes, (void**)&slots, &uses) == TT_OK) {
+        ws.emplace().get_optional(s, kWsSoftmaxPartials, bytes, (void**)&slots, &uses)) {
       const unsigned gen = (unsigned)(uses % 0xffffffffull) + 1;  // 1 .. 2^32 - 1
       if (gen == 1 &&  // a new buffer (or a wrapped count): no word may hold a live generation
           (rc = tt_elementwise(TT_EW_FILL, TT_F32, slots, nullptr, nullptr, (int64_t)(bytes / 4), 0.0, 0.0, 0, s)))

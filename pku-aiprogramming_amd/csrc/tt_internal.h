@@ -56,6 +56,12 @@ class WorkspaceLease {
   // *uses (optional): earlier get() calls that returned the same buffer (0:
   // a new buffer with undefined contents).
   int get(hipStream_t stream, int user, size_t bytes, void** ptr, uint64_t* uses = nullptr);
+  // For a launcher that also runs without the buffer: true and *ptr, or false
+  // where none may be had (a refused allocation; a stream under capture, whose
+  // graph would keep the address; the library stream under capture, which a new
+  // buffer would order the stream behind).  Leaves captures of other streams
+  // alone: an allocation of this thread would end them otherwise.
+  bool get_optional(hipStream_t stream, int user, size_t bytes, void** ptr, uint64_t* uses = nullptr);
 
  private:
   struct Impl;

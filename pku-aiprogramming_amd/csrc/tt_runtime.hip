@@ -67,6 +67,21 @@ bool stream_capturing(hipStream_t s) {
   return st != hipStreamCaptureStatusNone;
 }
 
+// While it lives, this thread's allocations and waits do not end the captures
+// of other streams (or fail because of them): for runtime calls that a library
+// call makes on its own account.
+class RelaxedCapture {
+ public:
+  RelaxedCapture() : set_(hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess) {}
+  ~RelaxedCapture() {
+    if (set_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+  }
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;  // the thread's own mode, once exchanged
+  bool set_;
+};
+
 // ---------------------------------------------------------------- allocator
 // hipMalloc / hipFree / hipStreamSynchronize as the backend of the caching
 // allocator and the workspace cache (device_cache.h).  Allocation failures,
@@ -151,6 +166,11 @@ WorkspaceLease::WorkspaceLease() : impl_(new Impl) {}
 WorkspaceLease::~WorkspaceLease() { delete impl_; }
 int WorkspaceLease::get(hipStream_t s, int user, size_t bytes, void** ptr, uint64_t* uses) {
   return impl_->lease.get(static_cast<void*>(s), user, bytes, ptr, uses);
+}
+bool WorkspaceLease::get_optional(hipStream_t s, int user, size_t bytes, void** ptr, uint64_t* uses) {
+  if (stream_capturing(s) || (s != g_stream && stream_capturing(g_stream))) return false;
+  RelaxedCapture relaxed;
+  return get(s, user, bytes, ptr, uses) == TT_OK;
 }
 
 // ---------------------------------------------------------------- elementwise
@@ -462,6 +482,7 @@ int tt_malloc(void** ptr, size_t bytes) {
   // one of them goes to a caller who may use it on any stream, wait.
   if (g_blocks.wants_settle(bytes) && !stream_capturing(g_stream)) {
     rc = g_blocks.settle([] {
+      RelaxedCapture relaxed;
       const hipError_t e = hipStreamSynchronize(g_stream);
       return e == hipSuccess ? TT_OK : hip_fail(e, "hipStreamSynchronize (tt_malloc)");
     });
