@@ -334,7 +334,9 @@ int tt_col2im(int dtype, const void* col, void* im, int64_t N, int C, int H, int
  * weight[Cout][C][kh][kw] gives out[N][Cout][OH][OW]; the backward writes
  * grad_in (every element) and grad_weight.  The products gather their
  * operands from the images (no column matrix) and split long sums over
- * workgroups like tt_gemm_*, through the same per-stream workspace. */
+ * workgroups like tt_gemm_*, through the same per-stream workspace.  As with
+ * im2col and col2im, an infinite or NaN weight shows in the padding's products
+ * of the forward, and in grad_in only at the pixels that its tap reads. */
 int tt_conv_forward(int dtype, const void* in, const void* weight, void* out, int64_t N, int C, int H, int W,
                     int cout, int kh, int kw, int pad_h, int pad_w, int stride_h, int stride_w, void* stream);
 int tt_conv_backward(int dtype, const void* in, const void* weight, const void* grad_out, void* grad_in,

@@ -475,23 +475,59 @@ struct GradImageSource : Gather<T, false, GradImageSource<T>> {
   }
 };
 
+// The image gradient multiplies the weights of taps that have no output pixel
+// (at the image's border) by zero, which gives NaN where such a weight is
+// infinite or NaN.  A sum that came out as NaN is formed again by this function
+// from the other taps alone: channel c at (py, px) of the padded image, of the
+// image's output gradient go; false (and no sum) where no tap is missing.  Not
+// inlined: that cost the bf16 products 3-6 % (scalar registers of the k loop).
+template <typename T>
+__device__ __attribute__((noinline)) bool conv_dx_present(const T* w, const T* go, ConvGeom g, int cout, int c, int py,
+                                                          int px, float& sum) {
+  const int ky0 = py % g.sh, oy0 = py / g.sh, kx0 = px % g.sw, ox0 = px / g.sw;  // tap ky0 + sh i reads row oy0 - i
+  const int nky = (g.kh - ky0 + g.sh - 1) / g.sh, nkx = (g.kw - kx0 + g.sw - 1) / g.sw;
+  if (oy0 < g.oh && oy0 >= nky - 1 && ox0 < g.ow && ox0 >= nkx - 1) return false;
+  const int64_t kk = (int64_t)g.kh * g.kw, P = (int64_t)g.oh * g.ow;
+  sum = 0.f;
+  for (int co = 0; co < cout; ++co) {
+    const T *wc = w + ((int64_t)co * g.C + c) * kk + ky0 * g.kw + kx0, *plane = go + co * P;
+    for (int i = max(0, oy0 - g.oh + 1); i < nky && i <= oy0; ++i)
+      for (int j = max(0, ox0 - g.ow + 1); j < nkx && j <= ox0; ++j)
+        sum = fmaf(split_load(wc + i * g.sh * g.kw + j * g.sw), split_load(plane + (oy0 - i) * g.ow + ox0 - j), sum);
+  }
+  return true;
+}
+
 // gX[n][c][y][x] for product column p = (n, pixel of the phase).
 template <typename T>
 struct PhaseEpilogue {
   T* gx;
+  const T *w, *go;
   ConvGeom g;
-  int images, z0, phases_x;
+  int cout, images, z0, phases_x;
   FastDiv pix, nx;
+  int fy, fx;
   __device__ __forceinline__ int columns() const { return images * (int)pix.d; }
   __device__ __forceinline__ void enter(int z) {
     const ConvPhase f(g, z0 + z, phases_x);
     pix = FastDiv(f.ny * f.nx), nx = FastDiv(f.nx);
-    gx += (int64_t)f.fy * g.W + f.fx;
+    fy = f.fy, fx = f.fx;
   }
-  __device__ __forceinline__ void operator()(int m, int q, float acc) const {
+  __device__ __forceinline__ T* at(int m, int n, int y, int x) const {
+    return gx + ((int64_t)n * g.C + m) * g.H * g.W + (int64_t)(fy + y * g.sh) * g.W + fx + x * g.sw;
+  }
+  __device__ __forceinline__ bool operator()(int m, int q, float acc) const {
     int p, x;
     const int n = pix.divmod(q, p), y = nx.divmod(p, x);
-    split_store(gx + ((int64_t)n * g.C + m) * g.H * g.W + (int64_t)y * g.sh * g.W + (int64_t)x * g.sw, acc);
+    split_store(at(m, n, y, x), acc);
+    return acc != acc;
+  }
+  __device__ __forceinline__ void again(int m, int q) const {
+    int p, x;
+    const int n = pix.divmod(q, p), y = nx.divmod(p, x);
+    float s;
+    if (conv_dx_present(w, go + (int64_t)n * cout * g.oh * g.ow, g, cout, m, fy + y * g.sh + g.ph, fx + x * g.sw + g.pw, s))
+      split_store(at(m, n, y, x), s);
   }
 };
 
@@ -572,8 +608,11 @@ __global__ __launch_bounds__(256) void k_conv_dx_few(const T* __restrict__ w, co
 #pragma unroll
   for (int c = 0; c < C; ++c) red[grp][c][l] = acc[c];
   __syncthreads();
-  if (grp < C && p < pixels)  // C <= 4 groups: one channel each
-    split_store(gx + (n * C + grp) * HW + q, (red[0][grp][l] + red[1][grp][l]) + (red[2][grp][l] + red[3][grp][l]));
+  if (grp < C && p < pixels) {  // C <= 4 groups: one channel each
+    float v = (red[0][grp][l] + red[1][grp][l]) + (red[2][grp][l] + red[3][grp][l]);
+    if (v != v) conv_dx_present(w, go + n * cout * P, g, cout, grp, y, x, v);
+    split_store(gx + (n * C + grp) * HW + q, v);
+  }
 }
 
 // Whether k_conv_dx_few takes the image gradient.  Measured (the whole
@@ -684,7 +723,7 @@ int conv_backward(const char* fn, const T* in, const T* w, const T* go, T* gin, 
       const int rc = launch_split_gemm<T>(
           fn, g.C, images * pixels, cout * taps, WeightSource<T>(w, g, cout, (int)z0, phases_x),
           GradImageSource<T>(go + n * cout * P, g, cout, (int)images, (int)z0, phases_x),
-          PhaseEpilogue<T>{gin + n * g.C * HW, g, (int)images, (int)z0, phases_x}, s,
+          PhaseEpilogue<T>{gin + n * g.C * HW, w, go + n * cout * P, g, cout, (int)images, (int)z0, phases_x}, s,
           (int)std::min<int64_t>(kConvPhases, phases - z0));
       if (rc) return rc;
     }

@@ -25,6 +25,8 @@
 // A phased product (SB::kPhased) is several products in one launch: enter(z)
 // of the sources and the epilogue sets them up for product z, whose N and K
 // are then B.Q and B.K (M is common).  blockIdx.z = phase * nsplit + split.
+// Its epilogue returns whether an output has to be formed again, which
+// again(m, n) does (rare, so that one loop behind the stores is enough).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -215,7 +217,6 @@ __global__ __launch_bounds__(256) void k_split_gemm(int M, int N, int K, int nsp
     split = blockIdx.z - phase * nsplit;
     A.enter(phase);
     B.enter(phase);
-    ep.enter(phase);
     N = B.Q;
     K = B.K;
     if (n0 >= N) return;  // uniform: the grid covers the largest phase
@@ -259,15 +260,21 @@ __global__ __launch_bounds__(256) void k_split_gemm(int M, int N, int K, int nsp
   }
   const int n = n0 + wn + (l & 31);
   if (n >= N) return;
+  if constexpr (SB::kPhased) ep.enter(blockIdx.z / nsplit);  // here: its values need no registers during the loop
+  unsigned again = 0;  // bit r: output r
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int m = m0 + wm + acc_row(r, l >> 5);
     if (m >= M) continue;
     if (part)
       part[(int64_t)m * pitch + n] = acc[r];
+    else if constexpr (SB::kPhased)
+      again |= (unsigned)ep(m, n, acc[r]) << r;
     else
       ep(m, n, acc[r]);
   }
+  if constexpr (SB::kPhased)
+    for (; again; again &= again - 1) ep.again(m0 + wm + acc_row(__ffs(again) - 1, l >> 5), n);
 }
 
 // Adds the splits' sums in a fixed order and runs the epilogue, phase by
@@ -301,7 +308,12 @@ __global__ __launch_bounds__(64 * (G < 4 ? 4 : G)) void k_split_reduce(const flo
 #pragma unroll
     for (int k = 1; k < G; ++k) s += red[w + k][l];
   }
-  if (in) ep(m, n, s);
+  if (!in) return;
+  if constexpr (PHASED) {
+    if (ep(m, n, s)) ep.again(m, n);
+  } else {
+    ep(m, n, s);
+  }
 }
 
 // Splits of the contraction for a grid of `tiles` tiles and nk BK-steps: to

@@ -89,3 +89,35 @@ def test_conv_products(dt, case):
         e = orc.max_rel_err(a, r)
         print(f"  {name} {e:.2e}", flush=True)
         assert e <= TOL[dt], (name, e)
+
+
+@pytest.mark.parametrize("dt", ["float", "bf16"])
+@pytest.mark.parametrize("case", [(2, 1, 9, 7, 8, 5, 5, 2, 2, 1, 1), (1, 4, 6, 9, 24, 4, 4, 1, 2, 1, 1),  # a lane per pixel
+                                  (2, 6, 9, 7, 8, 5, 5, 2, 2, 1, 1), (2, 3, 11, 13, 6, 5, 5, 2, 2, 2, 2),  # products: one split,
+                                  (1, 200, 7, 7, 40, 3, 3, 1, 1, 1, 1), (1, 40, 14, 14, 200, 3, 3, 1, 1, 2, 2),  # several
+                                  (2, 3, 16, 12, 5, 4, 3, 1, 0, 4, 3)], ids=str)  # windows that do not overlap
+def test_image_gradient_of_non_finite_weights(dt, case):
+    """An infinite or NaN weight reaches the pixels its tap has an output pixel for, and no other."""
+    import myLayer as ml
+    import myTensor as mt
+
+    T = getattr(mt, "Tensor_" + dt)
+    N, C, H, W, Co, kh, kw, ph, pw, sh, sw = case
+    rng = np.random.default_rng(sum(case))
+    oh, ow = (H + 2 * ph - kh) // sh + 1, (W + 2 * pw - kw) // sw + 1
+    x, w, go = (rng.standard_normal(s).astype(np.float32) for s in ((N, C, H, W), (Co, C, kh, kw), (N, Co, oh, ow)))
+    w[0, 0, 0, 0], w[1, C - 1, kh - 1, kw - 1], w[2, C - 1, 0, kw - 1] = np.inf, np.nan, -np.inf
+    if dt == "bf16":
+        x, w, go = orc.bf16_round(x), orc.bf16_round(w), orc.bf16_round(go)
+    X, Wt, GO = (T(a, "gpu") for a in (x, w, go))
+    out, gx, gw = (T([1], "gpu") for _ in range(3))
+    ml.ConvBackward(X, out, Wt, gx, GO, gw, ph, pw, sh, sw)
+    with np.errstate(invalid="ignore"):
+        ref = _ref(x.astype(np.float64), w.astype(np.float64), go.astype(np.float64), ph, pw, sh, sw)[2]
+    got = np.asarray(gx.numpy()).reshape(ref.shape)
+    fin = np.isfinite(ref)
+    assert fin.any() and not fin.all()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    np.testing.assert_array_equal(got[inf], ref[inf])
+    assert np.abs(got[fin] - ref[fin]).max() <= TOL[dt] * np.abs(ref[fin]).max()
