@@ -732,7 +732,9 @@ int conv_backward(const char* fn, const T* in, const T* w, const T* go, T* gin, 
 }
 
 // Clamps strides to the padded extent (a longer one also leaves one output)
-// and returns whether the products' 32-bit indices and grids cover the shape.
+// and returns whether the products' 32-bit indices and grids cover the shape
+// (their rows: cout forward and for dW; C, or C kh kw under windows that do not
+// overlap, for dX).
 bool conv_fits(ConvGeom& g, int cout) {
   const int64_t lim = int64_t(1) << 30, kk = (int64_t)g.kh * g.kw, P = (int64_t)g.oh * g.ow;
   const int64_t eh = (int64_t)g.H + 2 * (int64_t)g.ph, ew = (int64_t)g.W + 2 * (int64_t)g.pw;
@@ -740,6 +742,8 @@ bool conv_fits(ConvGeom& g, int cout) {
   if (eh >= lim / 2 || ew >= lim / 2 || P > lim || (int64_t)g.H * g.W > lim || kk > lim || g.C * ((int64_t)g.H * g.W) > lim ||
       cout * P > lim || g.C * kk > lim || cout * (g.C * kk) > lim)
     return false;
+  const bool apart = g.sh >= g.kh && g.sw >= g.kw;
+  if (std::max<int64_t>(cout, apart ? g.C * kk : g.C) > split_max_rows(64)) return false;
   g.sh = std::min(g.sh, (int)eh + 1);
   g.sw = std::min(g.sw, (int)ew + 1);
   return true;
@@ -767,7 +771,7 @@ extern "C" int tt_conv_forward(int dtype, const void* in, const void* weight, vo
   if (dtype != TT_F32 && dtype != TT_BF16) return fail(TT_ERR_ARG, std::string(fn) + ": dtype must be TT_F32 or TT_BF16");
   if (N == 0 || cout == 0) return ok();
   if (!in || !weight || !out) return fail(TT_ERR_ARG, std::string(fn) + ": null pointer");
-  if (!conv_fits(g, cout)) return fail(TT_ERR_UNSUPPORTED, std::string(fn) + ": one image, its output or the weights above 2^30 elements, or an axis above 2^29");
+  if (!conv_fits(g, cout)) return fail(TT_ERR_UNSUPPORTED, std::string(fn) + ": one image, its output or the weights above 2^30 elements, an axis above 2^29 or the channels above 65535 * 64");
   if ((rc = ensure_init())) return rc;
   hipStream_t s = stream_or_default(stream);
   if (dtype == TT_F32) return conv_forward(fn, (const float*)in, (const float*)weight, (float*)out, N, cout, g, s);
@@ -785,7 +789,7 @@ extern "C" int tt_conv_backward(int dtype, const void* in, const void* weight, c
   if (dtype != TT_F32 && dtype != TT_BF16) return fail(TT_ERR_ARG, std::string(fn) + ": dtype must be TT_F32 or TT_BF16");
   if (!in || !weight || !grad_out || !grad_in || !grad_weight)
     return fail(TT_ERR_ARG, std::string(fn) + ": null pointer");
-  if (!conv_fits(g, cout)) return fail(TT_ERR_UNSUPPORTED, std::string(fn) + ": one image, its output or the weights above 2^30 elements, or an axis above 2^29");
+  if (!conv_fits(g, cout)) return fail(TT_ERR_UNSUPPORTED, std::string(fn) + ": one image, its output or the weights above 2^30 elements, an axis above 2^29 or the channels (times the kernel under separate windows) above 65535 * 64");
   if ((rc = ensure_init())) return rc;
   hipStream_t s = stream_or_default(stream);
   if (dtype == TT_F32)

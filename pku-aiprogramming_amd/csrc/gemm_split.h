@@ -328,6 +328,10 @@ inline int split_count(int64_t tiles, int64_t nk) {
   return s < 1 ? 1 : (int)s;
 }
 
+// Rows that a launch takes: the grid's y extent is 16 bits.  (Splits and phases
+// share z: with more than one split there are fewer than 768 of both.)
+constexpr int64_t split_max_rows(int tm) { return int64_t(65535) * tm; }
+
 // Scratch of one split product: nsplit x M x N floats, at most
 // kSplitWorkBytes (with more than one split, nsplit x tiles is below 768; a
 // tile is 16 KB).  One fixed size per stream, so the buffer is allocated once.
@@ -345,7 +349,7 @@ int launch_split_tiles(const char* fn, int64_t M, int64_t N, int64_t K, int phas
   const int64_t gx = (N + TN - 1) / TN, gy = (M + TM - 1) / TM;
   const int64_t nk = (K + BK - 1) / BK;
   int nsplit = split_count(gx * gy * phases, nk);
-  if (!grid_fits(gx, 256) || gy > 65535 || (int64_t)phases * nsplit > 65535)
+  if (!grid_fits(gx, 256) || M > split_max_rows(TM) || (int64_t)phases * nsplit > 65535)
     return fail(TT_ERR_ARG, std::string(fn) + ": too large");
   float* part = nullptr;
   std::optional<WorkspaceLease> ws;  // held until the reduction is queued

@@ -121,3 +121,31 @@ def test_image_gradient_of_non_finite_weights(dt, case):
     inf = np.isinf(ref)
     np.testing.assert_array_equal(got[inf], ref[inf])
     assert np.abs(got[fin] - ref[fin]).max() <= TOL[dt] * np.abs(ref[fin]).max()
+
+
+@pytest.mark.parametrize("case", [(1, 3, 1200, 1200, 1, 1200, 1200, 0, 0, 1200, 1200),  # C kh kw rows, windows apart
+                                  (1, 1, 1, 1, 4194304, 1, 1, 0, 0, 1, 1),  # output channels
+                                  (1, 4194304, 1, 1, 1, 2, 1, 1, 0, 1, 1)],  # input channels
+                         ids=["kernel", "out_channels", "in_channels"])
+def test_rows_beyond_the_grid(case):
+    """More rows than 65535 tiles of 64: the layer takes the column matrix."""
+    import myLayer as ml
+    import myTensor as mt
+
+    N, C, H, W, Co, kh, kw, ph, pw, sh, sw = case
+    rng = np.random.default_rng(Co + kh)
+    oh, ow = (H + 2 * ph - kh) // sh + 1, (W + 2 * pw - kw) // sw + 1
+    x, w, go = (rng.standard_normal(s).astype(np.float32) for s in ((N, C, H, W), (Co, C, kh, kw), (N, Co, oh, ow)))
+    X, Wt, GO = (mt.Tensor_float(a, "gpu") for a in (x, w, go))
+    out, gx, gw = (mt.Tensor_float([1], "gpu") for _ in range(3))
+    ml.ConvForward(X, out, Wt, ph, pw, sh, sw)
+    ml.ConvBackward(X, out, Wt, gx, GO, gw, ph, pw, sh, sw)
+    if oh * ow == 1 and Co == 1:  # one window: the kernel's sums are single products
+        refs = ((x * w).sum(dtype=np.float64), go.item() * x, go.item() * w)
+    else:
+        refs = _ref(x.astype(np.float64), w.astype(np.float64), go.astype(np.float64), ph, pw, sh, sw)
+    for name, got, r in zip(("out", "grad_weight", "grad_input"), (out, gw, gx), refs):
+        r = np.asarray(r, np.float64)
+        e = orc.max_rel_err(np.asarray(got.numpy()).reshape(r.size), r.ravel())
+        print(f"  {name} {e:.2e}", flush=True)
+        assert e <= TOL["float"], (name, e)
