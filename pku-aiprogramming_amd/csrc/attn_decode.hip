@@ -335,6 +335,10 @@ __global__ __launch_bounds__(NT) void attn_decode_combine_kernel(const float* __
 }
 
 constexpr int64_t kDecShortBytes = int64_t(56) << 20;
+// Scratch of the short splits' partials, of one size so that it is allocated
+// once per stream: 4064 of them at d = 128.  The rule below makes at most
+// 56 MB / 32 KB (a split's keys) and one more for each of fewer than 1792 heads.
+constexpr size_t kDecShortWork = size_t(2) << 20;
 
 template <typename T, int D>
 static int launch_decode(const T* q, const T* k, const T* v, T* o, float* lse, int64_t BH, int64_t Lkv,
@@ -374,17 +378,15 @@ static int launch_decode(const T* q, const T* k, const T* v, T* o, float* lse, i
   const float sl2 = scale * kLog2e;
   void* ws = nullptr;
   std::optional<WorkspaceLease> lease;  // held until both kernels are launched
-  if (nsplit > 1) {
-    // A head that one long split covers runs without scratch where none may be
-    // allocated (a stream under capture, a refused allocation).
-    int rc = long_splits == 1 && stream_capturing(st)
-                 ? TT_ERR_NOMEM
-                 : lease.emplace().get(st, kWsDecodePartials, (size_t)(BH * nsplit) * (D + 1) * sizeof(float), &ws);
-    if (rc && long_splits > 1) return rc;
-    if (rc) {
-      is_short = false;
-      nsplit = 1;
-    }
+  auto partials = [&](int64_t n) { return (size_t)(BH * n) * (D + 1) * sizeof(float); };
+  if (is_short && short_splits > 1 &&
+      (partials(short_splits) > kDecShortWork || !lease.emplace().get_fixed(st, kWsDecodeShort, kDecShortWork, &ws))) {
+    is_short = false;  // no scratch for them: long splits
+    nsplit = long_splits;
+  }
+  if (!is_short && nsplit > 1) {
+    const int rc = lease.emplace().get(st, kWsDecodePartials, partials(nsplit), &ws);
+    if (rc) return rc;
   }
   const dim3 grid((unsigned)(nsplit * BH)), block(DEC_THREADS);
   if (nsplit == 1) {  // one split per head: no partials, no combine

@@ -253,6 +253,12 @@ class WorkspaceCache {
     int get(void* stream, int user, size_t bytes, void** ptr, uint64_t* uses = nullptr) {
       return c_.get_locked(stream, user, bytes, ptr, uses);
     }
+    // The same only where the buffer is there already.
+    bool get_held(void* stream, int user, size_t bytes, void** ptr) {
+      auto it = c_.slots_.find({stream, user});
+      if (it == c_.slots_.end() || it->second.bytes < bytes) return false;
+      return c_.get_locked(stream, user, bytes, ptr, nullptr) == 0;
+    }
 
    private:
     WorkspaceCache& c_;

@@ -46,7 +46,7 @@ void* noalloc_scratch(size_t* bytes);
 // grown on demand and kept for reuse.  A lease holds the workspace lock from
 // get() until it is destroyed: keep it alive until every kernel that reads
 // the buffer has been launched on that stream.
-enum { kWsBackwardRows = 0, kWsDecodePartials = 1, kWsForwardSplits = 2, kWsSoftmaxPartials = 3, kWsGemmSplits = 4 };
+enum { kWsBackwardRows = 0, kWsDecodePartials = 1, kWsForwardSplits = 2, kWsSoftmaxPartials = 3, kWsGemmSplits = 4, kWsDecodeShort = 5 };
 class WorkspaceLease {
  public:
   WorkspaceLease();
@@ -62,6 +62,10 @@ class WorkspaceLease {
   // buffer would order the stream behind).  Leaves captures of other streams
   // alone: an allocation of this thread would end them otherwise.
   bool get_optional(hipStream_t stream, int user, size_t bytes, void** ptr, uint64_t* uses = nullptr);
+  // The same for a user whose requests are all of one size: its buffer is never
+  // replaced, so a graph may keep the address, and a stream under capture gets
+  // the one that an earlier call left.
+  bool get_fixed(hipStream_t stream, int user, size_t bytes, void** ptr);
 
  private:
   struct Impl;

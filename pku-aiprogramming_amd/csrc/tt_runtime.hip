@@ -172,6 +172,9 @@ bool WorkspaceLease::get_optional(hipStream_t s, int user, size_t bytes, void** 
   RelaxedCapture relaxed;
   return get(s, user, bytes, ptr, uses) == TT_OK;
 }
+bool WorkspaceLease::get_fixed(hipStream_t s, int user, size_t bytes, void** ptr) {
+  return impl_->lease.get_held(static_cast<void*>(s), user, bytes, ptr) || get_optional(s, user, bytes, ptr);
+}
 
 // ---------------------------------------------------------------- elementwise
 __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {

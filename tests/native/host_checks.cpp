@@ -101,6 +101,10 @@ static void workspace_checks() {
     CHECK(l.get(&s1, 0, 64, &q, &uses) == 0 && q == p && uses == 1);  // fits: same buffer, no sync, no new ordering
     CHECK(l.get(&s1, 0, 100, &q, &uses) == 0 && q == p && uses == 2);
     CHECK(be.orders == 1);
+    // get_held: what is there, never a new or larger buffer
+    CHECK(l.get_held(&s1, 0, 100, &q) && q == p && l.get_held(&s1, 0, 1, &q) && q == p);
+    CHECK(!l.get_held(&s1, 0, 101, &q) && !l.get_held(&s1, 1, 1, &q) && !l.get_held(&s2, 0, 1, &q));
+    CHECK(be.orders == 1 && be.allocs == 1);
     CHECK(l.get(&s2, 0, 64, &r) == 0 && r != p);  // another stream: its own buffer
     CHECK(be.orders == 2 && be.last_ordered == (void*)&s2);
   }
