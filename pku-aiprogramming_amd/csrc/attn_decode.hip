@@ -364,12 +364,16 @@ static int launch_decode(const T* q, const T* k, const T* v, T* o, float* lse, i
   // 27.6 (1024, 67 MB), [64,32] x 1024 160 / 175 against 1024-key splits; fp32 d = 64
   // [16,16] x 700 16.2 / 16.5 (768), d = 32 [40,16] x 500 13.5 / 14.6 (more
   // cross-lane steps per byte than bf16).  Nor where a head's last short split
-  // is mostly empty (bf16 d = 32 [16,32] x 513 10.7 / 11.8), or two replace one
-  // long split, no merge, of many heads (d = 128 [30,32] x 129 12.3 / 17.5).
+  // is mostly empty (bf16 d = 32 [16,32] x 513 10.7 / 11.8; one split at most half
+  // full of many heads, d = 32 1520 x 200 8.6 / 9.0, 2040 x 128 9.1 / 9.8, d = 64 2040 x
+  // 128 11.1 / 11.8, but 1200 x 128 7.3 / 7.0 and 8.4 / 7.8, and d = 128 1520 x 64 9.6 /
+  // 9.6), or two replace one long split, no merge, of many heads (d = 128 [30,32] x
+  // 129 12.3 / 17.5).
   const int64_t kbytes = BH * Lkv * D * (int64_t)sizeof(T);
   bool is_short = chunk == 256 && (sizeof(T) == 2 ? splits(256) < 1024 || kbytes < kDecShortBytes : splits(256) < 640);
   const int64_t short_splits = (Lkv + dec_short_chunk<T, D>() - 1) / dec_short_chunk<T, D>();
   if (Lkv <= 256 && short_splits > 1 && BH >= 256) is_short = false;
+  if (D < 128 && 2 * Lkv <= dec_short_chunk<T, D>() && BH >= 1300) is_short = false;
   if (short_splits > 1 && BH >= 64 && 10 * Lkv < 6 * short_splits * dec_short_chunk<T, D>()) is_short = false;
   if (Lkv < chunk) chunk = (int)((Lkv + 63) / 64 * 64);
   const int64_t long_splits = (Lkv + chunk - 1) / chunk;

@@ -51,6 +51,16 @@ def test_short_splits(capi, dt, d, chunks):
     assert orc.max_rel_err(lse.reshape(np.shape(rl)), rl) <= 1e-5  # fp32 weights and sums
 
 
+@pytest.mark.parametrize("BH,L,d", [(1299, 256, 32), (1300, 256, 32), (1300, 257, 32), (1300, 128, 64), (1300, 129, 64)])
+def test_one_split_of_many_heads(capi, BH, L, d):
+    """Both sides of the rule that leaves them to the long split's kernel."""
+    q, k, v = _inputs("bf16", 1, BH, L, d, BH + L)
+    o, lse = _run(capi, "bf16", q, k, v)
+    ro, rl = orc.attn_decode_f64(q, k, v, 0.125)
+    assert orc.max_rel_err(o, ro) <= orc.TOL["bf16"]
+    assert orc.max_rel_err(lse.reshape(np.shape(rl)), rl) <= 1e-5
+
+
 def test_split_without_finite_scores(capi):
     q, k, v = _inputs("f32", 1, 2, 1000, 64, 1)
     q[..., 0] = 1.0
