@@ -742,7 +742,7 @@ static int fwd_bf16(const u16* q, const u16* k, const u16* v, u16* o, float* lse
   float* part = nullptr;
   std::optional<WorkspaceLease> lease;  // held until both kernels are launched
   if (nsplit > 1 && lease.emplace().get_optional(
-                        st, kWsForwardSplits, (size_t)(nsplit * BH * Lq) * (D + 2) * sizeof(float), (void**)&part)) {
+                        st, kWsForwardSplitsBf16, (size_t)(nsplit * BH * Lq) * (D + 2) * sizeof(float), (void**)&part)) {
     // two key groups per workgroup at d = 128 (below: [1,32] 256 x 4096 31.8 ->
     // 29.5 us), one at d <= 64 (two: [2,16] 77 x 4099 14.9 -> 15.5, [2,8] 333 x 2000
     // d = 32 14.0 -> 17.3)

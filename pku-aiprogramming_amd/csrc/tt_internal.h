@@ -45,8 +45,10 @@ void* noalloc_scratch(size_t* bytes);
 // Device scratch of the attention launchers: one buffer per (stream, user),
 // grown on demand and kept for reuse.  A lease holds the workspace lock from
 // get() until it is destroyed: keep it alive until every kernel that reads
-// the buffer has been launched on that stream.
-enum { kWsBackwardRows = 0, kWsDecodePartials = 1, kWsForwardSplits = 2, kWsSoftmaxPartials = 3, kWsGemmSplits = 4, kWsDecodeShort = 5 };
+// the buffer has been launched on that stream.  A user that also runs under
+// capture (the fp32 forward, the backward, the long decode splits) shares its
+// buffer with no other: their requests would replace the one a graph keeps.
+enum { kWsBackwardRows = 0, kWsDecodePartials = 1, kWsForwardSplits = 2, kWsSoftmaxPartials = 3, kWsGemmSplits = 4, kWsDecodeShort = 5, kWsForwardSplitsBf16 = 6 };
 class WorkspaceLease {
  public:
   WorkspaceLease();

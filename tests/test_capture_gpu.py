@@ -189,3 +189,32 @@ def test_malloc_of_a_freed_tensors_block_beside_a_capture(capi, mode):
         L.check(L.lib.tt_malloc(C.byref(p), 4 * n), "tt_malloc")
     L.call("tt_free", p)
     c.destroy()
+
+
+def test_captured_fp32_forward_keeps_its_scratch(capi):
+    """The key splits of a later, larger bf16 forward on the stream take another buffer."""
+    st = capi.Stream()
+
+    def fwd(dt, Lq, Lk):
+        x = [orc.bf16_round(np.random.default_rng(Lk).standard_normal((1, 2, n, 64)).astype(np.float32))
+             for n in (Lq, Lk, Lk)]
+        b = [capi.DeviceBuffer.from_numpy(a, dt) for a in x] + [capi.DeviceBuffer((1, 2, Lq, 64), dt)]
+        return b, orc.attn_fwd_f64(*x, 0.125, False)[0]
+
+    f32, ref = fwd("f32", 100, 300)
+    capi.attn_fwd(*f32, None, 0.125, False, stream=st.handle)  # leaves the scratch on the stream
+    st.sync()
+    with Capture(capi, st.handle) as c:
+        capi.attn_fwd(*f32, None, 0.125, False, stream=st.handle)
+    held = []
+    for Lk in (2000, 8000):
+        b16, ref16 = fwd("bf16", 200, Lk)
+        capi.attn_fwd(*b16, None, 0.125, False, stream=st.handle)
+        held += [capi.DeviceBuffer((n,), "f32") for n in (100000, 400000, 1600000)]  # what a replaced buffer would become
+        for h in held:
+            h.zero()
+        c.launch()
+        assert orc.max_rel_err(f32[3].download(), ref) <= orc.TOL["f32"]
+        assert orc.max_rel_err(b16[3].download(), ref16) <= orc.TOL["bf16"]
+        assert not any(h.download().any() for h in held)
+    c.destroy()
