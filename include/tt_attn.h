@@ -176,6 +176,8 @@ int tt_elementwise(int op, int dtype, void* c, const void* a, const void* b, int
  * generator (SplitMix64 of (seed, index) -> Box-Muller).  Synthetic benchmark
  * data only; not part of the reference. */
 int tt_fill_normal(int dtype, void* dst, int64_t n, uint64_t seed, float scale, void* stream);
+/* dst[i] = src[i] rounded to bf16, nearest even (NaN stays NaN). */
+int tt_round_bf16(const float* src, uint16_t* dst, int64_t n, void* stream);
 
 /* ------------------------------------------------------------- attention */
 
@@ -301,6 +303,9 @@ int tt_gemm_f32(int transa, int transb, int64_t m, int64_t n, int64_t k, float a
                 const float* A, const float* B, float beta, float* C, void* stream);
 int tt_gemm_bf16(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha,
                  const uint16_t* A, const uint16_t* B, float beta, uint16_t* C, void* stream);
+/* bf16 A and B, C in fp32 (not rounded): for results that are summed further. */
+int tt_gemm_bf16_f32(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha,
+                     const uint16_t* A, const uint16_t* B, float beta, float* C, void* stream);
 
 /* The fully connected layer on that GEMM: out[batch x fout] = in[batch x fin]
  * weight[fin x fout] + bias, the bias added to the fp32 sum before the store

@@ -164,9 +164,9 @@ __device__ __forceinline__ auto operand(const T* s, int rbase, int ks) {
   }
 }
 
-template <typename T, bool TA, bool TB>
+template <typename T, bool TA, bool TB, class EP>
 __global__ __launch_bounds__(256, 2) void k_gemm(int M, int N, int K, const T* __restrict__ A, int64_t lda,
-                                                const T* __restrict__ B, int64_t ldb, MatrixEpilogue<T> ep) {
+                                                const T* __restrict__ B, int64_t ldb, EP ep) {
   using G = GemmT<T>;
   constexpr int GN = G::GN, NB = GN / 64;  // MFMA blocks per wave along n
   constexpr int BK = G::BK, KS = sizeof(T) == 2 ? BK / 16 : BK / 2;  // MFMA k-steps per BK
@@ -304,9 +304,9 @@ __device__ __forceinline__ bf16x8 dma_operand(const u16* s, int rbase, int ks) {
   }
 }
 
-template <bool TA, bool TB>
+template <bool TA, bool TB, class EP>
 __global__ __launch_bounds__(256, 3) void k_gemm_dma(int M, int N, int K, const u16* __restrict__ A, int64_t lda,
-                                                    const u16* __restrict__ B, int64_t ldb, MatrixEpilogue<u16> ep) {
+                                                    const u16* __restrict__ B, int64_t ldb, EP ep) {
   constexpr int GN = kDmaGN, NB = GN / 64, BK = 32, KS = BK / 16, S = kDmaStages;
   using TileA = DmaTile<GM, !TA>;
   using TileB = DmaTile<GN, TB>;
@@ -390,9 +390,10 @@ bool use_split_tiles(int64_t m, int64_t n, int64_t k, bool dma) {
   return 10 * tiles < 8 * 512 * rounds && tiles < 8192;
 }
 
-template <typename T>
+// O: the type of C and the bias.
+template <typename T, typename O>
 int gemm_launch(const char* fn, int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha, const T* A,
-                const T* B, float beta, T* C, const T* bias, int64_t bias_step, void* stream) {
+                const T* B, float beta, O* C, const O* bias, int64_t bias_step, void* stream) {
   if (m < 0 || n < 0 || k < 0) return fail(TT_ERR_ARG, std::string(fn) + ": negative size");
   if (transa != 0 && transa != 1) return fail(TT_ERR_ARG, std::string(fn) + ": transa must be 0 or 1");
   if (transb != 0 && transb != 1) return fail(TT_ERR_ARG, std::string(fn) + ": transb must be 0 or 1");
@@ -408,7 +409,8 @@ int gemm_launch(const char* fn, int transa, int transb, int64_t m, int64_t n, in
   if (rc) return rc;
   hipStream_t s = stream_or_default(stream);
   const int64_t lda = transa ? m : k, ldb = transb ? k : n;
-  const MatrixEpilogue<T> ep{C, bias, bias_step, alpha, beta, (int)n};
+  using EP = MatrixEpilogue<O>;
+  const EP ep{C, bias, bias_step, alpha, beta, (int)n};
   // direct-to-LDS kernel: k in whole steps, aligned rows (m, n multiples of 8
   // where they are the contiguous axis), every per-lane tile offset within 32
   // bits
@@ -431,7 +433,7 @@ int gemm_launch(const char* fn, int transa, int transb, int64_t m, int64_t n, in
     if (dma) {
       const dim3 g2((unsigned)((n + kDmaGN - 1) / kDmaGN), (unsigned)gy);
 #define TT_GEMM_D(TA, TB) \
-  hipLaunchKernelGGL((k_gemm_dma<TA, TB>), g2, dim3(256), 0, s, (int)m, (int)n, (int)k, A, lda, B, ldb, ep)
+  hipLaunchKernelGGL((k_gemm_dma<TA, TB, EP>), g2, dim3(256), 0, s, (int)m, (int)n, (int)k, A, lda, B, ldb, ep)
       switch (transa * 2 + transb) {
         case 0: TT_GEMM_D(false, false); break;
         case 1: TT_GEMM_D(false, true); break;
@@ -444,7 +446,7 @@ int gemm_launch(const char* fn, int transa, int transb, int64_t m, int64_t n, in
     }
   }
 #define TT_GEMM(TA, TB) \
-  hipLaunchKernelGGL((k_gemm<T, TA, TB>), grid, block, 0, s, (int)m, (int)n, (int)k, A, lda, B, ldb, ep)
+  hipLaunchKernelGGL((k_gemm<T, TA, TB, EP>), grid, block, 0, s, (int)m, (int)n, (int)k, A, lda, B, ldb, ep)
   switch (transa * 2 + transb) {
     case 0: TT_GEMM(false, false); break;
     case 1: TT_GEMM(false, true); break;
@@ -533,10 +535,10 @@ extern "C" int tt_fc_forward(int dtype, int64_t batch, int64_t fin, int64_t fout
   if (batch > 0 && fout > 0 && !bias) return fail(TT_ERR_ARG, std::string(fn) + ": null pointer");
   const int64_t step = bias_scalar ? 0 : 1;
   if (dtype == TT_F32)
-    return gemm_launch<float>(fn, 0, 0, batch, fout, fin, 1.f, (const float*)in, (const float*)weight, 0.f,
+    return gemm_launch<float, float>(fn, 0, 0, batch, fout, fin, 1.f, (const float*)in, (const float*)weight, 0.f,
                               (float*)out, (const float*)bias, step, stream);
   if (dtype == TT_BF16)
-    return gemm_launch<u16>(fn, 0, 0, batch, fout, fin, 1.f, (const u16*)in, (const u16*)weight, 0.f, (u16*)out,
+    return gemm_launch<u16, u16>(fn, 0, 0, batch, fout, fin, 1.f, (const u16*)in, (const u16*)weight, 0.f, (u16*)out,
                             (const u16*)bias, step, stream);
   return fail(TT_ERR_ARG, std::string(fn) + ": dtype must be TT_F32 or TT_BF16");
 }
@@ -556,10 +558,15 @@ extern "C" int tt_col_sum(int dtype, const void* x, void* y, int64_t rows, int64
 
 extern "C" int tt_gemm_f32(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha, const float* A,
                            const float* B, float beta, float* C, void* stream) {
-  return gemm_launch<float>("tt_gemm_f32", transa, transb, m, n, k, alpha, A, B, beta, C, nullptr, 0, stream);
+  return gemm_launch<float, float>("tt_gemm_f32", transa, transb, m, n, k, alpha, A, B, beta, C, nullptr, 0, stream);
 }
 
 extern "C" int tt_gemm_bf16(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha, const uint16_t* A,
                             const uint16_t* B, float beta, uint16_t* C, void* stream) {
-  return gemm_launch<u16>("tt_gemm_bf16", transa, transb, m, n, k, alpha, A, B, beta, C, nullptr, 0, stream);
+  return gemm_launch<u16, u16>("tt_gemm_bf16", transa, transb, m, n, k, alpha, A, B, beta, C, nullptr, 0, stream);
+}
+
+extern "C" int tt_gemm_bf16_f32(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha,
+                                const uint16_t* A, const uint16_t* B, float beta, float* C, void* stream) {
+  return gemm_launch<u16, float>("tt_gemm_bf16_f32", transa, transb, m, n, k, alpha, A, B, beta, C, nullptr, 0, stream);
 }

@@ -7,6 +7,7 @@
 // perceptron's step ran 360 us, now 170.
 #include "layers.h"
 
+#include <algorithm>
 #include <initializer_list>
 #include <stdexcept>
 #include <string>
@@ -183,6 +184,24 @@ void gemm(const char* fn, bool ta, bool tb, int64_t m, int64_t n, int64_t k, flo
     rc = tt_gemm_bf16(ta ? 1 : 0, tb ? 1 : 0, m, n, k, alpha, reinterpret_cast<const uint16_t*>(A),
                       reinterpret_cast<const uint16_t*>(B), beta, reinterpret_cast<uint16_t*>(C), nullptr);
   tt_check(rc, fn);
+}
+
+// C = op(A) op(B) + beta C with C in fp32 whatever T is.
+template <typename T>
+void gemm_to_f32(const char* fn, bool ta, bool tb, int64_t m, int64_t n, int64_t k, const T* A, const T* B, float beta,
+                 float* C) {
+  int rc;
+  if constexpr (std::is_same<T, float>::value)
+    rc = tt_gemm_f32(ta ? 1 : 0, tb ? 1 : 0, m, n, k, 1.f, A, B, beta, C, nullptr);
+  else
+    rc = tt_gemm_bf16_f32(ta ? 1 : 0, tb ? 1 : 0, m, n, k, 1.f, reinterpret_cast<const uint16_t*>(A),
+                          reinterpret_cast<const uint16_t*>(B), beta, C, nullptr);
+  tt_check(rc, fn);
+}
+
+template <typename T>
+void to_bf16(const char* fn, const float* src, T* dst, int64_t n) {
+  tt_check(tt_round_bf16(src, reinterpret_cast<uint16_t*>(dst), n, nullptr), fn);
 }
 
 struct FcDims {
@@ -385,6 +404,98 @@ ConvDims conv_dims(const std::string& fn, const TinyTensor<T>& input, const Tiny
   return d;
 }
 
+// A device block of the library stream; p is null where it was refused.
+struct Scratch {
+  void* p = nullptr;
+  explicit Scratch(size_t bytes) { (void)tt_malloc_ordered(&p, bytes); }
+  ~Scratch() { (void)tt_free_ordered(p); }
+  Scratch(const Scratch&) = delete;
+  Scratch& operator=(const Scratch&) = delete;
+};
+
+// The column-matrix convolution: im2col, one product per image, col2im, a few
+// images' columns at a time.  Sums over images and over an image's taps stay
+// in fp32.  False where its scratch is refused (nothing is written then).
+constexpr int64_t kColumnBytes = int64_t(64) << 20;  // of columns at a time, or one image's
+
+template <typename T>
+bool conv_forward_columns(const std::string& fn, const T* in, const T* w, T* out, const ConvDims& d, int ph, int pw,
+                          int sh, int sw) {
+  const int64_t P = d.P(), K = d.K(), image = (int64_t)d.in.C * d.in.H * d.in.W;
+  const int64_t slab = std::min(d.in.batch, std::max<int64_t>(1, kColumnBytes / (P * K * (int64_t)sizeof(T))));
+  Scratch scratch((size_t)(slab * P * K) * sizeof(T));
+  if (!scratch.p) return false;
+  T* col = static_cast<T*>(scratch.p);
+  for (int64_t n = 0; n < d.in.batch; n += slab) {
+    const ConvShape s{std::min(slab, d.in.batch - n), d.in.C, d.in.H, d.in.W};
+    im2col_call(fn, in + n * image, col, s, d.kh, d.kw, ph, pw, sh, sw);
+    for (int64_t i = 0; i < s.batch; ++i)
+      gemm<T>(fn.c_str(), false, true, d.cout, P, K, 1.f, w, col + i * P * K, 0.f, out + (n + i) * d.cout * P);
+  }
+  return true;
+}
+
+template <typename T>
+bool conv_backward_columns(const std::string& fn, const T* in, const T* w, const T* go, T* gin, T* gw,
+                           const ConvDims& d, int ph, int pw, int sh, int sw) {
+  constexpr bool F32 = std::is_same<T, float>::value;
+  const int64_t P = d.P(), K = d.K(), image = (int64_t)d.in.C * d.in.H * d.in.W;
+  const int64_t slab = std::min(d.in.batch, std::max<int64_t>(1, kColumnBytes / (P * K * (int64_t)sizeof(float))));
+  // the columns, their fp32 gradients and, for bf16, both results in fp32, each
+  // part 256-byte aligned
+  auto part = [](int64_t n, size_t size) { return ((size_t)n * size + 255) / 256 * 256; };
+  const size_t cols = part(slab * P * K, sizeof(T)), gcols = part(slab * P * K, sizeof(float));
+  const bool sums = !F32 && d.in.batch > 1;  // the weight gradient is a sum over products
+  const size_t weights = sums ? part(d.cout * K, sizeof(float)) : 0, images = F32 ? 0 : part(slab * image, sizeof(float));
+  Scratch scratch(cols + gcols + weights + images);
+  if (!scratch.p) return false;
+  char* at = static_cast<char*>(scratch.p);
+  T* col = reinterpret_cast<T*>(at);
+  float *gcol = reinterpret_cast<float*>(at += cols), *gw32 = reinterpret_cast<float*>(at + gcols), *gin32;
+  for (int64_t n = 0; n < d.in.batch; n += slab) {
+    const ConvShape s{std::min(slab, d.in.batch - n), d.in.C, d.in.H, d.in.W};
+    im2col_call(fn, in + n * image, col, s, d.kh, d.kw, ph, pw, sh, sw);
+    for (int64_t i = 0; i < s.batch; ++i) {
+      const T* goi = go + (n + i) * d.cout * P;
+      const float beta = n + i == 0 ? 0.f : 1.f;
+      if (sums)
+        gemm_to_f32<T>(fn.c_str(), false, false, d.cout, K, P, goi, col + i * P * K, beta, gw32);
+      else
+        gemm<T>(fn.c_str(), false, false, d.cout, K, P, 1.f, goi, col + i * P * K, beta, gw);
+      gemm_to_f32<T>(fn.c_str(), true, false, P, K, d.cout, goi, w, 0.f, gcol + i * P * K);
+    }
+    if constexpr (F32)
+      gin32 = gin + n * image;
+    else
+      gin32 = reinterpret_cast<float*>(at + gcols + weights);
+    col2im_call<float>(fn, gcol, gin32, s, d.kh, d.kw, ph, pw, sh, sw);
+    if constexpr (!F32) to_bf16(fn.c_str(), gin32, gin + n * image, s.batch * image);
+  }
+  if (sums) to_bf16(fn.c_str(), gw32, gw, d.cout * K);
+  return true;
+}
+
+// Whether the column matrix takes a convolution instead of the products that
+// gather their operands (tt_conv_*).  Those gather an image once per 64 output
+// channels (the backward also the weights once per 64 pixels), at 50-170
+// TFLOP/s in bf16 and 50-70 in fp32 whatever the size; the columns are written
+// once and their products run at the GEMM's rate where one image's fill the
+// chip.  Measured (us, one image unless given, gathered / columns): bf16 forward
+// 2048 channels 28 x 28 3 x 3 414 / 246, 1024 64 x 64 3 x 3 411 / 265, but 512 28 x 28
+// 39 / 42 and 8 images of 512 28 x 28 234 / 310; backward 512 64 x 64 442 / 250,
+// 1024 64 x 64 1387 / 490, 2048 28 x 28 1423 / 459, 8 images of 768 64 x 64 stride
+// 2 1952 / 1186, but 8 of 384 28 x 28 351 / 520; fp32 backward 2048 28 x 28 2224 /
+// 1300, 512 64 x 64 727 / 581.  With a stride the gathered backward loses from
+// 256 channels on (256 of 512, 64 x 64, 102 / 80).  Windows that do not overlap
+// need no phases and are gathered with less work: 1 x 1 64 x 64 bf16 backward 48 /
+// 55 at 512 channels, 146 / 114 at 1024, fp32 832 / 689 at 2048.
+bool wide_products(const ConvDims& d, bool bf16, bool backward, int sh, int sw) {
+  const double products = (double)d.P() * d.cout * (double)d.K();  // per image
+  if (sh >= d.kh && sw >= d.kw) return d.cout >= 512 && products >= (bf16 ? 0x1p31 : 0x1p34);
+  const int wide = !backward ? 512 : sh > 1 || sw > 1 ? 256 : 384;
+  return d.cout >= wide && products >= (d.in.batch == 1 ? 0x1p30 : 0x1p32) / (backward ? 2 : 1);
+}
+
 }  // namespace
 
 template <typename T>
@@ -398,18 +509,13 @@ void ConvForward(const TinyTensor<T>& input, TinyTensor<T>& output, const TinyTe
   oshape.insert(oshape.end(), {d.cout, d.oh, d.ow});
   output.resize_output(oshape);
   if (d.in.batch == 0 || d.cout == 0) return;
+  auto columns = [&] {
+    return conv_forward_columns(fn, input.p_data, weight.p_data, output.p_data, d, pad_h, pad_w, stride_h, stride_w);
+  };
+  if (wide_products(d, !std::is_same<T, float>::value, false, stride_h, stride_w) && columns()) return;
   const int rc = tt_conv_forward(dtype_code<T>(), input.p_data, weight.p_data, output.p_data, d.in.batch, d.in.C,
                                  d.in.H, d.in.W, d.cout, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w, nullptr);
-  if (rc == TT_ERR_UNSUPPORTED) {  // planes past its 32-bit indices: column matrix and one product per image
-    const int64_t P = d.P(), K = d.K();
-    TinyTensor<T> col(std::vector<int>{(int)d.in.batch, (int)P, (int)K}, "gpu");
-    im2col_call(fn, input.p_data, col.p_data, d.in, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w);
-    for (int64_t n = 0; n < d.in.batch; ++n)
-      gemm<T>(fn.c_str(), false, true, d.cout, P, K, 1.f, weight.p_data, col.p_data + n * P * K, 0.f,
-              output.p_data + n * d.cout * P);
-  } else {
-    tt_check(rc, fn.c_str());
-  }
+  tt_check(rc != TT_ERR_UNSUPPORTED ? rc : columns() ? TT_OK : TT_ERR_NOMEM, fn.c_str());  // past its indices or grid
 }
 
 template <typename T>
@@ -434,23 +540,15 @@ void ConvBackward(const TinyTensor<T>& input, const TinyTensor<T>& output, const
     grad_weight.zeros();
     return;
   }
+  auto columns = [&] {
+    return conv_backward_columns(fn, input.p_data, weight.p_data, grad_output.p_data, grad_input.p_data,
+                                 grad_weight.p_data, d, pad_h, pad_w, stride_h, stride_w);
+  };
+  if (wide_products(d, !std::is_same<T, float>::value, true, stride_h, stride_w) && columns()) return;
   const int rc = tt_conv_backward(dtype_code<T>(), input.p_data, weight.p_data, grad_output.p_data, grad_input.p_data,
                                   grad_weight.p_data, d.in.batch, d.in.C, d.in.H, d.in.W, d.cout, d.kh, d.kw, pad_h,
                                   pad_w, stride_h, stride_w, nullptr);
-  if (rc == TT_ERR_UNSUPPORTED) {  // as in ConvForward
-    TinyTensor<T> col(std::vector<int>{(int)d.in.batch, (int)P, (int)K}, "gpu");
-    im2col_call(fn, input.p_data, col.p_data, d.in, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w);
-    TinyTensor<T> grad_col(std::vector<int>{(int)d.in.batch, (int)P, (int)K}, "gpu");
-    for (int64_t n = 0; n < d.in.batch; ++n) {
-      const T* go = grad_output.p_data + n * d.cout * P;
-      gemm<T>(fn.c_str(), false, false, d.cout, K, P, 1.f, go, col.p_data + n * P * K, n == 0 ? 0.f : 1.f,
-              grad_weight.p_data);
-      gemm<T>(fn.c_str(), true, false, P, K, d.cout, 1.f, go, weight.p_data, 0.f, grad_col.p_data + n * P * K);
-    }
-    col2im_call(fn, grad_col.p_data, grad_input.p_data, d.in, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w);
-  } else {
-    tt_check(rc, fn.c_str());
-  }
+  tt_check(rc != TT_ERR_UNSUPPORTED ? rc : columns() ? TT_OK : TT_ERR_NOMEM, fn.c_str());  // as in ConvForward
 }
 
 namespace {

@@ -388,6 +388,12 @@ __global__ void k_fill_normal(T* dst, int64_t n, uint64_t seed, float scale) {
   }
 }
 
+__global__ __launch_bounds__(256) void k_round_bf16(const float* __restrict__ src, uint16_t* __restrict__ dst,
+                                                    int64_t n) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = f2bf(src[i]);
+}
+
 static int grid_for(int64_t n) {
   int64_t g = (n + 255) / 256;
   if (g > 65536) g = 65536;
@@ -679,6 +685,18 @@ int tt_elementwise(int op, int dtype, void* c, const void* a, const void* b, int
       return fail(TT_ERR_ARG, "tt_elementwise: bad dtype");
   }
   TT_LAUNCH_CHECK("tt_elementwise");
+  return ok();
+}
+
+int tt_round_bf16(const float* src, uint16_t* dst, int64_t n, void* stream) {
+  if (n < 0) return fail(TT_ERR_ARG, "tt_round_bf16: negative size");
+  if (n == 0) return TT_OK;
+  if (!src || !dst) return fail(TT_ERR_ARG, "tt_round_bf16: null pointer");
+  int rc = ensure_init();
+  if (rc) return rc;
+  hipStream_t s = stream_or_default(stream);
+  hipLaunchKernelGGL(k_round_bf16, dim3(grid_for(n)), dim3(256), 0, s, src, dst, n);
+  TT_LAUNCH_CHECK("tt_round_bf16");
   return ok();
 }
 

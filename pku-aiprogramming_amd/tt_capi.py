@@ -76,6 +76,8 @@ _SIGS = {
     "tt_softmax_rows_f32": (C.c_int, [_p, _p, _i64, _i64, _p]),
     "tt_gemm_f32": (C.c_int, [C.c_int, C.c_int, _i64, _i64, _i64, C.c_float, _p, _p, C.c_float, _p, _p]),
     "tt_gemm_bf16": (C.c_int, [C.c_int, C.c_int, _i64, _i64, _i64, C.c_float, _p, _p, C.c_float, _p, _p]),
+    "tt_gemm_bf16_f32": (C.c_int, [C.c_int, C.c_int, _i64, _i64, _i64, C.c_float, _p, _p, C.c_float, _p, _p]),
+    "tt_round_bf16": (C.c_int, [_p, _p, _i64, _p]),
     "tt_conv_forward": (C.c_int, [C.c_int, _p, _p, _p, _i64] + [C.c_int] * 10 + [_p]),
     "tt_conv_backward": (C.c_int, [C.c_int, _p, _p, _p, _p, _p, _i64] + [C.c_int] * 10 + [_p]),
     "tt_fc_forward": (C.c_int, [C.c_int, _i64, _i64, _i64, _p, _p, _p, C.c_int, _p, _p]),

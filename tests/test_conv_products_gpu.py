@@ -6,11 +6,16 @@ or leave pixels uncovered, sums split over workgroups.  Reference: numpy
 float64 on the same (for bf16: bf16-rounded) values.  Bars (normwise
 max|x - ref| / max|ref|): fp32 1e-5 (fp32 products and sums), bf16 8e-3 (one
 rounding of the result)."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 from oracle import attn_oracle as orc
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 pytestmark = pytest.mark.gpu
 
 TOL = {"float": 1e-5, "bf16": 8e-3}
@@ -47,7 +52,7 @@ CASES = [
 ]
 
 
-def _ref(x, w, go, ph, pw, sh, sw):
+def _ref(x, w, go, ph, pw, sh, sw, blas=False):
     N, C, H, W = x.shape
     Co, _, kh, kw = w.shape
     oh, ow = (H + 2 * ph - kh) // sh + 1, (W + 2 * pw - kw) // sw + 1
@@ -57,9 +62,9 @@ def _ref(x, w, go, ph, pw, sh, sw):
     for ky in range(kh):
         for kx in range(kw):
             at = (slice(None), slice(None), slice(ky, ky + sh * (oh - 1) + 1, sh), slice(kx, kx + sw * (ow - 1) + 1, sw))
-            out += np.einsum("oc,ncyx->noyx", w[:, :, ky, kx], xp[at])
-            gw[:, :, ky, kx] = np.einsum("noyx,ncyx->oc", go, xp[at])
-            gxp[at] += np.einsum("oc,noyx->ncyx", w[:, :, ky, kx], go)
+            out += np.einsum("oc,ncyx->noyx", w[:, :, ky, kx], xp[at], optimize=blas)
+            gw[:, :, ky, kx] = np.einsum("noyx,ncyx->oc", go, xp[at], optimize=blas)
+            gxp[at] += np.einsum("oc,noyx->ncyx", w[:, :, ky, kx], go, optimize=blas)
     return out, gw, gxp[:, :, ph:ph + H, pw:pw + W]
 
 
@@ -149,3 +154,64 @@ def test_rows_beyond_the_grid(case):
         e = orc.max_rel_err(np.asarray(got.numpy()).reshape(r.size), r.ravel())
         print(f"  {name} {e:.2e}", flush=True)
         assert e <= TOL["float"], (name, e)
+
+
+# Channels wide enough for the column matrix: one image both ways, a batch in
+# two parts backward, a stride, windows apart (bf16)
+@pytest.mark.parametrize("dt", ["float", "bf16"])
+@pytest.mark.parametrize("case", [(1, 320, 28, 28, 512, 3, 3, 1, 1, 1, 1), (4, 320, 40, 40, 512, 3, 3, 1, 1, 1, 1),
+                                  (1, 257, 63, 64, 257, 3, 3, 1, 1, 2, 2), (1, 3, 1024, 1024, 768, 16, 16, 0, 0, 16, 16)],
+                         ids=str)
+def test_wide_products(dt, case):
+    import myLayer as ml
+    import myTensor as mt
+
+    T = getattr(mt, "Tensor_" + dt)
+    N, C, H, W, Co, kh, kw, ph, pw, sh, sw = case
+    rng = np.random.default_rng(sum(case))
+    oh, ow = (H + 2 * ph - kh) // sh + 1, (W + 2 * pw - kw) // sw + 1
+    x, w, go = (rng.standard_normal(s).astype(np.float32) for s in ((N, C, H, W), (Co, C, kh, kw), (N, Co, oh, ow)))
+    if dt == "bf16":
+        x, w, go = orc.bf16_round(x), orc.bf16_round(w), orc.bf16_round(go)
+    X, Wt, GO = (T(a, "gpu") for a in (x, w, go))
+    out, gx, gw = (T([1], "gpu") for _ in range(3))
+    ml.ConvForward(X, out, Wt, ph, pw, sh, sw)
+    ml.ConvBackward(X, out, Wt, gx, GO, gw, ph, pw, sh, sw)
+    ref = _ref(x.astype(np.float64), w.astype(np.float64), go.astype(np.float64), ph, pw, sh, sw, blas=True)
+    for name, got, r in zip(("out", "grad_weight", "grad_input"), (out, gw, gx), ref):
+        a = np.asarray(got.numpy()).reshape(r.shape)
+        e, two = orc.max_rel_err(a, r), np.linalg.norm(a - r) / np.linalg.norm(r)
+        print(f"  {name} {e:.2e} 2-norm {two:.2e}", flush=True)
+        assert e <= TOL[dt], (name, e)
+        # bf16: one rounding of each result and none before it: 2^-8 / sqrt(3) x 0.74 = 1.66e-3 over significands
+        # spread evenly in the logarithm (a rounding of the columns' gradients too would give 2.3e-3)
+        assert two <= (1e-6 if dt == "float" else 2e-3), (name, two)
+
+
+def test_wide_products_without_scratch():
+    """The gathered products take over where the columns' memory is refused."""
+    code = (
+        "import ctypes as C, numpy as np, myLayer as ml, myTensor as mt, tt_capi as T\n"
+        "from test_conv_products_gpu import _ref\n"
+        "from oracle import attn_oracle as orc\n"
+        "r = np.random.default_rng(1)\n"
+        "x, w, go = (r.standard_normal(s).astype(np.float32) for s in ((1, 320, 28, 28), (512, 320, 3, 3), (1, 512, 28, 28)))\n"
+        "t = [mt.Tensor_float(a, 'gpu') for a in (x, w, go)]\n"
+        "out, gx, gw = (mt.Tensor_float(list(s), 'gpu') for s in ((1, 512, 28, 28), x.shape, w.shape))\n"
+        "def in_use():\n"
+        "    a = C.c_size_t(); T.lib().call('tt_mem_stats', C.byref(a), None); return a.value\n"
+        "before = in_use()\n"
+        "ml.ConvForward(t[0], out, t[1], 1, 1, 1, 1)\n"
+        "ml.ConvBackward(t[0], out, t[1], gx, t[2], gw, 1, 1, 1, 1)\n"
+        "assert in_use() == before, 'scratch was not refused'\n"
+        "ref = _ref(*(a.astype(np.float64) for a in (x, w, go)), 1, 1, 1, 1, blas=True)\n"
+        "for a, b in zip((out, gw, gx), ref):\n"
+        "    assert orc.max_rel_err(np.asarray(a.numpy()).reshape(b.shape), b) <= 1e-5\n"
+        "try:\n"
+        "    T.DeviceBuffer((1 << 20,))\n"
+        "except T.TTError as e:\n"
+        "    print('REFUSED', e.code == T.TT_ERR_NOMEM)\n")
+    env = dict(os.environ, TT_FAIL_ALLOC_AFTER="6", PYTHONPATH=os.pathsep.join(
+        [ROOT, os.path.join(ROOT, "tests"), os.path.join(ROOT, "pku-aiprogramming_amd"), os.environ.get("PYTHONPATH", "")]))
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "REFUSED True" in r.stdout, r.stdout + r.stderr
