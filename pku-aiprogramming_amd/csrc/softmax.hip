@@ -325,11 +325,21 @@ __global__ __launch_bounds__(64 * W) void k_softmax_stream(const float* __restri
 constexpr int kSplitMaxChunks = 64;
 
 // ALIGNED: cols % 4 == 0 and 16-byte aligned x and y.  Otherwise rows begin
-// at any float and a row's last vector may be partial.
+// at any float and a row's last vector may be partial.  ANEW, the unaligned rows
+// beyond 65536 columns: exp(x - M) / S is formed anew from x, as the two-pass
+// kernel did that took them before; the sum's own terms rescaled by the chunk's
+// exp(m - M) / S are 6-8 % further from float64 there (1024 x 100003 7.9e-8 against
+// 7.3e-8, 1024 x 150001 8.2e-8 against 7.7e-8) and 2-4 % faster (145 / 149, 212 / 220
+// us; two passes 313, 500).  Elsewhere they are no further off than what they
+// replaced (1000 x 65535 7.2e-8, before 1.2e-7).
+__device__ __forceinline__ f32x4v exps(f32x4v x, float m) {
+  return f32x4v{ex(x.x - m), ex(x.y - m), ex(x.z - m), ex(x.w - m)};
+}
 template <int NE4, bool ALIGNED>
 __global__ __launch_bounds__(kBlock) void k_softmax_split(const float* x, float* y, int64_t cols, int nchunk,
                                                          unsigned long long* slots, unsigned gen) {
   constexpr int CW = 1024 * NE4;  // columns per chunk
+  constexpr bool ANEW = !ALIGNED && NE4 >= 16;
   __shared__ float red_m[4], red_s[4];
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
   const int64_t row = (int64_t)blockIdx.x / nchunk;
@@ -365,11 +375,9 @@ __global__ __launch_bounds__(kBlock) void k_softmax_split(const float* x, float*
   float s = 0.f;
 #pragma unroll
   for (int k = 0; k < NE4; ++k) {
-    v[k].x = ex(v[k].x - mb);
-    v[k].y = ex(v[k].y - mb);
-    v[k].z = ex(v[k].z - mb);
-    v[k].w = ex(v[k].w - mb);
-    s += (v[k].x + v[k].y) + (v[k].z + v[k].w);
+    const f32x4v e = exps(v[k], mb);
+    s += (e.x + e.y) + (e.z + e.w);
+    if constexpr (!ANEW) v[k] = e;
   }
   s = group_sum<64>(s);
   if (l == 0) red_s[w] = s;
@@ -416,10 +424,11 @@ __global__ __launch_bounds__(kBlock) void k_softmax_split(const float* x, float*
   // exp(m - M) / S; a row with no finite value gives NaN (0 / 0 and
   // -inf - -inf), as the reference's x - max does
   const float f = bad ? NAN : (m == -INFINITY && M != -INFINITY ? 0.f : ex(m - M)) / S;
+  if (bad) S = NAN;
 #pragma unroll
   for (int k = 0; k < NE4; ++k) {
     const int c = 4 * t + 1024 * k;
-    const f32x4v r = v[k] * f;
+    const f32x4v r = ANEW ? exps(v[k], M) / S : v[k] * f;
     if constexpr (ALIGNED) {
       if (c < rem) __builtin_nontemporal_store(r, reinterpret_cast<f32x4v*>(yr + c));
     } else if (c + 4 <= rem) {

@@ -53,6 +53,26 @@ def test_chunks_without_finite_values(capi):
     assert np.all(y[2, :4096] == 0) and np.all(y[3, 12288:] == 0)
 
 
+@pytest.mark.parametrize("cols", [65537, 100003, 262145])
+def test_long_rows_round_each_element_alike(capi, cols):
+    """Unaligned rows beyond 65536 columns: exp(x - M) / S from the row's maximum, so that equal elements
+    give equal bits whatever the maximum of their chunk; rows and chunks without a finite value."""
+    x = (3 * np.random.default_rng(cols).standard_normal((12, cols))).astype(np.float32)
+    last = cols - 700
+    x[:, last:last + 500] = x[:, 100:600]
+    x[1, last + 600] = 25.0  # a chunk far above the others
+    x[2, 20000:60000] = -np.inf
+    x[3, :] = -np.inf
+    x[4, 17] = np.nan
+    x[5, -1] = np.inf
+    y = _run(capi, x, 1, 2)
+    assert np.isnan(y[[3, 4, 5]]).all()
+    keep = np.delete(np.arange(12), [3, 4, 5])
+    assert orc.max_rel_err(y[keep], orc.softmax_rows_f64(x[keep])) <= 1e-5
+    np.testing.assert_array_equal(y[keep, last:last + 500], y[keep, 100:600])
+    assert np.all(y[2, 20000:60000] == 0)
+
+
 # one workgroup per row, vectors from 128-byte lines: around its range and the
 # counts of vectors per lane (1024 k and 2048 k floats less the shift of up to 31)
 @pytest.mark.parametrize("cols", [3328, 3329, 4064, 4065, 4096, 4097, 8160, 8161, 8162, 8192, 8193, 10209, 10240, 12257,
