@@ -10,9 +10,10 @@
 // few heads and keys to fill the chip that way.)  Phase 1 streams its K rows
 // (16-byte non-temporal loads, TPR threads per row, several rows in flight per thread) and writes the log2-domain scores
 // to LDS; phase 2 reduces max and sum over the chunk; phase 3 streams the V
-// rows and accumulates sum_j p_j V_j.  Each split writes a normalised partial
-// (o_c, lse_c) in fp32; a combine kernel merges them by LSE rescaling:
-//   lse = log2 sum_c 2^lse_c,  o = sum_c 2^(lse_c - lse) o_c.
+// rows and accumulates sum_j p_j V_j.  Each split writes its sums, not yet
+// divided, and its max and sum of weights (o_c, m_c, l_c) in fp32; a combine kernel
+// merges them:
+//   m = max_c m_c,  l = sum_c 2^(m_c - m) l_c,  o = sum_c 2^(m_c - m) o_c / l.
 // When one split covers a whole head, the split kernel writes o and lse
 // itself and there is no combine launch.
 #include <hip/hip_runtime.h>
@@ -72,11 +73,11 @@ __device__ __forceinline__ float block_reduce(float v, float* red, bool is_max) 
 
 // MAXC: largest chunk the LDS score buffer holds.  DIRECT (nsplit == 1): o
 // and lse (natural log, may be null) are written here in the output type;
-// otherwise the fp32 partials go to part_o / part_lse.
+// otherwise the fp32 partials go to part_o / part_ml.
 template <typename T, int D, int UNROLL, int MAXC, bool DIRECT>
 __global__ __launch_bounds__(DEC_THREADS) void attn_decode_split_kernel(
     const T* __restrict__ q, const T* __restrict__ K, const T* __restrict__ V,
-    float* __restrict__ part_o, float* __restrict__ part_lse, T* __restrict__ o, float* __restrict__ lse,
+    float* __restrict__ part_o, float2* __restrict__ part_ml, T* __restrict__ o, float* __restrict__ lse,
     int Lkv, int nsplit, int chunk, float sl2) {
   constexpr int EPT = Vec16<T>::N;     // elements per 16-byte load
   constexpr int TPR = D / EPT;         // threads per key row
@@ -164,7 +165,7 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_split_kernel(
 #pragma unroll 8
     for (int r = 0; r < RPP; ++r) s += sAcc[r * D + dd];
     if constexpr (!DIRECT)
-      part_o[pidx * D + dd] = s * inv;
+      part_o[pidx * D + dd] = s;
     else if constexpr (sizeof(T) == 2)
       o[bh * D + dd] = f32_to_bf16(s * inv);
     else
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_split_kernel(
   }
   if (tid == 0) {
     if constexpr (!DIRECT)
-      part_lse[pidx] = mx + __log2f(sm);
+      part_ml[pidx] = float2{mx, sm};
     else if (lse)
       lse[bh] = (mx + __log2f(sm)) * kLn2;
   }
@@ -190,7 +191,7 @@ constexpr int dec_short_chunk() { return kDecRows * DEC_THREADS / (D / Vec16<T>:
 template <typename T, int D>
 __global__ __launch_bounds__(DEC_THREADS) void attn_decode_short_kernel(
     const T* __restrict__ q, const T* __restrict__ K, const T* __restrict__ V, float* __restrict__ part_o,
-    float* __restrict__ part_lse, T* __restrict__ o, float* __restrict__ lse, int Lkv, int nsplit, float sl2) {
+    float2* __restrict__ part_ml, T* __restrict__ o, float* __restrict__ lse, int Lkv, int nsplit, float sl2) {
   constexpr int EPT = Vec16<T>::N, TPR = D / EPT, RPP = DEC_THREADS / TPR, R = kDecRows;
   constexpr int NW = DEC_THREADS / 64;
   __shared__ __align__(16) float s_acc[NW][D];
@@ -273,9 +274,9 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_short_kernel(
   }
   const int64_t pidx = bh * nsplit + split;
   if (nsplit > 1) {
-    // a split whose scores are all -inf: lse = -inf and o = 0, weight 0 in the merge
-    part_o[pidx * D + tid] = den == 0.f ? 0.f : num / den;
-    if (tid == 0) part_lse[pidx] = M + __log2f(den);
+    // a split whose scores are all -inf: m = -inf, weight 0 in the merge
+    part_o[pidx * D + tid] = num;
+    if (tid == 0) part_ml[pidx] = float2{M, den};
     return;
   }
   const float inv = 1.f / den;
@@ -291,10 +292,12 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_short_kernel(
 // (One thread per column walking the splits in turn took 6 us for 17 splits
 // and 40 us for 128.)  NT = 256, or max(64, D) for up to 8 splits: a decode of
 // 928 heads in two splits each took 15.3 us with 256 threads a head, 14.9 with
-// D.
+// D.  The splits' weights come from their max and sum: taken from an LSE each,
+// they carry its rounding (fp32 d = 128, 128 keys in two splits: 1.7e-7 from float64,
+// 1.5e-7 in one).
 template <typename T, int D, int NT>
 __global__ __launch_bounds__(NT) void attn_decode_combine_kernel(const float* __restrict__ part_o,
-                                                                  const float* __restrict__ part_lse,
+                                                                  const float2* __restrict__ part_ml,
                                                                   T* __restrict__ o, float* __restrict__ lse,
                                                                   int nsplit) {
   constexpr int TPR = D / 4, G = NT / TPR;
@@ -302,18 +305,19 @@ __global__ __launch_bounds__(NT) void attn_decode_combine_kernel(const float* __
   __shared__ float s_w[G];
   const int64_t bh = blockIdx.x;
   const int tid = threadIdx.x, c = tid % TPR, g = tid / TPR;
-  const float* pl = part_lse + bh * nsplit;
+  const float2* pl = part_ml + bh * nsplit;
   const float* po = part_o + bh * nsplit * D + 4 * c;
   float mx = -INFINITY;  // every wave forms the maximum by itself
-  for (int s = tid & 63; s < nsplit; s += 64) mx = vmax(mx, pl[s]);
+  for (int s = tid & 63; s < nsplit; s += 64) mx = vmax(mx, pl[s].x);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) mx = vmax(mx, __shfl_xor(mx, off, 64));
   float sw = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int s = g; s < nsplit; s += G) {
-    const float wgt = fast_exp2(pl[s] - mx);
-    sw += wgt;
+    const float2 ml = pl[s];
+    const float wgt = fast_exp2(ml.x - mx);
+    sw += wgt * ml.y;
     acc += wgt * *reinterpret_cast<const f32x4*>(po + (int64_t)s * D);
   }
   *reinterpret_cast<f32x4*>(&s_acc[g][4 * c]) = acc;
@@ -336,7 +340,7 @@ __global__ __launch_bounds__(NT) void attn_decode_combine_kernel(const float* __
 
 constexpr int64_t kDecShortBytes = int64_t(56) << 20;
 // Scratch of the short splits' partials, of one size so that it is allocated
-// once per stream: 4064 of them at d = 128.  The rule below makes at most
+// once per stream: 4032 of them at d = 128.  The rule below makes at most
 // 56 MB / 32 KB (a split's keys) and one more for each of fewer than 1792 heads.
 constexpr size_t kDecShortWork = size_t(2) << 20;
 
@@ -382,7 +386,7 @@ static int launch_decode(const T* q, const T* k, const T* v, T* o, float* lse, i
   const float sl2 = scale * kLog2e;
   void* ws = nullptr;
   std::optional<WorkspaceLease> lease;  // held until both kernels are launched
-  auto partials = [&](int64_t n) { return (size_t)(BH * n) * (D + 1) * sizeof(float); };
+  auto partials = [&](int64_t n) { return (size_t)(BH * n) * (D + 2) * sizeof(float); };
   if (is_short && short_splits > 1 &&
       (partials(short_splits) > kDecShortWork || !lease.emplace().get_fixed(st, kWsDecodeShort, kDecShortWork, &ws))) {
     is_short = false;  // no scratch for them: long splits
@@ -407,24 +411,24 @@ static int launch_decode(const T* q, const T* k, const T* v, T* o, float* lse, i
     return ok();
   }
   float* part_o = (float*)ws;
-  float* part_lse = part_o + BH * nsplit * D;
+  float2* part_ml = (float2*)(part_o + BH * nsplit * D);
   if (is_short)
-    hipLaunchKernelGGL((attn_decode_short_kernel<T, D>), grid, block, 0, st, q, k, v, part_o, part_lse, nullptr,
+    hipLaunchKernelGGL((attn_decode_short_kernel<T, D>), grid, block, 0, st, q, k, v, part_o, part_ml, nullptr,
                        nullptr, (int)Lkv, (int)nsplit, sl2);
   else if (chunk <= DEC_SMALL_CHUNK)
     hipLaunchKernelGGL((attn_decode_split_kernel<T, D, 8, DEC_SMALL_CHUNK, false>), grid, block, 0, st, q, k, v,
-                       part_o, part_lse, nullptr, nullptr, (int)Lkv, (int)nsplit, chunk, sl2);
+                       part_o, part_ml, nullptr, nullptr, (int)Lkv, (int)nsplit, chunk, sl2);
   else
     hipLaunchKernelGGL((attn_decode_split_kernel<T, D, 8, DEC_MAX_CHUNK, false>), grid, block, 0, st, q, k, v,
-                       part_o, part_lse, nullptr, nullptr, (int)Lkv, (int)nsplit, chunk, sl2);
+                       part_o, part_ml, nullptr, nullptr, (int)Lkv, (int)nsplit, chunk, sl2);
   TT_LAUNCHED("attention decode split launch", st);
   constexpr int kFew = D > 64 ? D : 64;
   if (nsplit <= 8)
     hipLaunchKernelGGL((attn_decode_combine_kernel<T, D, kFew>), dim3((unsigned)BH), dim3(kFew), 0, st, part_o,
-                       part_lse, o, lse, (int)nsplit);
+                       part_ml, o, lse, (int)nsplit);
   else
     hipLaunchKernelGGL((attn_decode_combine_kernel<T, D, 256>), dim3((unsigned)BH), dim3(256), 0, st, part_o,
-                       part_lse, o, lse, (int)nsplit);
+                       part_ml, o, lse, (int)nsplit);
   TT_LAUNCHED("attention decode combine launch", st);
   return ok();
 }

@@ -25,10 +25,10 @@ def capi():
     return tt_capi
 
 
-def _run(capi, dt, q, k, v):
+def _run(capi, dt, q, k, v, scale=0.125):
     bufs = [capi.DeviceBuffer.from_numpy(a, dt) for a in (q, k, v)]
     o, lse = capi.DeviceBuffer(q.shape, dt), capi.DeviceBuffer(q.shape[:2], "f32")
-    capi.attn_decode(*bufs, o, lse, 0.125)
+    capi.attn_decode(*bufs, o, lse, scale)
     return o.download(), lse.download()
 
 
@@ -49,6 +49,22 @@ def test_short_splits(capi, dt, d, chunks):
     ro, rl = orc.attn_decode_f64(q, k, v, 0.125)
     assert orc.max_rel_err(o, ro) <= orc.TOL[dt]
     assert orc.max_rel_err(lse.reshape(np.shape(rl)), rl) <= 1e-5  # fp32 weights and sums
+
+
+@pytest.mark.parametrize("d,L", [(64, 128), (64, 200), (64, 256), (128, 64), (128, 128), (128, 200), (128, 256)])
+def test_merged_splits_are_as_precise_as_one(capi, d, L):
+    """fp32, one and several splits.  The 2-norm error of one split is that of its weights: 2^(s - m) to a few
+    2^-24 each, 1.35e-7 to 1.6e-7 here.  Weights of the splits taken from an LSE each (a number of about 8,
+    rounded to 2^-21) would add to it: 1.7e-7 to 1.95e-7 beyond one split."""
+    q, k, v = _inputs("f32", 1, 240, L, d, L + d)
+    scale = float(np.float32(d ** -0.5))
+    o, _ = _run(capi, "f32", q, k, v, scale)
+    s = np.einsum("bhqd,bhkd->bhqk", q.astype(np.float64), k.astype(np.float64)) * scale
+    p = np.exp(s - s.max(-1, keepdims=True))
+    ref = (p / p.sum(-1, keepdims=True)) @ v.astype(np.float64)
+    e = np.linalg.norm(o - ref) / np.linalg.norm(ref)
+    print(f"  {e:.2e}", flush=True)
+    assert e <= 1.65e-7
 
 
 @pytest.mark.parametrize("BH,L,d", [(1299, 256, 32), (1300, 256, 32), (1300, 257, 32), (1300, 128, 64), (1300, 129, 64)])
