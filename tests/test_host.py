@@ -50,6 +50,21 @@ def test_library_exports_nothing_else_but_the_abi(capi):
     assert tt == capi.header_functions()
 
 
+def test_ctypes_signatures_match_the_header(capi):
+    """Count and kind of every declared function's parameters."""
+    import ctypes as C
+    import re
+
+    text = re.sub(r"/\*.*?\*/", "", open(capi.HEADER).read(), flags=re.S)
+    scalars = {"int": C.c_int, "int64_t": C.c_int64, "uint64_t": C.c_uint64, "size_t": C.c_size_t, "float": C.c_float,
+               "double": C.c_double}
+    for name, (_, args) in capi._SIGS.items():
+        params = re.search(r"\b" + name + r"\s*\(([^)]*)\)", text)[1].split(",")
+        want = [None if "*" in p else scalars[p.split()[0]] for p in params if p.strip() != "void"]
+        got = [a if a in scalars.values() else None for a in args]
+        assert got == want, name
+
+
 def _gpu_present():
     return os.path.exists("/dev/kfd")
 
