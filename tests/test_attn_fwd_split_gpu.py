@@ -75,19 +75,23 @@ def test_split_forward_extreme_scores(capi):
 
 def test_refused_scratch_runs_unsplit(capi):
     code = (
-        "import numpy as np, tt_capi as T\n"
+        "import ctypes as C, numpy as np, tt_capi as T\n"
         "from oracle import attn_oracle as orc\n"
         "r = np.random.default_rng(1)\n"
         "q, k, v = (orc.bf16_round(r.standard_normal((1, 1, n, 64)).astype(np.float32)) for n in (9, 2000, 2000))\n"
         "b = [T.DeviceBuffer.from_numpy(a, 'bf16') for a in (q, k, v)]\n"
         "o, l = T.DeviceBuffer(q.shape, 'bf16'), T.DeviceBuffer(q.shape[:3], 'f32')\n"
+        "def in_use():\n"
+        "    n = C.c_size_t(); T.lib().call('tt_mem_stats', C.byref(n), None); return n.value\n"
+        "before = in_use()\n"
         "T.attn_fwd(*b, o, l, 0.125, False)\n"
+        "assert in_use() == before, 'the scratch was not refused'\n"
         "assert orc.max_rel_err(o.download(), orc.attn_fwd_f64(q, k, v, 0.125, False)[0]) <= 2e-2\n"
         "try:\n"
         "    T.DeviceBuffer((1 << 20,))\n"
         "except T.TTError as x:\n"
         "    print('REFUSED', x.code == T.TT_ERR_NOMEM)\n")
-    env = dict(os.environ, TT_FAIL_ALLOC_AFTER="6", PYTHONPATH=os.pathsep.join(
+    env = dict(os.environ, TT_FAIL_ALLOC_AFTER="5", PYTHONPATH=os.pathsep.join(
         [ROOT, os.path.join(ROOT, "pku-aiprogramming_amd"), os.environ.get("PYTHONPATH", "")]))
     r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "REFUSED True" in r.stdout, r.stdout + r.stderr

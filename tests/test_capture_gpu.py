@@ -1,17 +1,21 @@
-"""GPU tests of the library under stream capture: the calls that take scratch
-only where they can (products, column sums, convolutions, the bf16 forward,
-long softmax rows) captured into a graph and replayed on new inputs with eager
-work in between, the same calls on one stream while another is being captured
-(they may neither end that capture nor join it), and tt_malloc then.  Each
-result against float64 at the bars of the eager tests: 1e-5 normwise where
-sums and products are fp32, 2e-2 for bf16 attention."""
+"""GPU tests of the calls that take scratch only where they can (products,
+column sums, convolutions, the bf16 forward, long softmax rows): with the
+scratch refused, captured into a graph and replayed on new inputs with eager
+work in between, and on one stream while another is being captured (they may
+neither end that capture nor join it); and of tt_malloc then.  Each result
+against float64 at the bars of the eager tests: 1e-5 normwise where sums and
+products are fp32, 2e-2 for bf16 attention."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
 from oracle import attn_oracle as orc
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 pytestmark = pytest.mark.gpu
 
 GLOBAL, THREAD_LOCAL = 0, 1  # hipStreamCaptureMode
@@ -129,6 +133,55 @@ class Capture:
             self.hip.hipGraphExecDestroy(self.exec)
         if self.graph:
             self.hip.hipGraphDestroy(self.graph)
+
+
+REFUSED = """
+import ctypes as C
+import tt_capi as T
+from test_capture_gpu import Op
+
+def in_use():
+    n = C.c_size_t()
+    T.lib().call("tt_mem_stats", C.byref(n), None)
+    return n.value
+
+op = Op(T, "%s")
+op.fill(0)
+before = in_use()
+op.run(None)
+assert in_use() == before, "the scratch was not refused"
+op.check()
+try:
+    T.DeviceBuffer((1 << 20,))
+except T.TTError as e:
+    print("REFUSED", e.code == T.TT_ERR_NOMEM)
+"""
+
+
+@pytest.mark.parametrize("kind", OPS)
+def test_refused_scratch_runs_unsplit(capi, kind):
+    """Every allocation after the operands' fails: the call's scratch is the first of them."""
+    op = Op(capi, kind)
+    env = dict(os.environ, TT_FAIL_ALLOC_AFTER=str(len(op.inp) + len(op.out)), PYTHONPATH=os.pathsep.join(
+        [ROOT, os.path.join(ROOT, "tests"), os.path.join(ROOT, "pku-aiprogramming_amd"),
+         os.environ.get("PYTHONPATH", "")]))
+    r = subprocess.run([sys.executable, "-c", REFUSED % kind], env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "REFUSED True" in r.stdout, r.stdout + r.stderr
+
+
+def test_scratch_is_taken_where_it_is_there(capi):
+    """The operations above do split: each leaves its workspace behind."""
+    n = C.c_size_t()
+    for kind in OPS:
+        op, st = Op(capi, kind), capi.Stream()
+        op.fill(0)
+        capi.lib().call("tt_mem_stats", C.byref(n), None)
+        before = n.value
+        op.run(st.handle)
+        st.sync()
+        capi.lib().call("tt_mem_stats", C.byref(n), None)
+        assert n.value > before, kind
+        st.destroy()
 
 
 @pytest.mark.parametrize("kind", OPS)

@@ -215,3 +215,34 @@ def test_wide_products_without_scratch():
         [ROOT, os.path.join(ROOT, "tests"), os.path.join(ROOT, "pku-aiprogramming_amd"), os.environ.get("PYTHONPATH", "")]))
     r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "REFUSED True" in r.stdout, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("k,stride,cout", [(2, 1000, 3), (3, 2, 1)], ids=["windows_apart", "phases"])
+def test_batches_beyond_one_launch(k, stride, cout):
+    """Two images of more than 2^29 elements are taken one by one: the outputs and image gradients of each alone,
+    bit for bit; the weight gradient their sum (bf16, three roundings of 2^-8)."""
+    import tt_capi as T
+
+    L, H = T.lib(), 23200
+    oh = (H - k) // stride + 1
+    x, go, w = (T.DeviceBuffer(s, "bf16") for s in ((2, 1, H, H), (2, cout, oh, oh), (cout, 1, k, k)))
+    for i, b in enumerate((x, go, w)):
+        b.fill_normal(i + 1)
+
+    def run(n, first):
+        out, gx, gw = (T.DeviceBuffer(s, "bf16") for s in ((n, cout, oh, oh), (n, 1, H, H), (cout, 1, k, k)))
+        geo = (n, 1, H, H, cout, k, k, 0, 0, stride, stride, None)
+        xp, gp = x.ptr + 2 * first * H * H, go.ptr + 2 * first * cout * oh * oh
+        L.call("tt_conv_forward", T.TT_BF16, xp, w.ptr, out.ptr, *geo)
+        L.call("tt_conv_backward", T.TT_BF16, xp, w.ptr, gp, gx.ptr, gw.ptr, *geo)
+        return out.download_bytes(), gx.download_bytes(), gw.download()
+
+    both, first, second = run(2, 0), run(1, 0), run(1, 1)
+    for i, name in ((0, "out"), (1, "grad_input")):
+        print(f"  {name}", flush=True)
+        assert both[i].any()
+        np.testing.assert_array_equal(both[i][0], first[i][0])
+        np.testing.assert_array_equal(both[i][1], second[i][0])
+    bound = 2.0 ** -8 * (np.abs(both[2]) + np.abs(first[2]) + np.abs(second[2]))
+    # the sums themselves: fp32 over up to 1.3e8 products of either sign
+    assert np.all(np.abs(both[2] - first[2] - second[2]) <= bound + 1e-4 * oh)

@@ -92,13 +92,17 @@ def test_col_sum(capi, dt, rows, cols):
 
 
 def test_refused_scratch_runs_unsplit(capi):
-    """With the scratch allocation refused the product still comes out."""
+    """With the scratch allocation (the one after the three matrices) refused the product still comes out."""
     code = (
-        "import numpy as np, tt_capi as T\n"
+        "import ctypes as C, numpy as np, tt_capi as T\n"
+        "def in_use():\n"
+        "    n = C.c_size_t(); T.lib().call('tt_mem_stats', C.byref(n), None); return n.value\n"
         "r = np.random.default_rng(1)\n"
         "A, B = (r.standard_normal(s).astype(np.float32) for s in ((48, 4096), (4096, 40)))\n"
         "a, b, c = T.DeviceBuffer.from_numpy(A), T.DeviceBuffer.from_numpy(B), T.DeviceBuffer((48, 40))\n"
+        "before = in_use()\n"
         "T.gemm(False, False, 48, 40, 4096, 1.0, a, b, 0.0, c)\n"
+        "assert in_use() == before, 'the scratch was not refused'\n"
         "ref = A.astype(np.float64) @ B.astype(np.float64)\n"
         "e = np.abs(c.download() - ref).max() / np.abs(ref).max()\n"
         "assert e <= 1e-5, e\n"
@@ -106,7 +110,7 @@ def test_refused_scratch_runs_unsplit(capi):
         "    T.DeviceBuffer((1 << 20,))\n"
         "except T.TTError as x:\n"
         "    print('REFUSED', x.code == T.TT_ERR_NOMEM)\n")
-    env = dict(os.environ, TT_FAIL_ALLOC_AFTER="4",
+    env = dict(os.environ, TT_FAIL_ALLOC_AFTER="3",
                PYTHONPATH=os.path.join(ROOT, "pku-aiprogramming_amd") + os.pathsep + os.environ.get("PYTHONPATH", ""))
     r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "REFUSED True" in r.stdout, r.stdout + r.stderr

@@ -1,7 +1,9 @@
-"""GPU tests of the split row softmax on rows that are not 16-byte aligned
-(csrc/softmax.hip): lengths around its chunks, partial last vectors, buffers
-that begin at any float, in place, chunks without a finite value.  Against
-float64 at the softmax tests' bar (1e-5 normwise)."""
+"""GPU tests of the row softmax on rows that are not 16-byte aligned
+(csrc/softmax.hip): the split kernel beyond 12288 columns (lengths around its
+chunks, partial last vectors, buffers that begin at any float, in place, chunks
+without a finite value) and the rows of up to 16384 columns that are too few
+to split, the one-workgroup kernel from 3329 to 12288 columns.  Against float64
+at the softmax tests' bar (1e-5 normwise)."""
 import numpy as np
 import pytest
 
@@ -30,7 +32,9 @@ def _run(capi, x, xo, yo, in_place=False):
 
 
 @pytest.mark.parametrize("rows,cols", [(17, 8193), (16, 12287), (16, 12289), (20, 16383), (5, 16385), (3, 65535),
-                                       (3, 65537), (2, 262143), (2, 262145), (1, 2097151), (16, 12288)])
+                                       (3, 65537), (2, 262143), (2, 262145), (1, 2097151), (16, 12288),
+                                       # on both sides of the fewest unaligned rows that are split, and aligned ones
+                                       (15, 12289), (15, 16383), (16, 12290), (3, 12292), (1, 16384)])
 @pytest.mark.parametrize("xo,yo", [(0, 0), (1, 2), (3, 0)])
 def test_unaligned_rows(capi, rows, cols, xo, yo):
     x = (3 * np.random.default_rng(cols).standard_normal((rows, cols))).astype(np.float32)
