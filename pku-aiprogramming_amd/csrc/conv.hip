@@ -207,11 +207,12 @@ int conv_entry(const char* fn, int dtype, const void* src, void* dst, int64_t N,
 // launches dominated (a product per image at 5-76 us each), at large ones the
 // dW product, one or a few tiles walking every pixel.  Forward / backward
 // through myLayer, us, before -> now: 64 x 8 x 14 x 14, 16 kernels 5 x 5 fp32
-// 1557 / 2212 -> 22 / 47; 64 x 64 x 56 x 56, 64 kernels 3 x 3 fp32 4128 /
-// 22291 -> 241 / 566 (61 / 52 TF), bf16 1683 / 7425 -> 109 / 360; 8 x 512 x
-// 28 x 28, 512 kernels 3 x 3 fp32 3468 / 1648 -> 566 / 1248; 1 x 3 x 224 x 224,
-// 768 kernels 16 x 16 stride 16 fp32 85 / 123 -> 27 / 44.  What bounds them now
-// is the gather's index arithmetic, about ten VALU instructions an element.
+// 1551 / 2214 -> 12 / 35; 64 x 64 x 56 x 56, 64 kernels 3 x 3 fp32 4121 /
+// 22257 -> 208 / 512 (71 / 58 TF), bf16 1660 / 7464 -> 89 / 320; 8 x 512 x
+// 28 x 28, 512 kernels 3 x 3 fp32 3477 / 1617 -> 506 / 1169; 1 x 3 x 224 x 224,
+// 768 kernels 16 x 16 stride 16 fp32 85 / 122 -> 17 / 33.  What bounds them now
+// is the gather's index arithmetic, about ten VALU instructions an element; the
+// layer leaves its widest products to the column matrix (layers.cpp).
 // n / d for 0 <= n < 2^31 by a multiplication (Granlund and Montgomery's
 // round-up method).
 struct FastDiv {

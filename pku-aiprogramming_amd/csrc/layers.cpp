@@ -480,15 +480,15 @@ bool conv_backward_columns(const std::string& fn, const T* in, const T* w, const
 // channels (the backward also the weights once per 64 pixels), at 50-170
 // TFLOP/s in bf16 and 50-70 in fp32 whatever the size; the columns are written
 // once and their products run at the GEMM's rate where one image's fill the
-// chip.  Measured (us, one image unless given, gathered / columns): bf16 forward
-// 2048 channels 28 x 28 3 x 3 414 / 246, 1024 64 x 64 3 x 3 411 / 265, but 512 28 x 28
-// 39 / 42 and 8 images of 512 28 x 28 234 / 310; backward 512 64 x 64 442 / 250,
-// 1024 64 x 64 1387 / 490, 2048 28 x 28 1423 / 459, 8 images of 768 64 x 64 stride
-// 2 1952 / 1186, but 8 of 384 28 x 28 351 / 520; fp32 backward 2048 28 x 28 2224 /
-// 1300, 512 64 x 64 727 / 581.  With a stride the gathered backward loses from
-// 256 channels on (256 of 512, 64 x 64, 102 / 80).  Windows that do not overlap
-// need no phases and are gathered with less work: 1 x 1 64 x 64 bf16 backward 48 /
-// 55 at 512 channels, 146 / 114 at 1024, fp32 832 / 689 at 2048.
+// chip.  Measured (us, C to C channels 3 x 3, one image unless given, gathered /
+// columns): bf16 forward 2048 28 x 28 501 / 356, 1024 64 x 64 440 / 288, but 512 28
+// x 28 39 / 42 and 16 images of it 349 / 591; backward 512 64 x 64 441 / 243, 1024
+// 64 x 64 1383 / 489, 2048 28 x 28 1421 / 437, 8 images of 768 64 x 64 stride 2 1964 /
+// 1211, but 16 of 512 28 x 28 1306 / 1393; fp32 backward 2048 28 x 28 2208 / 1288,
+// 512 64 x 64 715 / 585.  With a stride the gathered backward loses from 256
+// output channels on (512 to 256, 64 x 64, 102 / 75).  Windows that do not
+// overlap need no phases and are gathered with less work: 1 x 1 64 x 64 bf16
+// backward 48 / 56 at 512 channels, 146 / 111 at 1024, fp32 823 / 689 at 2048.
 bool wide_products(const ConvDims& d, bool bf16, bool backward, int sh, int sw) {
   const double products = (double)d.P() * d.cout * (double)d.K();  // per image
   if (sh >= d.kh && sw >= d.kw) return d.cout >= 512 && products >= (bf16 ? 0x1p31 : 0x1p34);
