@@ -247,8 +247,11 @@ int tt_attn_bwd_bf16_noalloc(const uint16_t* q, const uint16_t* k, const uint16_
  * q [B,H,1,d], k/v cache [B,H,Lkv,d] contiguous, o [B,H,1,d], lse [B,H] (may
  * be NULL).  The same composition as the forward with Lq = 1 (a3 -> a4 -> a6
  * -> a7 of the reference's op chain).  Splits Lkv across workgroups and merges
- * the partial (o, lse) pairs by LSE rescaling; partials live in a
- * library-owned scratch buffer. */
+ * their sums by each split's max and sum.  The partials live in per-stream
+ * library workspaces (allocated on first use): a fixed 2 MiB for the short
+ * splits of few heads and keys, without which (refused, or under graph capture
+ * before a call has left it on the stream) long splits run; those need theirs
+ * where a head takes several, TT_ERR_NOMEM if that fails. */
 int tt_attn_decode_bf16(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* o,
                         float* lse, int64_t B, int64_t H, int64_t Lkv, int64_t d,
                         float scale, void* stream);
