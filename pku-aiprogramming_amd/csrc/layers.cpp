@@ -417,10 +417,13 @@ struct Scratch {
 // images' columns at a time.  Sums over images and over an image's taps stay
 // in fp32.  False where its scratch is refused (nothing is written then).
 constexpr int64_t kColumnBytes = int64_t(64) << 20;  // of columns at a time, or one image's
+// One image's columns: within any memory, so that their bytes fit 64 bits.
+bool columns_countable(const ConvDims& d) { return (double)d.P() * (double)d.K() <= 0x1p40; }
 
 template <typename T>
 bool conv_forward_columns(const std::string& fn, const T* in, const T* w, T* out, const ConvDims& d, int ph, int pw,
                           int sh, int sw) {
+  if (!columns_countable(d)) return false;
   const int64_t P = d.P(), K = d.K(), image = (int64_t)d.in.C * d.in.H * d.in.W;
   const int64_t slab = std::min(d.in.batch, std::max<int64_t>(1, kColumnBytes / (P * K * (int64_t)sizeof(T))));
   Scratch scratch((size_t)(slab * P * K) * sizeof(T));
@@ -439,6 +442,7 @@ template <typename T>
 bool conv_backward_columns(const std::string& fn, const T* in, const T* w, const T* go, T* gin, T* gw,
                            const ConvDims& d, int ph, int pw, int sh, int sw) {
   constexpr bool F32 = std::is_same<T, float>::value;
+  if (!columns_countable(d)) return false;
   const int64_t P = d.P(), K = d.K(), image = (int64_t)d.in.C * d.in.H * d.in.W;
   const int64_t slab = std::min(d.in.batch, std::max<int64_t>(1, kColumnBytes / (P * K * (int64_t)sizeof(float))));
   // the columns, their fp32 gradients and, for bf16, both results in fp32, each
@@ -489,7 +493,9 @@ bool conv_backward_columns(const std::string& fn, const T* in, const T* w, const
 // output channels on (512 to 256, 64 x 64, 102 / 75).  Windows that do not
 // overlap need no phases and are gathered with less work: 1 x 1 64 x 64 bf16
 // backward 48 / 56 at 512 channels, 146 / 111 at 1024, fp32 823 / 689 at 2048.
+// At most 2^28 elements of columns an image (1 GiB in fp32).
 bool wide_products(const ConvDims& d, bool bf16, bool backward, int sh, int sw) {
+  if ((double)d.P() * (double)d.K() > 0x1p28) return false;
   const double products = (double)d.P() * d.cout * (double)d.K();  // per image
   if (sh >= d.kh && sw >= d.kw) return d.cout >= 512 && products >= (bf16 ? 0x1p31 : 0x1p34);
   const int wide = !backward ? 512 : sh > 1 || sw > 1 ? 256 : 384;
