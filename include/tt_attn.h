@@ -68,6 +68,9 @@ void* tt_stream(void);
 int tt_stream_create(void** stream);
 int tt_stream_sync(void* stream);
 int tt_stream_destroy(void* stream);
+/* *yes = whether a stream (NULL: the library stream) is being captured into a
+ * graph, which then keeps the addresses that calls use. */
+int tt_stream_capturing(void* stream, int* yes);
 
 /* Caching device allocator (hipMalloc-backed).
  * Replaces cudaMalloc at src/Tinytensor.cu:21,39,60,77,116,252,375.

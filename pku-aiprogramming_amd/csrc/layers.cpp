@@ -493,13 +493,19 @@ bool conv_backward_columns(const std::string& fn, const T* in, const T* w, const
 // output channels on (512 to 256, 64 x 64, 102 / 75).  Windows that do not
 // overlap need no phases and are gathered with less work: 1 x 1 64 x 64 bf16
 // backward 48 / 56 at 512 channels, 146 / 111 at 1024, fp32 823 / 689 at 2048.
-// At most 2^28 elements of columns an image (1 GiB in fp32).
+// At most 2^28 elements of columns an image (1 GiB in fp32), and not under
+// capture: the graph would keep the address of columns that are freed with the
+// call.
 bool wide_products(const ConvDims& d, bool bf16, bool backward, int sh, int sw) {
   if ((double)d.P() * (double)d.K() > 0x1p28) return false;
   const double products = (double)d.P() * d.cout * (double)d.K();  // per image
   if (sh >= d.kh && sw >= d.kw) return d.cout >= 512 && products >= (bf16 ? 0x1p31 : 0x1p34);
   const int wide = !backward ? 512 : sh > 1 || sw > 1 ? 256 : 384;
   return d.cout >= wide && products >= (d.in.batch == 1 ? 0x1p30 : 0x1p32) / (backward ? 2 : 1);
+}
+bool capturing() {
+  int yes = 0;
+  return tt_stream_capturing(nullptr, &yes) != TT_OK || yes;
 }
 
 }  // namespace
@@ -518,7 +524,8 @@ void ConvForward(const TinyTensor<T>& input, TinyTensor<T>& output, const TinyTe
   auto columns = [&] {
     return conv_forward_columns(fn, input.p_data, weight.p_data, output.p_data, d, pad_h, pad_w, stride_h, stride_w);
   };
-  if (wide_products(d, !std::is_same<T, float>::value, false, stride_h, stride_w) && columns()) return;
+  if (wide_products(d, !std::is_same<T, float>::value, false, stride_h, stride_w) && !capturing() && columns())
+    return;
   const int rc = tt_conv_forward(dtype_code<T>(), input.p_data, weight.p_data, output.p_data, d.in.batch, d.in.C,
                                  d.in.H, d.in.W, d.cout, d.kh, d.kw, pad_h, pad_w, stride_h, stride_w, nullptr);
   tt_check(rc != TT_ERR_UNSUPPORTED ? rc : columns() ? TT_OK : TT_ERR_NOMEM, fn.c_str());  // past its indices or grid
@@ -550,7 +557,8 @@ void ConvBackward(const TinyTensor<T>& input, const TinyTensor<T>& output, const
     return conv_backward_columns(fn, input.p_data, weight.p_data, grad_output.p_data, grad_input.p_data,
                                  grad_weight.p_data, d, pad_h, pad_w, stride_h, stride_w);
   };
-  if (wide_products(d, !std::is_same<T, float>::value, true, stride_h, stride_w) && columns()) return;
+  if (wide_products(d, !std::is_same<T, float>::value, true, stride_h, stride_w) && !capturing() && columns())
+    return;
   const int rc = tt_conv_backward(dtype_code<T>(), input.p_data, weight.p_data, grad_output.p_data, grad_input.p_data,
                                   grad_weight.p_data, d.in.batch, d.in.C, d.in.H, d.in.W, d.cout, d.kh, d.kw, pad_h,
                                   pad_w, stride_h, stride_w, nullptr);

@@ -473,6 +473,15 @@ int tt_stream_sync(void* stream) {
   return ok();
 }
 
+int tt_stream_capturing(void* stream, int* yes) {
+  if (!yes) return fail(TT_ERR_ARG, "tt_stream_capturing: null pointer");
+  *yes = 0;
+  int rc = ensure_init();
+  if (rc) return rc;
+  *yes = stream_capturing(stream_or_default(stream)) ? 1 : 0;
+  return ok();
+}
+
 int tt_stream_destroy(void* stream) {
   if (!stream) return TT_OK;
   if (stream == (void*)g_stream) return fail(TT_ERR_ARG, "tt_stream_destroy: the library stream is not the caller's");

@@ -35,6 +35,7 @@ _SIGS = {
     "tt_stream": (_p, []),
     "tt_stream_create": (C.c_int, [C.POINTER(_p)]),
     "tt_stream_sync": (C.c_int, [_p]),
+    "tt_stream_capturing": (C.c_int, [_p, C.POINTER(C.c_int)]),
     "tt_stream_destroy": (C.c_int, [_p]),
     "tt_malloc": (C.c_int, [C.POINTER(_p), C.c_size_t]),
     "tt_free": (C.c_int, [_p]),

@@ -188,6 +188,45 @@ def test_wide_products(dt, case):
         assert two <= (1e-6 if dt == "float" else 2e-3), (name, two)
 
 
+def test_wide_products_under_capture():
+    """Captured on the library stream they are gathered: no memory that other tensors get before a replay."""
+    import ctypes as C
+
+    import myLayer as ml
+    import myTensor as mt
+    import tt_capi as T
+    from test_capture_gpu import Capture
+
+    rng = np.random.default_rng(3)
+    shapes = ((1, 320, 28, 28), (512, 320, 3, 3), (1, 512, 28, 28))
+    x, w, go = (rng.standard_normal(s).astype(np.float32) for s in shapes)
+    X, Wt, GO = (mt.Tensor_float(a, "gpu") for a in (x, w, go))
+    out, gx, gw = (mt.Tensor_float(list(s), "gpu") for s in (shapes[2], shapes[0], shapes[1]))
+
+    def run():
+        ml.ConvForward(X, out, Wt, 1, 1, 1, 1)
+        ml.ConvBackward(X, out, Wt, gx, GO, gw, 1, 1, 1, 1)
+
+    run()  # leaves the columns' block with the allocator
+    stream = T.lib().lib.tt_stream()
+    yes = C.c_int()
+    with Capture(T, stream) as c:
+        T.lib().call("tt_stream_capturing", None, C.byref(yes))
+        run()
+    assert yes.value == 1
+    ref = _ref(x.astype(np.float64), w.astype(np.float64), go.astype(np.float64), 1, 1, 1, 1, blas=True)
+    others = [mt.Tensor_float([n], "gpu").zeros() for n in (1 << 20, 2 << 20, 4 << 20, 8 << 20)]
+    for _ in range(2):
+        for t in (out, gx, gw):
+            t.zeros()
+        T.lib().sync()
+        c.launch()
+        for got, r in zip((out, gw, gx), ref):
+            assert orc.max_rel_err(np.asarray(got.numpy()).reshape(r.shape), r) <= TOL["float"]
+        assert not any(np.asarray(t.numpy()).any() for t in others)
+    c.destroy()
+
+
 def test_wide_products_without_scratch():
     """The gathered products take over where the columns' memory is refused."""
     code = (
