@@ -59,6 +59,32 @@ def test_split_gemm(capi, dt, ta, tb, off, shape):
     assert orc.max_rel_err(out[off:].reshape(m, n), ref) <= TOL[dt]
 
 
+# bf16 operands with C in fp32: the split, the direct-to-LDS and the other 128-row kernel
+@pytest.mark.parametrize("ta", [0, 1])
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("shape", [(33, 129, 65), (64, 200, 4097), (2048, 4096, 64), (2100, 4100, 50)], ids=str)
+def test_gemm_fp32_result(capi, ta, tb, shape):
+    """No rounding of C: the products of bf16 values are exact in fp32, the sums fp32."""
+    m, n, k = shape
+    rng = np.random.default_rng(m + n + k + ta + 2 * tb)
+    A, B = _vals(rng, (k, m) if ta else (m, k), "bf16"), _vals(rng, (n, k) if tb else (k, n), "bf16")
+    C = _vals(rng, (m, n), "f32")
+    a, b, c = (capi.DeviceBuffer.from_numpy(x, dt) for x, dt in ((A, "bf16"), (B, "bf16"), (C, "f32")))
+    capi.lib().call("tt_gemm_bf16_f32", ta, tb, m, n, k, 0.5, a.ptr, b.ptr, 1.5, c.ptr, None)
+    assert orc.max_rel_err(c.download(), orc.gemm_f64(bool(ta), bool(tb), 0.5, A, B, 1.5, C)) <= TOL["f32"]
+
+
+@pytest.mark.parametrize("n", [1, 255, 70000])
+def test_round_bf16(capi, n):
+    x = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+    x[:4] = np.array([np.nan, np.inf, -np.inf, 3.3895e38], np.float32)[:n]  # the last one rounds to infinity
+    src, dst = capi.DeviceBuffer.from_numpy(x), capi.DeviceBuffer((n,), "bf16")
+    capi.lib().call("tt_round_bf16", src.ptr, dst.ptr, n, None)
+    bits = dst.download_bytes()
+    assert np.isnan(orc.bf16_to_f32(bits[:1]))[0]
+    np.testing.assert_array_equal(bits[1:], capi.bf16_bits(x)[1:])
+
+
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("scalar", [0, 1])
 @pytest.mark.parametrize("shape", [(5, 9, 3), (64, 200, 100), (2048, 512, 4096)], ids=str)
