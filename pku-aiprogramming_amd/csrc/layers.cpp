@@ -486,11 +486,12 @@ bool conv_backward_columns(const std::string& fn, const T* in, const T* w, const
 // once and their products run at the GEMM's rate where one image's fill the
 // chip.  Measured (us, C to C channels 3 x 3, one image unless given, gathered /
 // columns): bf16 forward 2048 28 x 28 501 / 356, 1024 64 x 64 440 / 288, but 512 28
-// x 28 39 / 42 and 16 images of it 349 / 591; backward 512 64 x 64 441 / 243, 1024
+// x 28 39 / 42 and 16 images of it 349 / 591, 8 of 1024 28 x 28 739 / 859; backward 512 64 x 64 441 / 243, 1024
 // 64 x 64 1383 / 489, 2048 28 x 28 1421 / 437, 8 images of 768 64 x 64 stride 2 1964 /
 // 1211, but 16 of 512 28 x 28 1306 / 1393; fp32 backward 2048 28 x 28 2208 / 1288,
-// 512 64 x 64 715 / 585.  With a stride the gathered backward loses from 256
-// output channels on (512 to 256, 64 x 64, 102 / 75).  Windows that do not
+// 512 64 x 64 715 / 585.  With a stride the gathered backward of one image loses
+// from 256 output channels on (512 to 256, 64 x 64, 102 / 75; 8 fp32 images of 1024
+// to 256, 1339 / 1576).  Windows that do not
 // overlap need no phases and are gathered with less work: 1 x 1 64 x 64 bf16
 // backward 48 / 56 at 512 channels, 146 / 111 at 1024, fp32 823 / 689 at 2048.
 // At most 2^28 elements of columns an image (1 GiB in fp32), and not under
@@ -500,8 +501,9 @@ bool wide_products(const ConvDims& d, bool bf16, bool backward, int sh, int sw) 
   if ((double)d.P() * (double)d.K() > 0x1p28) return false;
   const double products = (double)d.P() * d.cout * (double)d.K();  // per image
   if (sh >= d.kh && sw >= d.kw) return d.cout >= 512 && products >= (bf16 ? 0x1p31 : 0x1p34);
-  const int wide = !backward ? 512 : sh > 1 || sw > 1 ? 256 : 384;
-  return d.cout >= wide && products >= (d.in.batch == 1 ? 0x1p30 : 0x1p32) / (backward ? 2 : 1);
+  const bool one = d.in.batch == 1;
+  if (!backward) return d.cout >= 512 && products >= (one ? 0x1p30 : 0x1p33);
+  return d.cout >= (one && (sh > 1 || sw > 1) ? 256 : 384) && products >= (one ? 0x1p29 : 0x1p31);
 }
 bool capturing() {
   int yes = 0;
